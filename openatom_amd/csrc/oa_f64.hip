@@ -9,25 +9,51 @@
 //                       weight, mirror to the lower triangle, max|S - d I|.
 //   ns_* kernels        guarded Newton-Schulz S->T iteration (device flags).
 //
-// Tiling: 256-thread workgroups (4 wave64s in a 2x2 grid), each wave owns a
-// (16*WM) x (16*WM) block of v_mfma_f64_16x16x4f64 accumulators.  Operand
-// lanes: lane l supplies A[l%16][l/16] and B[l/16][l%16]; result register v
-// of lane l holds D[l/16 + 4v][l%16] (measured on gfx950).  Operand
-// panels of BK=16 doubles are staged through LDS with a row stride of 18
-// doubles, which makes the 16-byte fragment reads of 16 lanes cover all 64
-// banks once.  Each lane reads two consecutive k per LDS access and feeds
-// them to two MFMAs; the k order inside a panel is therefore permuted the
-// same way for both operands, which leaves every product sum unchanged.
+// What bounds the products: v_mfma_f64_16x16x4f64 (78.6 TFLOP/s nominal).  A
+// register-only loop of independent MFMAs reaches 77 TF from two or four
+// waves per SIMD but only 35-38 TF from one: a single wave issues at most
+// every other MFMA slot, so with two waves per SIMD each must always have its
+// next MFMA ready and no stall of one is made up by the other.  The tiles
+// are therefore split so that four waves share a SIMD (at most 128 registers
+// each), and the operands go from global memory to LDS by direct-to-LDS loads
+// that need no registers.  T psi at n = 1024, npw = 262144: 17.1 ms (64 TF,
+// MFMA busy 84 % at 2.29 GHz) with two waves of 64 x 64 per SIMD and register
+// staging, 15.5 ms (71 TF, busy 91 % at 2.2 GHz) so; HBM fetch 17.3 -> 6.3 GB.
+// What is left is mostly the clock, which falls as the matrix cores fill.
+//
+// Tiling: a BM x BN tile per workgroup of WR x WC waves; a wave owns WM x WN
+// blocks of 16 x 16.  Operand lanes: lane l supplies A[l%16][l/16] and
+// B[l/16][l%16]; result register v of lane l holds D[l/16 + 4v][l%16]
+// (measured on gfx950).  A stage is BK = 16 contraction indices.  MFMA
+// (kk, e) of a stage contracts k = 8 kk + 2 g + e over the lane groups g =
+// 0..3, the same for both operands and for every tile, so each output's sum
+// runs in one order whatever the tile: all launch forms give the same bits.
+//
+// LDS panels (R rows of one operand, one stage):
+//   KC  (k contiguous in memory): row-major rows of 128 bytes, the eight
+//       16-byte k pairs of row r permuted by XOR with (r >> 1) & 7, so that
+//       the 16-byte fragment reads of 16 consecutive rows cover all 64 banks.
+//       A fragment read returns two consecutive k (both MFMAs e of a kk).
+//   !KC (rows contiguous in memory): [k][row], as in memory.  A fragment read
+//       returns two consecutive rows of one k, which feed two blocks: blocks
+//       2b and 2b + 1 of a wave then hold the even and odd rows of a 32-row
+//       span (a wave with one block reads 8 bytes per lane instead).
+// MFMAs of blocks past an edge are not issued: row blocks (or spans) are dealt
+// to the wave rows in turn, so a ragged last tile drops them from every wave
+// alike; the overlap deals the blocks of a ragged or diagonal tile to its
+// waves one by one.
+#include <type_traits>
+
 #include "oa_internal.h"
 
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2v __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // 8-byte aligned pair
 
-constexpr int NT = 256;
+constexpr int NT = 256;  // threads of the elementwise kernels
 constexpr int BK = 16;
-constexpr int LS = BK + 2;
 
 __host__ __device__ __forceinline__ int cdiv(int a, int b) { return (a + b - 1) / b; }
 
@@ -38,191 +64,309 @@ __device__ __forceinline__ int xcd_logical(int b, int nb) {
   return (b & 7) * per + (b >> 3);
 }
 
-// Per-thread loader of one BR x BK operand panel, 16 bytes per load.
-//   KC  (element (r, k) at p[r*ld + k], k contiguous): a row holds 8 chunks;
-//       thread t owns chunk (t % 8) of rows t/8 + 32j.
-//   !KC (element (r, k) at p[k*ld + r], r contiguous): a k-row holds BR/2
-//       chunks; thread t owns chunk (t % (BR/2)) of k-rows t/(BR/2) + NT/(BR/2)*j.
-// load_fast() needs a 16-byte aligned, fully in-range panel; load_masked()
-// reads element by element and zero-fills outside [rlim) x [klim).
-template <int BR, bool KC>
-struct PanelLoader {
-  static constexpr int CH = BR * BK / 2 / NT;
-  static constexpr int KSTEP = KC ? 0 : NT / (BR / 2);
-  const double *base;  // matrix origin
-  long ld;
-  int rb, kb;          // this thread's first (row, k) inside the panel
-  d2v v[CH];
+// Tile configurations.  WPE waves per SIMD are allowed (512 / WPE registers a
+// wave); NBUF stages rotate through LDS (NBUF - 1 in flight).
+//   T128   the large products: 64 x 32 wave tiles, two workgroups per CU.  Two
+//          stages suffice: one stage is 8192 MFMA cycles of a SIMD.  T psi at
+//          n = 1024 / 512 / 301 (npw 262144 / 65536 / 20011): 15.5 / 1.05 /
+//          0.175 ms; with 64 x 64 wave tiles 15.8 / 1.03 / 0.185; one
+//          workgroup of 16 waves per CU and four stages 16.9 / 1.14 / 0.179.
+//   T64    many small tiles: 32 x 32 wave tiles, four workgroups per CU.
+//   T64W   few tiles (about one per CU): 16 x 32 wave tiles, so that a lone
+//          workgroup still puts two waves on a SIMD.
+//   T32    fewer still: a quarter of the tile, four times the workgroups.
+template <int BM_, int BN_, int WR_, int WC_, int WPE_, int NBUF_>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, WR = WR_, WC = WC_, WPE = WPE_, NBUF = NBUF_;
+  static constexpr int NW = WR * WC, NTHR = 64 * NW;
+  static constexpr int WM = BM / (16 * WR), WN = BN / (16 * WC);
+  static constexpr int STAGE = (BM + BN) * BK;  // doubles of one stage, X panel then Y
+  static constexpr int SMEM = NBUF * STAGE;
+};
+typedef Tile<128, 128, 2, 4, 4, 2> T128;
+typedef Tile<64, 64, 2, 2, 4, 2> T64;
+typedef Tile<64, 64, 4, 2, 4, 4> T64W;
+typedef Tile<32, 32, 2, 2, 4, 4> T32;
 
-  __device__ __forceinline__ void init(const double *p, long ld_, int tid) {
-    base = p;
-    ld = ld_;
-    if (KC) { rb = tid / 8; kb = (tid % 8) * 2; }
-    else { rb = (tid % (BR / 2)) * 2; kb = tid / (BR / 2); }
+__device__ __forceinline__ bool aligned16(const void *p) {
+  return ((uintptr_t)p & 15) == 0;
+}
+
+// Position of block i (16 rows) of a wave inside its panel, and the panel row
+// of the block's operand lane idx.  PAIR: blocks 2b, 2b + 1 interleave the
+// rows of one 32-row span.
+template <int W, int NWAVE, bool KC>
+struct RowMap {
+  static constexpr bool PAIR = !KC && (W % 2) == 0;
+  __device__ static __forceinline__ int first(int i, int wv) {
+    return PAIR ? ((i / 2) * NWAVE + wv) * 32 + (i & 1) : (i * NWAVE + wv) * 16;
   }
-  __device__ __forceinline__ void load_fast(int r0, int k0) {
-    if (KC) {
-      const double *q = base + (long)(r0 + rb) * ld + k0 + kb;
+  __device__ static __forceinline__ int row(int i, int wv, int idx) {
+    return first(i, wv) + (PAIR ? 2 * idx : idx);
+  }
+};
+
+// Fills one operand's R x BK panel of a stage.  The panel is R*8 chunks of 16
+// bytes in LDS order; chunk pos = (w + NW*j)*64 + lane belongs to load j of
+// wave w.  Three ways to fetch a stage:
+//   dma     global_load_lds_dwordx4 straight into the panel: 16-byte aligned
+//           operand, whole stage (rows past the edge read the last row, whose
+//           products only reach outputs that are not stored)
+//   pair    8-byte aligned pairs through registers (odd leading dimensions)
+//   masked  element by element, zeros outside [rlim) x [klim): a stage cut by
+//           the end of the contraction, or an edge tile that pair cannot read
+template <int R, bool KC, int NW>
+struct Panel {
+  static constexpr int CH = R * BK / 2 / 64 / NW;
+  static_assert(CH * NW * 64 * 2 == R * BK, "whole wave loads per stage");
+  const double *p[CH];  // this lane's chunks of the next stage to fetch
+  long step;            // elements from one stage to the next
+  bool dmaok, pairok;
+
+  __device__ __forceinline__ static int pos(int j, int w, int lane) {
+    return (w + NW * j) * 64 + lane;
+  }
+  __device__ __forceinline__ static int kc_pair(int row, int slot) {
+    return slot ^ ((row >> 1) & 7);
+  }
+  __device__ __forceinline__ void init(const double *b, long ld, int r0, int rlim, int k0, int w,
+                                       int lane) {
+    const bool inner = r0 + R <= rlim;
+    const bool al = aligned16(b) && (ld % 2) == 0;
+    dmaok = al && (KC ? (k0 % 2) == 0 : (inner || (rlim % 2) == 0));
+    pairok = KC || inner;
+    step = KC ? (long)BK : BK * ld;
 #pragma unroll
-      for (int j = 0; j < CH; j++) v[j] = *reinterpret_cast<const d2v *>(q + (long)(32 * j) * ld);
-    } else {
-      const double *q = base + (long)(k0 + kb) * ld + r0 + rb;
-#pragma unroll
-      for (int j = 0; j < CH; j++)
-        v[j] = *reinterpret_cast<const d2v *>(q + (long)(KSTEP * j) * ld);
+    for (int j = 0; j < CH; j++) {
+      const int c = pos(j, w, lane);
+      if (KC) {
+        const int row = c >> 3;
+        p[j] = b + (long)min(r0 + row, rlim - 1) * ld + k0 + 2 * kc_pair(row, c & 7);
+      } else {
+        const int kr = c / (R / 2), col = r0 + 2 * (c % (R / 2));
+        p[j] = b + (long)(k0 + kr) * ld + (inner ? col : max(0, min(col, rlim - 2)));
+      }
     }
   }
-  __device__ __forceinline__ void load_masked(int r0, int rlim, int k0, int klim) {
+  // a whole stage straight into `buf`; the loads stay in flight
+  __device__ __forceinline__ void dma(double *buf, int w) {
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      __builtin_amdgcn_global_load_lds(
+          p[j], (__attribute__((address_space(3))) void *)(buf + (w + NW * j) * 128), 16, 0, 0);
+      p[j] += step;
+    }
+  }
+  // a whole stage into registers, and from them into `buf`
+  __device__ __forceinline__ void pair(d2v (&v)[CH]) {
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      v[j] = *reinterpret_cast<const d2u *>(p[j]);
+      p[j] += step;
+    }
+  }
+  __device__ __forceinline__ static void put(const d2v (&v)[CH], double *buf, int w, int lane) {
 #pragma unroll
     for (int j = 0; j < CH; j++)
-#pragma unroll
-      for (int e = 0; e < 2; e++) {
-        const int r = KC ? r0 + rb + 32 * j : r0 + rb + e;
-        const int k = KC ? k0 + kb + e : k0 + kb + KSTEP * j;
-        v[j][e] = (r < rlim && k < klim) ? base[KC ? (long)r * ld + k : (long)k * ld + r] : 0.0;
-      }
+      *reinterpret_cast<d2v *>(buf + 2 * pos(j, w, lane)) = v[j];
   }
-  __device__ __forceinline__ void store(double *s) const {
-    if (KC) {
-#pragma unroll
-      for (int j = 0; j < CH; j++) *reinterpret_cast<d2v *>(s + (rb + 32 * j) * LS + kb) = v[j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < CH; j++) {
-        s[rb * LS + kb + KSTEP * j] = v[j][0];
-        s[(rb + 1) * LS + kb + KSTEP * j] = v[j][1];
-      }
+  __device__ __forceinline__ static void masked(const double *b, long ld, int r0, int rlim,
+                                                int k0, int klim, double *buf, int w, int lane) {
+#pragma unroll 1
+    for (int j = 0; j < 2 * CH; j++) {
+      const int c = pos(j >> 1, w, lane), e = j & 1;
+      const int row = KC ? r0 + (c >> 3) : r0 + 2 * (c % (R / 2)) + e;
+      const int k = KC ? k0 + 2 * kc_pair(c >> 3, c & 7) + e : k0 + c / (R / 2);
+      buf[2 * c + e] =
+          (row < rlim && k < klim) ? b[KC ? (long)row * ld + k : (long)k * ld + row] : 0.0;
     }
   }
 };
 
-// One BK-deep LDS stage of MFMAs for a wave's WM x WM block grid.
-template <int WM>
-__device__ __forceinline__ void mma_stage(const double *Xs, const double *Ys, int xrow0,
-                                          int yrow0, int lane, d4 (&acc)[WM][WM]) {
+// One operand's fragments of k step kk of a stage: get(e, i) is this lane's
+// value of block i (of the first NI) for MFMA e.
+template <int R, bool KC, int W, int NWAVE, int NI>
+struct Frags {
+  static constexpr bool PAIR = RowMap<W, NWAVE, KC>::PAIR;
+  static constexpr int NF = PAIR ? (NI + 1) / 2 : NI;
+  d2v f[KC ? NI : 2 * NF];
+  __device__ __forceinline__ void load(const double *s, int wv, int kk, int lane) {
+    const int r = lane & 15, g = lane >> 4;
+    if constexpr (KC) {
+#pragma unroll
+      for (int i = 0; i < NI; i++) {
+        const int row = (i * NWAVE + wv) * 16 + r;
+        f[i] = *reinterpret_cast<const d2v *>(s + row * BK +
+                                              2 * ((4 * kk + g) ^ ((row >> 1) & 7)));
+      }
+    } else if constexpr (PAIR) {
+#pragma unroll
+      for (int e = 0; e < 2; e++)
+#pragma unroll
+        for (int b = 0; b < NF; b++)
+          f[e * NF + b] = *reinterpret_cast<const d2v *>(s + (8 * kk + 2 * g + e) * R +
+                                                         (b * NWAVE + wv) * 32 + 2 * r);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 2; e++)
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+          f[e * NF + i][0] = s[(8 * kk + 2 * g + e) * R + (i * NWAVE + wv) * 16 + r];
+    }
+  }
+  __device__ __forceinline__ double get(int e, int i) const {
+    if constexpr (KC) return f[i][e];
+    else if constexpr (PAIR) return f[e * NF + i / 2][i & 1];
+    else return f[e * NF + i][0];
+  }
+};
+
+// The MFMAs of one stage over the first NI row blocks of the wave.  (A count
+// tested per MFMA made the compiler copy the accumulators at every branch, so
+// the count is a template argument and the choice lies outside the k loop.)
+template <class C, bool XKC, bool YKC, int NI>
+__device__ __forceinline__ void mma_rows(const double *Xs, const double *Ys, int wr, int wc,
+                                         int lane, d4 (&acc)[C::WM * C::WN]) {
+  constexpr int WN = C::WN;
+  if constexpr (NI > 0) {
+#pragma unroll
+    for (int kk = 0; kk < BK / 8; kk++) {
+      Frags<C::BM, XKC, C::WM, C::WR, NI> a;
+      Frags<C::BN, YKC, WN, C::WC, WN> b;
+      a.load(Xs, wr, kk, lane);
+      b.load(Ys, wc, kk, lane);
+#pragma unroll
+      for (int e = 0; e < 2; e++)
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+          for (int j = 0; j < WN; j++)
+            acc[i * WN + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.get(e, i), b.get(e, j),
+                                                                   acc[i * WN + j], 0, 0, 0);
+    }
+  }
+}
+
+// The MFMAs of one stage over NB single blocks (KC operands): block t has its
+// operand rows at panel rows xr[t] and yr[t].
+template <int NB, int CAP>
+__device__ __forceinline__ void mma_list(const double *Xs, const double *Ys,
+                                         const int (&xr)[NB], const int (&yr)[NB], int lane,
+                                         d4 (&acc)[CAP]) {
   const int r = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int kk2 = 0; kk2 < BK / 8; kk2++) {
-    d2v a[WM], b[WM];
+  for (int kk = 0; kk < BK / 8; kk++) {
+    // rows start at multiples of 16, so the pair permutation depends on r only
+    const int off = r * BK + 2 * ((4 * kk + g) ^ ((r >> 1) & 7));
 #pragma unroll
-    for (int i = 0; i < WM; i++)
-      a[i] = *reinterpret_cast<const d2v *>(Xs + (xrow0 + i * 16 + r) * LS + kk2 * 8 + 2 * g);
+    for (int t = 0; t < NB; t++) {
+      const d2v a = *reinterpret_cast<const d2v *>(Xs + xr[t] * BK + off);
+      const d2v b = *reinterpret_cast<const d2v *>(Ys + yr[t] * BK + off);
 #pragma unroll
-    for (int j = 0; j < WM; j++)
-      b[j] = *reinterpret_cast<const d2v *>(Ys + (yrow0 + j * 16 + r) * LS + kk2 * 8 + 2 * g);
-#pragma unroll
-    for (int e = 0; e < 2; e++)
-#pragma unroll
-      for (int i = 0; i < WM; i++)
-#pragma unroll
-        for (int j = 0; j < WM; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+      for (int e = 0; e < 2; e++)
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], b[e], acc[t], 0, 0, 0);
+    }
   }
 }
 
-// Main K loop shared by every FP64 kernel.  Two LDS buffers per operand and
-// one barrier per BK stage: stage s+1 is fetched into registers while stage s
-// feeds the MFMAs, then written to the other buffer.  `fast` selects 16-byte
-// unmasked loads (interior, aligned tiles); the last stage falls back to
-// masked loads when K is not a multiple of BK.  When YSAME the Y panel is the
-// X panel (diagonal tile of a symmetric product) and is loaded once.
-template <int WM, bool XKC, bool YKC, bool YSAME>
+// Calls f(integral_constant<int, V>) with V = v clamped into [LO, HI].
+template <int LO, int HI, class F>
+__device__ __forceinline__ void count_switch(int v, F &&f) {
+  if constexpr (LO < HI) {
+    if (v <= LO) f(std::integral_constant<int, LO>{});
+    else count_switch<LO + 1, HI>(v, f);
+  } else {
+    f(std::integral_constant<int, HI>{});
+  }
+}
+
+// Runs mma(X panel, Y panel) over the stages of k in [ka, kb) of one tile.
+// YSAME: the Y panel is the X panel (diagonal tile of a symmetric product),
+// loaded once.
+template <class C, bool XKC, bool YKC, bool YSAME, class Mma>
 __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mlim,
                                       const double *Y, long ldy, int n0, int nlim, int ka,
-                                      int kb, bool fast, double *smem, d4 (&acc)[WM][WM]) {
-  constexpr int BM = 32 * WM;
-  constexpr int PANEL = BM * LS;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int xrow0 = (w >> 1) * 16 * WM, yrow0 = (w & 1) * 16 * WM;
-  PanelLoader<BM, XKC> lx;
-  PanelLoader<BM, YKC> ly;
-  lx.init(X, ldx, tid);
-  if (!YSAME) ly.init(Y, ldy, tid);
-  const int nst = (kb - ka + BK - 1) / BK;
-  if (nst <= 0) return;
-  auto fetch = [&](int k0) {
-    if (fast && k0 + BK <= kb) {
-      lx.load_fast(m0, k0);
-      if (!YSAME) ly.load_fast(n0, k0);
-    } else {
-      lx.load_masked(m0, mlim, k0, kb);
-      if (!YSAME) ly.load_masked(n0, nlim, k0, kb);
+                                      int kb, double *smem, Mma &&mma) {
+  constexpr int NBUF = C::NBUF, YOFF = YSAME ? 0 : C::BM * BK;
+  typedef Panel<C::BM, XKC, C::NW> PX;
+  typedef Panel<C::BN, YKC, C::NW> PY;
+  const int nfull = (kb - ka) / BK;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  PX lx;
+  PY ly;
+  lx.init(X, ldx, m0, mlim, ka, w, lane);
+  if (!YSAME) ly.init(Y, ldy, n0, nlim, ka, w, lane);
+  const bool dx = lx.dmaok, dy = YSAME || ly.dmaok;
+  if (dx && dy) {
+    constexpr int PER = PX::CH + (YSAME ? 0 : PY::CH);  // loads of a stage per wave
+    auto issue = [&](int s) {
+      double *buf = smem + (s % NBUF) * C::STAGE;
+      lx.dma(buf, w);
+      if (!YSAME) ly.dma(buf + YOFF, w);
+    };
+#pragma unroll
+    for (int s = 0; s < NBUF - 1; s++)
+      if (s < nfull) issue(s);
+    for (int s = 0; s < nfull; s++) {
+      // stages s + 1 .. min(nfull - 1, s + NBUF - 2) may stay in flight
+      const int ahead = min(nfull - 1, s + NBUF - 2) - s;
+      if (NBUF >= 4 && ahead >= 2) wait_vm<2 * PER>();
+      else if (NBUF >= 3 && ahead >= 1) wait_vm<PER>();
+      else wait_vm<0>();
+      ring_barrier();
+      if (s + NBUF - 1 < nfull) issue(s + NBUF - 1);
+      const double *cur = smem + (s % NBUF) * C::STAGE;
+      mma(cur, cur + YOFF);
     }
-  };
-  // buffers: X at smem + b*PANEL, Y at smem + (2 + b)*PANEL (plain pointer
-  // arithmetic keeps the LDS address space visible to the compiler)
-  fetch(ka);
-  lx.store(smem);
-  if (!YSAME) ly.store(smem + 2 * PANEL);
-  __syncthreads();
-  for (int s = 0; s < nst; s++) {
-    const int cur = (s & 1) * PANEL, nxt = PANEL - cur;
-    const bool more = s + 1 < nst;
-    if (more) fetch(ka + (s + 1) * BK);
-    mma_stage<WM>(smem + cur, YSAME ? smem + cur : smem + 2 * PANEL + cur, xrow0, yrow0, lane,
-                  acc);
-    if (more) {
-      lx.store(smem + nxt);
-      if (!YSAME) ly.store(smem + 2 * PANEL + nxt);
+  } else {
+    // one operand at least goes through registers: loaded while the stage
+    // before it is multiplied, stored after it
+    const bool px = !dx && lx.pairok, py = !dy && ly.pairok;
+    d2v vx[PX::CH], vy[PY::CH];
+    auto load = [&](int s) {
+      double *buf = smem + (s & 1) * C::STAGE;
+      if (dx) lx.dma(buf, w);
+      else if (px) lx.pair(vx);
+      if (!YSAME) {
+        if (dy) ly.dma(buf + YOFF, w);
+        else if (py) ly.pair(vy);
+      }
+    };
+    auto finish = [&](int s) {
+      double *buf = smem + (s & 1) * C::STAGE;
+      const int k0 = ka + s * BK;
+      if (!dx) {
+        if (px) PX::put(vx, buf, w, lane);
+        else PX::masked(X, ldx, m0, mlim, k0, kb, buf, w, lane);
+      }
+      if (!YSAME && !dy) {
+        if (py) PY::put(vy, buf + YOFF, w, lane);
+        else PY::masked(Y, ldy, n0, nlim, k0, kb, buf + YOFF, w, lane);
+      }
+    };
+    if (nfull > 0) {
+      load(0);
+      finish(0);
     }
-    __syncthreads();
+    for (int s = 0; s < nfull; s++) {
+      wait_vm<0>();
+      ring_barrier();
+      if (s + 1 < nfull) load(s + 1);
+      const double *cur = smem + (s & 1) * C::STAGE;
+      mma(cur, cur + YOFF);
+      if (s + 1 < nfull) finish(s + 1);
+    }
   }
-}
-
-// kloop with the loads issued two stages ahead in two register sets, for the
-// 64 x 64 tiles of the small n x n products (S->T, small back-multiplies),
-// where one stage of MFMA work is shorter than a global load's latency.  The
-// stages and their products run in kloop's order, so the sums are
-// bit-identical.  Register set s % 2 holds stage s + 1 when stage s starts.
-template <int WM, bool XKC, bool YKC>
-__device__ __forceinline__ void kloop_pf2(const double *X, long ldx, int m0, int mlim,
-                                          const double *Y, long ldy, int n0, int nlim, int ka,
-                                          int kb, bool fast, double *smem, d4 (&acc)[WM][WM]) {
-  constexpr int BM = 32 * WM;
-  constexpr int PANEL = BM * LS;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int xrow0 = (w >> 1) * 16 * WM, yrow0 = (w & 1) * 16 * WM;
-  PanelLoader<BM, XKC> lx0, lx1;
-  PanelLoader<BM, YKC> ly0, ly1;
-  lx0.init(X, ldx, tid);
-  lx1.init(X, ldx, tid);
-  ly0.init(Y, ldy, tid);
-  ly1.init(Y, ldy, tid);
-  const int nst = (kb - ka + BK - 1) / BK;
-  if (nst <= 0) return;
-  auto fetch = [&](PanelLoader<BM, XKC> &lx, PanelLoader<BM, YKC> &ly, int k0) {
-    if (fast && k0 + BK <= kb) {
-      lx.load_fast(m0, k0);
-      ly.load_fast(n0, k0);
-    } else {
-      lx.load_masked(m0, mlim, k0, kb);
-      ly.load_masked(n0, nlim, k0, kb);
-    }
-  };
-  fetch(lx0, ly0, ka);
-  lx0.store(smem);
-  ly0.store(smem + 2 * PANEL);
-  if (nst > 1) fetch(lx0, ly0, ka + BK);
-  if (nst > 2) fetch(lx1, ly1, ka + 2 * BK);
-  __syncthreads();
-  auto step = [&](int s, PanelLoader<BM, XKC> &lx, PanelLoader<BM, YKC> &ly) {
-    const int cur = (s & 1) * PANEL, nxt = PANEL - cur;
-    mma_stage<WM>(smem + cur, smem + 2 * PANEL + cur, xrow0, yrow0, lane, acc);
-    if (s + 1 < nst) {
-      lx.store(smem + nxt);
-      ly.store(smem + 2 * PANEL + nxt);
-      if (s + 3 < nst) fetch(lx, ly, ka + (s + 3) * BK);
-    }
-    __syncthreads();
-  };
-  for (int s = 0; s < nst; s += 2) {
-    step(s, lx0, ly0);
-    if (s + 1 < nst) step(s + 1, lx1, ly1);
+  // the rest of a contraction that is no multiple of BK
+  const int k0 = ka + nfull * BK;
+  if (k0 < kb) {
+    ring_barrier();
+    PX::masked(X, ldx, m0, mlim, k0, kb, smem, w, lane);
+    if (!YSAME) PY::masked(Y, ldy, n0, nlim, k0, kb, smem + YOFF, w, lane);
+    ring_barrier();
+    mma(smem, smem + YOFF);
   }
-}
-
-__device__ __forceinline__ bool aligned16(const void *p) {
-  return ((uintptr_t)p & 15) == 0;
+  ring_barrier();  // the ring may be refilled (a workgroup's next item)
 }
 
 // Field-by-field selection keeps the problem in scalar registers (indexing
@@ -261,75 +405,82 @@ __device__ __forceinline__ ProbRegs pick_problem(const oa_gemm_problem &p0,
   return r;
 }
 
-// One (BM x BM) output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I.
-template <bool TX, bool TY, int WM>
+// One BM x BN output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I.
+template <bool TX, bool TY, class C>
 __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double *smem) {
-  constexpr int BM = 32 * WM;
-  const int tmn = cdiv(P.M, BM), tnn = cdiv(P.N, BM);
+  constexpr int WM = C::WM, WN = C::WN;
+  typedef RowMap<WM, C::WR, !TX> RM;
+  typedef RowMap<WN, C::WC, TY> CM;
+  const int tmn = cdiv(P.M, C::BM), tnn = cdiv(P.N, C::BN);
   if (logical >= tmn * tnn) return;
   const int tm = logical % tmn, tn = logical / tmn;
-  const int m0 = tm * BM, n0 = tn * BM;
-  d4 acc[WM][WM];
+  const int m0 = tm * C::BM, n0 = tn * C::BN;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = w / C::WC, wc = w % C::WC;
+  int ni = 0;  // the wave's row blocks inside the matrix
+#pragma unroll
+  for (int i = 0; i < WM; i++)
+    if (m0 + RM::first(i, wr) < P.M) ni = i + 1;
+  d4 acc[WM * WN];
+#pragma unroll
+  for (int i = 0; i < WM * WN; i++) acc[i] = d4{0, 0, 0, 0};
+  count_switch<0, WM>(ni, [&](auto c) {
+    kloop<C, !TX, TY, false>(P.X, P.ldx, m0, P.M, P.Y, P.ldy, n0, P.N, 0, P.K, smem,
+                             [&](const double *Xs, const double *Ys) {
+                               mma_rows<C, !TX, TY, decltype(c)::value>(Xs, Ys, wr, wc, lane,
+                                                                        acc);
+                             });
+  });
+
+  const int r = lane & 15, g = lane >> 4;
+  const double alpha = P.alpha, beta = P.beta, dadd = P.diag_add;
+  // explicit fma: single and grouped launches inline this body and must
+  // round alike
 #pragma unroll
   for (int i = 0; i < WM; i++)
 #pragma unroll
-    for (int j = 0; j < WM; j++) acc[i][j] = d4{0, 0, 0, 0};
-  const bool fast = m0 + BM <= P.M && n0 + BM <= P.N && aligned16(P.X) && aligned16(P.Y) &&
-                    (P.ldx % 2) == 0 && (P.ldy % 2) == 0;
-  if constexpr (WM == 2)
-    kloop_pf2<WM, !TX, TY>(P.X, P.ldx, m0, P.M, P.Y, P.ldy, n0, P.N, 0, P.K, fast, smem, acc);
-  else
-    kloop<WM, !TX, TY, false>(P.X, P.ldx, m0, P.M, P.Y, P.ldy, n0, P.N, 0, P.K, fast, smem,
-                              acc);
-
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int xrow0 = (w >> 1) * 16 * WM, yrow0 = (w & 1) * 16 * WM;
-  const int r = lane & 15, g = lane >> 4;
-  const double alpha = P.alpha, beta = P.beta, dadd = P.diag_add;
-  if (beta == 0.0) {
+    for (int v = 0; v < 4; v++) {
+      const int m = m0 + RM::row(i, wr, g + 4 * v);
+      if (m >= P.M) continue;
+      double *crow = P.C + (long)m * P.ldc;
 #pragma unroll
-    for (int i = 0; i < WM; i++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int m = m0 + xrow0 + i * 16 + g + 4 * v;
-        if (m >= P.M) continue;
-        double *crow = P.C + (long)m * P.ldc;
-#pragma unroll
-        for (int j = 0; j < WM; j++) {
-          const int n = n0 + yrow0 + j * 16 + r;
-          const double al = (n < P.cw) ? P.alpha_w : alpha;
-          // explicit fma: single and grouped launches inline this body and
-          // must round alike
-          if (n < P.N) crow[n] = fma(al, acc[i][j][v], (m == n) ? dadd : 0.0);
+      for (int j = 0; j < WN; j++) {
+        const int n = n0 + CM::row(j, wc, r);
+        if (n >= P.N) continue;
+        const double al = (n < P.cw) ? P.alpha_w : alpha, d = (m == n) ? dadd : 0.0;
+        if constexpr (CM::PAIR) {
+          // blocks j and j + 1 hold columns n and n + 1: one 16-byte access
+          if (j & 1) continue;
+          const int jo = j + 1 < WN ? j + 1 : j;  // j + 1, spelt so that it stays in range
+          const double al1 = (n + 1 < P.cw) ? P.alpha_w : alpha;
+          const double d1 = (m == n + 1) ? dadd : 0.0;
+          if (n + 1 < P.N) {
+            d2v o;
+            if (beta == 0.0) {
+              o[0] = fma(al, acc[i * WN + j][v], d);
+              o[1] = fma(al1, acc[i * WN + jo][v], d1);
+            } else {
+              const d2v old = *reinterpret_cast<const d2u *>(crow + n);
+              o[0] = fma(al, acc[i * WN + j][v], fma(beta, old[0], d));
+              o[1] = fma(al1, acc[i * WN + jo][v], fma(beta, old[1], d1));
+            }
+            *reinterpret_cast<d2u *>(crow + n) = o;
+            continue;
+          }
         }
+        crow[n] = (beta == 0.0) ? fma(al, acc[i * WN + j][v], d)
+                                : fma(al, acc[i * WN + j][v], fma(beta, crow[n], d));
       }
-  } else {
-#pragma unroll
-    for (int i = 0; i < WM; i++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int m = m0 + xrow0 + i * 16 + g + 4 * v;
-        if (m >= P.M) continue;
-        double *crow = P.C + (long)m * P.ldc;
-#pragma unroll
-        for (int j = 0; j < WM; j++) {
-          const int n = n0 + yrow0 + j * 16 + r;
-          const double al = (n < P.cw) ? P.alpha_w : alpha;
-          if (n < P.N)
-            crow[n] = fma(al, acc[i][j][v], fma(beta, crow[n], (m == n) ? dadd : 0.0));
-        }
-      }
-  }
+    }
 }
 
-template <bool TX, bool TY, int WM>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool TX, bool TY, class C>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 void gemm_f64_kernel(oa_gemm_problem p0, oa_gemm_problem p1, const int32_t *skip) {
   if (skip && *skip) return;
   const ProbRegs P = pick_problem(p0, p1);
-  constexpr int BM = 32 * WM;
-  __shared__ __attribute__((aligned(16))) double smem[4 * BM * LS];
-  gemm_body<TX, TY, WM>(P, xcd_logical(blockIdx.x, gridDim.x), smem);
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
+  gemm_body<TX, TY, C>(P, xcd_logical(blockIdx.x, gridDim.x), smem);
 }
 
 // ------------------------------------------------------------------ grouped
@@ -357,12 +508,11 @@ __device__ __forceinline__ void for_items(int total, F &&f) {
 
 // Many row-major NN problems in one persistent launch; items are output
 // tiles; a problem whose skip flag is set contributes no work.
-template <int WM>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <class C>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 void gemm_f64_grouped(const oa_gemm_item *__restrict__ t, const int *__restrict__ prefix,
                       int count) {
-  constexpr int BM = 32 * WM;
-  __shared__ __attribute__((aligned(16))) double smem[4 * BM * LS];
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
   for_items(prefix[count], [&](int item) {
     const int i = group_find(prefix, count, item);
     const oa_gemm_item &it = t[i];
@@ -373,8 +523,7 @@ void gemm_f64_grouped(const oa_gemm_item *__restrict__ t, const int *__restrict_
     P.C = it.p.C; P.ldc = it.p.ldc;
     P.alpha = it.p.alpha; P.beta = it.p.beta; P.diag_add = it.p.diag_add;
     P.cw = it.p.cw; P.alpha_w = it.p.alpha_w;
-    gemm_body<false, false, WM>(P, item - prefix[i], smem);
-    __syncthreads();
+    gemm_body<false, false, C>(P, item - prefix[i], smem);
   });
 }
 
@@ -405,11 +554,14 @@ __device__ __forceinline__ void upper_tile(int tile, int T, int &bi, int &bj) {
 // XY (with SYM): the upper-tile map of the symmetric product over two
 // distinct operands X and Y (the complex overlap's Im S = psi (J psi)^T,
 // whose strict upper triangle is all a Hermitian S needs).
-template <int WM, bool SYM, bool XY = false>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <class C, bool SYM, bool XY = false>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 void ovl_f64_kernel(OvlArgs a) {
-  constexpr int BM = 32 * WM;
-  __shared__ __attribute__((aligned(16))) double smem[4 * BM * LS];
+  constexpr int BM = C::BM, WM = C::WM, WN = C::WN;
+  static_assert(C::BM == C::BN, "square tiles");
+  typedef RowMap<WM, C::WR, true> RM;
+  typedef RowMap<WN, C::WC, true> CM;
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
   const int Tm = cdiv(a.M, BM), Tn = cdiv(a.N, BM);
   const int ntiles = SYM ? Tm * (Tm + 1) / 2 : Tm * Tn;
   // The short kx = 0 slice (z = 0) takes the leading workgroups, which the
@@ -438,38 +590,63 @@ void ovl_f64_kernel(OvlArgs a) {
     ka = z * a.kchunk;
     kb = min(a.K, ka + a.kchunk);
   }
-  d4 acc[WM][WM];
-#pragma unroll
-  for (int i = 0; i < WM; i++)
-#pragma unroll
-    for (int j = 0; j < WM; j++) acc[i][j] = d4{0, 0, 0, 0};
   const int m0 = bi * BM, n0 = bj * BM;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = w / C::WC, wc = w % C::WC;
+  const int r = lane & 15, g = lane >> 4;
   const double *Yp = (SYM && !XY) ? a.X : a.Y;
   const long ldy = (SYM && !XY) ? a.ldx : a.ldy;
-  const bool fast = m0 + BM <= a.M && n0 + BM <= a.N && aligned16(a.X) && aligned16(Yp) &&
-                    (a.ldx % 2) == 0 && (ldy % 2) == 0 && (ka % 2) == 0;
-  if (ka < kb) {
-    if (SYM && !XY && bi == bj)
-      kloop<WM, true, true, true>(a.X, a.ldx, m0, a.M, a.X, a.ldx, n0, a.N, ka, kb, fast, smem,
-                                  acc);
-    else
-      kloop<WM, true, true, false>(a.X, a.ldx, m0, a.M, Yp, ldy, n0, a.N, ka, kb, fast, smem,
-                                   acc);
-  }
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int xrow0 = (w >> 1) * 16 * WM, yrow0 = (w & 1) * 16 * WM;
-  const int r = lane & 15, g = lane >> 4;
   double *pt = a.part + ((long)z * ntiles + tile) * (BM * BM);
+  // blocks inside the matrix; a symmetric diagonal tile needs those on or
+  // above its diagonal
+  const bool diag = SYM && bi == bj;
+  const int nbr = min(BM / 16, cdiv(a.M - m0, 16)), nbc = min(BM / 16, cdiv(a.N - n0, 16));
+  const int nblk = diag ? nbr * (nbr + 1) / 2 : nbr * nbc;
+  d4 acc[WM * WN];
 #pragma unroll
-  for (int i = 0; i < WM; i++)
+  for (int i = 0; i < WM * WN; i++) acc[i] = d4{0, 0, 0, 0};
+  if (nblk == (BM / 16) * (BM / 16)) {
+    kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, Yp, ldy, n0, a.N, ka, kb, smem,
+                                [&](const double *Xs, const double *Ys) {
+                                  mma_rows<C, true, true, WM>(Xs, Ys, wr, wc, lane, acc);
+                                });
 #pragma unroll
-    for (int j = 0; j < WM; j++)
+    for (int i = 0; i < WM; i++)
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int lm = xrow0 + i * 16 + g + 4 * v;
-        const int ln = yrow0 + j * 16 + r;
-        pt[lm * BM + ln] = acc[i][j][v];
-      }
+      for (int j = 0; j < WN; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          pt[RM::row(i, wr, g + 4 * v) * BM + CM::row(j, wc, r)] = acc[i * WN + j][v];
+    return;
+  }
+  // the blocks of a partial tile, dealt to the waves in turn (a diagonal tile
+  // of 128 has 36 of 64: 5 MFMA chains a wave instead of 8); a wave short of
+  // one repeats the last, unstored
+  count_switch<1, WM * WN>(cdiv(nblk, C::NW), [&](auto c) {
+    constexpr int NB = decltype(c)::value;
+    int xr[NB], yr[NB];
+#pragma unroll
+    for (int t = 0; t < NB; t++) {
+      const int idx = min(w + C::NW * t, nblk - 1);
+      int rb, cb;
+      if (diag) upper_tile(idx, nbr, rb, cb);
+      else { rb = idx % nbr; cb = idx / nbr; }
+      xr[t] = rb * 16;
+      yr[t] = cb * 16;
+    }
+    auto mma = [&](const double *Xs, const double *Ys) {
+      mma_list<NB>(Xs, Ys, xr, yr, lane, acc);
+    };
+    if (diag && !XY)
+      kloop<C, true, true, true>(a.X, a.ldx, m0, a.M, a.X, a.ldx, n0, a.N, ka, kb, smem, mma);
+    else
+      kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, Yp, ldy, n0, a.N, ka, kb, smem, mma);
+#pragma unroll
+    for (int t = 0; t < NB; t++)
+      if (w + C::NW * t < nblk)
+#pragma unroll
+        for (int v = 0; v < 4; v++) pt[(xr[t] + g + 4 * v) * BM + yr[t] + r] = acc[t][v];
+  });
 }
 
 template <int WM, bool SYM>
@@ -674,9 +851,9 @@ __global__ __launch_bounds__(NT) void ns_finish_grouped(const oa_ns_args *__rest
 }
 
 template <class K>
-int grouped_grid(K kernel, int total) {
+int grouped_grid(K kernel, int total, int threads = NT) {
   int per_cu = 1;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, NT, 0) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
   static thread_local int cached_dev = -1, cached_cus = 256;
@@ -693,24 +870,28 @@ int grouped_grid(K kernel, int total) {
   return g < cap ? g : cap;
 }
 
+template <bool TX, bool TY, class C>
+void launch_gemm_tile(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_t *skip) {
+  int tiles = 0;
+  for (int i = 0; i < nprob; i++)
+    tiles = max(tiles, cdiv(p[i].M, C::BM) * cdiv(p[i].N, C::BN));
+  hipLaunchKernelGGL((gemm_f64_kernel<TX, TY, C>), dim3(cdiv(tiles, 8) * 8, nprob),
+                     dim3(C::NTHR), 0, s, p[0], p[nprob > 1 ? 1 : 0], skip);
+}
+
 template <bool TX, bool TY>
 int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_t *skip) {
-  int tiles128 = 0;
-  for (int i = 0; i < nprob; i++)
-    tiles128 = max(tiles128, cdiv(p[i].M, 128) * cdiv(p[i].N, 128));
-  const oa_gemm_problem p0 = p[0], p1 = p[nprob > 1 ? 1 : 0];
-  if (tiles128 * nprob >= 512) {
-    const int nb = cdiv(tiles128, 8) * 8;
-    hipLaunchKernelGGL((gemm_f64_kernel<TX, TY, 4>), dim3(nb, nprob), dim3(NT), 0, s, p0, p1,
-                       skip);
-  } else {
-    int tiles64 = 0;
-    for (int i = 0; i < nprob; i++)
-      tiles64 = max(tiles64, cdiv(p[i].M, 64) * cdiv(p[i].N, 64));
-    const int nb = cdiv(tiles64, 8) * 8;
-    hipLaunchKernelGGL((gemm_f64_kernel<TX, TY, 2>), dim3(nb, nprob), dim3(NT), 0, s, p0, p1,
-                       skip);
+  // the largest tile that still gives every CU its two workgroups (T128), then
+  // four (T64), then about one (T64W)
+  long t128 = 0, t64 = 0;
+  for (int i = 0; i < nprob; i++) {
+    t128 = max(t128, (long)cdiv(p[i].M, 128) * cdiv(p[i].N, 128));
+    t64 = max(t64, (long)cdiv(p[i].M, 64) * cdiv(p[i].N, 64));
   }
+  if (t128 * nprob >= 512) launch_gemm_tile<TX, TY, T128>(s, p, nprob, skip);
+  else if (t64 * nprob >= 1024) launch_gemm_tile<TX, TY, T64>(s, p, nprob, skip);
+  else if (t64 * nprob >= 192) launch_gemm_tile<TX, TY, T64W>(s, p, nprob, skip);
+  else launch_gemm_tile<TX, TY, T32>(s, p, nprob, skip);
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
@@ -817,16 +998,16 @@ size_t oa_ntsplit_f64_ws_bytes(int M, int N, int K) {
   return (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double) + 256;
 }
 
-template <int WM, bool SYM, bool XY = false>
+template <class T, bool SYM, bool XY = false>
 static int launch_ovl(hipStream_t s, const OvlPlan &pl, OvlArgs a, int M, int N, int kx0_end,
                       double alpha, double *C, long ldc, double diag,
                       unsigned long long *maxdev) {
   const int nkx = kx0_end > 0 ? cdiv(pl.ntiles, 8) * 8 : 0;
   const int nb = nkx + cdiv(pl.ntiles * pl.nz_main, 8) * 8;
-  hipLaunchKernelGGL((ovl_f64_kernel<WM, SYM, XY>), dim3(nb), dim3(NT), 0, s, a);
+  hipLaunchKernelGGL((ovl_f64_kernel<T, SYM, XY>), dim3(nb), dim3(T::NTHR), 0, s, a);
   if (maxdev) hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(64), 0, s, maxdev, 0ull, 1);
   const long total = (long)pl.ntiles * pl.BM * pl.BM;
-  hipLaunchKernelGGL((ovl_reduce_kernel<WM, SYM>), dim3((unsigned)cdiv((int)total, NT)),
+  hipLaunchKernelGGL((ovl_reduce_kernel<T::BM / 32, SYM>), dim3((unsigned)cdiv((int)total, NT)),
                      dim3(NT), 0, s, (const double *)a.part, M, N, pl.nz,
                      kx0_end > 0 ? 1 : 0, alpha, C, ldc, diag, maxdev);
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
@@ -844,8 +1025,8 @@ int oa_launch_overlap_f64(hipStream_t s, int n, int K, const double *psi, long l
   a.kx0_end = kx0_end; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
   a.part = (double *)ws;
   unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
-  if (pl.WM == 4) return launch_ovl<4, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
-  return launch_ovl<2, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
+  if (pl.WM == 4) return launch_ovl<T128, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
+  return launch_ovl<T64, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
 }
 
 int oa_launch_overlap_f64_fit(hipStream_t s, int n, int K, const double *psi, long ld,
@@ -859,8 +1040,8 @@ int oa_launch_overlap_f64_fit(hipStream_t s, int n, int K, const double *psi, lo
   a.kx0_end = kx0_end; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
   a.part = (double *)ws;
   unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
-  if (pl.WM == 4) return launch_ovl<4, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
-  return launch_ovl<2, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
+  if (pl.WM == 4) return launch_ovl<T128, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
+  return launch_ovl<T64, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
 }
 
 int oa_launch_ntsplit_f64(hipStream_t s, int M, int N, int K, const double *X, long ldx,
@@ -874,8 +1055,8 @@ int oa_launch_ntsplit_f64(hipStream_t s, int M, int N, int K, const double *X, l
   a.M = M; a.N = N; a.K = K;
   a.kx0_end = 0; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
   a.part = (double *)ws;
-  if (pl.WM == 4) return launch_ovl<4, false>(s, pl, a, M, N, 0, alpha, C, ldc, 0.0, nullptr);
-  return launch_ovl<2, false>(s, pl, a, M, N, 0, alpha, C, ldc, 0.0, nullptr);
+  if (pl.WM == 4) return launch_ovl<T128, false>(s, pl, a, M, N, 0, alpha, C, ldc, 0.0, nullptr);
+  return launch_ovl<T64, false>(s, pl, a, M, N, 0, alpha, C, ldc, 0.0, nullptr);
 }
 
 int oa_launch_overlap_xy_f64(hipStream_t s, int n, int K, const double *X, long ldx,
@@ -889,8 +1070,8 @@ int oa_launch_overlap_xy_f64(hipStream_t s, int n, int K, const double *X, long 
   a.M = n; a.N = n; a.K = K;
   a.kx0_end = 0; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
   a.part = (double *)ws;
-  if (pl.WM == 4) return launch_ovl<4, true, true>(s, pl, a, n, n, 0, alpha, C, n, 0.0, nullptr);
-  return launch_ovl<2, true, true>(s, pl, a, n, n, 0, alpha, C, n, 0.0, nullptr);
+  if (pl.WM == 4) return launch_ovl<T128, true, true>(s, pl, a, n, n, 0, alpha, C, n, 0.0, nullptr);
+  return launch_ovl<T64, true, true>(s, pl, a, n, n, 0, alpha, C, n, 0.0, nullptr);
 }
 
 size_t oa_ns_ws_bytes(int n) {
@@ -969,11 +1150,13 @@ int oa_gemm_grouped(hipStream_t s, int wm, const oa_group &g) {
   if (g.count <= 0 || g.total <= 0) return OA_SUCCESS;
   const oa_gemm_item *t = reinterpret_cast<const oa_gemm_item *>(g.args);
   if (wm == 4)
-    hipLaunchKernelGGL(gemm_f64_grouped<4>, dim3(grouped_grid(gemm_f64_grouped<4>, g.total)),
-                       dim3(NT), 0, s, t, g.prefix, g.count);
+    hipLaunchKernelGGL(gemm_f64_grouped<T128>,
+                       dim3(grouped_grid(gemm_f64_grouped<T128>, g.total, T128::NTHR)),
+                       dim3(T128::NTHR), 0, s, t, g.prefix, g.count);
   else if (wm == 2)
-    hipLaunchKernelGGL(gemm_f64_grouped<2>, dim3(grouped_grid(gemm_f64_grouped<2>, g.total)),
-                       dim3(NT), 0, s, t, g.prefix, g.count);
+    hipLaunchKernelGGL(gemm_f64_grouped<T64W>,
+                       dim3(grouped_grid(gemm_f64_grouped<T64W>, g.total, T64W::NTHR)),
+                       dim3(T64W::NTHR), 0, s, t, g.prefix, g.count);
   else
     return OA_ERR_UNSUPPORTED;
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;

@@ -329,3 +329,21 @@ enum oa_ns_phase { OA_NS_INIT = 0, OA_NS_RESID0, OA_NS_RESID1, OA_NS_UPDATE, OA_
 int oa_gemm_grouped(hipStream_t s, int wm, const oa_group &g);
 int oa_ns_grouped(hipStream_t s, int phase, const oa_group &g);
 int oa_ns_items(int phase, int n, int nwg);
+
+// ---------------------------------------------------------------- device
+// s_waitcnt with vmcnt = N and the other counters left at their maximum.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// Workgroup barrier of the LDS ring.  __syncthreads() carries a workgroup
+// fence, for which the compiler drains every vector memory operation of the
+// wave (vmcnt(0)) before s_barrier: the direct-to-LDS loads of the stages
+// meant to stay in flight would be waited for at every stage.  The ring only
+// needs the wave's own LDS reads finished (lgkmcnt(0)) before the barrier;
+// the loads of a stage are awaited with wait_vm before it is read.  The
+// memory clobber keeps the compiler from moving LDS accesses across it.
+__device__ __forceinline__ void ring_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}

@@ -668,23 +668,6 @@ __device__ __forceinline__ void digit_stage(const char *Xs, const char *Ys, int 
   }
 }
 
-// s_waitcnt with vmcnt = N and the other counters left at their maximum.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-// Workgroup barrier of the LDS ring.  __syncthreads() carries a workgroup
-// fence, for which the compiler drains every vector memory operation of the
-// wave (vmcnt(0)) before s_barrier: the direct-to-LDS loads of the stages
-// meant to stay in flight would be waited for at every stage.  The ring only
-// needs the wave's own LDS reads finished (lgkmcnt(0)) before the barrier;
-// the loads of a stage are awaited with wait_vm before it is read.  The
-// memory clobber keeps the compiler from moving LDS accesses across it.
-__device__ __forceinline__ void ring_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // Digits of DB for 4 consecutive contraction rows (one dword group for int8,
 // one 8-byte group for 16-bit digits).
 template <int DT>

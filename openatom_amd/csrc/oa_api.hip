@@ -448,24 +448,28 @@ int oa_lambda(oa_handle_t c, int n, int npw, const double *psi, long ldpsi, cons
 
 int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
                    double *T, int *iters, double *err, void *ws, oa_ns_report *rep) {
-  int st = oa_ns_begin(c->stream, n, S, nspin, rep, ws);
+  oa_ns_args a;
+  oa_ns_fill(n, S, nspin, tol, maxit, T, rep, c->host_report, ws, &a);
+  c->host_report->done = 0;
+  int st = oa_ns_begin(c->stream, a);
   if (st) return st;
-  // Host loop with early exit: two guarded iterations per report read.
-  int it = 0;
-  for (;;) {
-    const int upto = (it + 2 < maxit) ? it + 2 : maxit;
-    for (; it < upto; it++) {
-      st = oa_ns_iterate(c->stream, n, it, tol, maxit, rep, ws);
+  // Host loop with early exit.  States a step away from orthonormal take
+  // three iterations (quadratic convergence), so the first look comes there.
+  for (int it = 1, look = 3;; look += 2) {
+    for (; it < look && it < maxit; it++) {
+      st = oa_ns_check(c->stream, a, it);
+      if (st == OA_SUCCESS) st = oa_ns_iterate(c->stream, a, it);
       if (st) return st;
     }
-    OA_HIP_CHECK(hipMemcpyAsync(c->host_report, rep, sizeof(oa_ns_report),
-                                hipMemcpyDeviceToHost, c->stream));
+    if (it > 1) st = oa_ns_check(c->stream, a, it);
+    if (st) return st;
     OA_HIP_CHECK(hipStreamSynchronize(c->stream));
     if (c->host_report->done || it >= maxit) break;
+    // C for the next iteration is formed already
+    st = oa_ns_iterate(c->stream, a, it);
+    if (st) return st;
+    it++;
   }
-  st = oa_ns_finish(c->stream, n, T, rep, ws);
-  if (st) return st;
-  OA_HIP_CHECK(hipStreamSynchronize(c->stream));
   if (iters) *iters = c->host_report->iterations;
   if (err) *err = c->host_report->error;
   return c->host_report->done ? c->host_report->status : OA_ERR_NOT_CONVERGED;

@@ -10,9 +10,9 @@
 // Sequence of one step (split precision):
 //   fill counters -> chunk max -> (adaptive: slice counts) -> slice ->
 //   overlap digit products (one launch per digit tile in use) -> reduce ->
-//   S->T init -> maxit x (GEMM C = 3I - AB, GEMM pair B' = BC/2,
-//   A' = CA/2, residual, update) -> finish -> slice T -> back-multiply
-//   digit products.
+//   S->T init and B' = BC/2 (the first iteration) -> (maxit - 1) x (residual
+//   check with GEMM C = 3I - AB, GEMM pair B' = BC/2, A' = CA/2) -> last
+//   check -> slice T -> back-multiply digit products.
 // FP64: the overlap and the back-multiply are per-instance FP64-MFMA launches
 // inside the same sequence; S->T is grouped as above.
 // Every launch reads device tables built at plan time; the sequence performs
@@ -28,8 +28,6 @@
 #include "oa_internal.h"
 
 namespace {
-
-constexpr int NS_NWG = 128;  // residual partial sums per instance (same order as oa_ns_iterate)
 
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 int cdivi(long a, long b) { return (int)((a + b - 1) / b); }
@@ -52,10 +50,11 @@ struct DevGuard {
   }
 };
 
-enum LaunchKind { LK_FILL = 0, LK_SPLIT, LK_GEMM, LK_NS, LK_F64_OVL, LK_F64_BACK };
+enum LaunchKind { LK_FILL = 0, LK_SPLIT, LK_NS, LK_F64_OVL, LK_F64_BACK };
 
 struct Launch {
   int kind, phase, variant;
+  int it;         // LK_NS: iterations done
   oa_group g;     // device tables (grouped kinds)
   int inst;       // per-instance kinds
 };
@@ -136,7 +135,7 @@ int grow(oa_workspace &w, size_t bytes) {
   return OA_SUCCESS;
 }
 
-size_t ns_bytes(int n) { return align256((size_t)5 * n * n * 8) + align256(NS_NWG * 8); }
+size_t ns_bytes(int n) { return align256(oa_ns_ws_bytes(n)); }
 
 size_t inst_bytes(int n, int npw, int prec, int tile, bool need_S, bool need_T) {
   const int K = 2 * npw;
@@ -196,8 +195,7 @@ int run_seq(oa_batch *b, hipStream_t s) {
     switch (L.kind) {
       case LK_FILL: st = oa_fill_u64(s, b->counters, b->ncounters); break;
       case LK_SPLIT: st = oa_split_grouped(s, b->prec, L.variant, L.phase, L.g); break;
-      case LK_GEMM: st = oa_gemm_grouped(s, L.variant, L.g); break;
-      case LK_NS: st = oa_ns_grouped(s, L.phase, L.g); break;
+      case LK_NS: st = oa_ns_grouped(s, L.phase, L.variant, L.it, L.g); break;
       case LK_F64_OVL: {
         const InstPlan &p = b->ip[L.inst];
         st = oa_launch_overlap_f64(s, p.n, p.K, p.psi, p.ld, p.kx0_end, 2.0, p.S, 0.0, nullptr,
@@ -355,85 +353,43 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
       b->seq.push_back(L);
     }
   }
-  // S->T, grouped for both precisions
+  // S->T, grouped for both precisions: one table for INIT, and per GEMM tile
+  // one for B1 / C and one for PAIR, shared by all iterations
   std::vector<oa_ns_args> na(count);
   for (int i = 0; i < count; i++) {
     const InstPlan &p = b->ip[i];
-    const long nn = (long)p.n * p.n;
-    oa_ns_args &a = na[i];
-    a.S = p.S;
-    a.n = p.n;
-    a.nspin = p.nspin;
-    a.A[0] = p.ns_ws;
-    a.A[1] = p.ns_ws + nn;
-    a.B[0] = p.ns_ws + 2 * nn;
-    a.B[1] = p.ns_ws + 3 * nn;
-    a.C = p.ns_ws + 4 * nn;
-    a.partial = (double *)((char *)p.ns_ws + align256((size_t)5 * nn * 8));
-    a.nwg = NS_NWG;
-    a.maxit = p.maxit;
-    a.tol = p.tol;
-    a.T = p.T;
-    a.rep = drep + i;
+    oa_ns_fill(p.n, p.S, p.nspin, p.tol, p.maxit, p.T, drep + i, nullptr, p.ns_ws, &na[i]);
   }
-  auto ns_group = [&](int phase) {
-    add_group<oa_ns_args>(
-        blob, b->seq, LK_NS, phase, 0, b->ip, [&](const InstPlan &, int i) { return na[i]; },
-        [&](const InstPlan &p, int) { return oa_ns_items(phase, p.n, NS_NWG); }, all, fix);
-  };
-  ns_group(OA_NS_INIT);
-  for (int it = 0; it < b->maxit; it++) {
-    const int cur = it & 1, nxt = cur ^ 1;
-    // do_iteration (ortho.C:848-870): C = 3I - A*B
-    for (int wm : {4, 2}) {
-      auto sel = [wm, it](const InstPlan &p) { return p.wm == wm && it < p.maxit; };
-      add_group<oa_gemm_item>(
-          blob, b->seq, LK_GEMM, 0, wm, b->ip,
-          [&](const InstPlan &p, int i) {
-            const oa_ns_args &a = na[i];
-            oa_gemm_item g;
-            g.p = oa_gemm_problem{p.n, p.n, p.n, a.A[cur], p.n, a.B[cur], p.n, a.C, p.n,
-                                  -1.0, 0.0, 3.0};
-            g.skip = &a.rep->done;
-            return g;
-          },
-          [&](const InstPlan &p, int) { return cdivi(p.n, 32 * wm) * cdivi(p.n, 32 * wm); },
-          sel, fix);
-    }
-    // step_2 / step_3 (ortho.C:880-929): B' = B*C/2 ; A' = C*A/2 (two
-    // problems per instance in one table)
-    for (int wm : {4, 2}) {
-      std::vector<oa_gemm_item> g2;
-      std::vector<int> prefix(1, 0);
-      for (int i = 0; i < count; i++) {
-        const InstPlan &p = b->ip[i];
-        if (p.wm != wm || it >= p.maxit) continue;
-        const oa_ns_args &a = na[i];
-        const int tiles = cdivi(p.n, 32 * wm) * cdivi(p.n, 32 * wm);
-        oa_gemm_item x;
-        x.skip = &a.rep->done;
-        x.p = oa_gemm_problem{p.n, p.n, p.n, a.B[cur], p.n, a.C, p.n, a.B[nxt], p.n, 0.5, 0.0, 0.0};
-        g2.push_back(x);
-        prefix.push_back(prefix.back() + tiles);
-        x.p = oa_gemm_problem{p.n, p.n, p.n, a.C, p.n, a.A[cur], p.n, a.A[nxt], p.n, 0.5, 0.0, 0.0};
-        g2.push_back(x);
-        prefix.push_back(prefix.back() + tiles);
-      }
-      if (g2.empty()) continue;
-      Launch L{};
-      L.kind = LK_GEMM;
-      L.variant = wm;
-      L.g.count = (int)g2.size();
-      L.g.total = prefix.back();
-      L.g.args = reinterpret_cast<const void *>(blob.put(g2.data(), g2.size() * sizeof(oa_gemm_item)));
-      L.g.prefix = reinterpret_cast<const int *>(blob.put(prefix.data(), prefix.size() * sizeof(int)));
+  auto ns_args = [&](const InstPlan &, int i) { return na[i]; };
+  add_group<oa_ns_args>(
+      blob, b->seq, LK_NS, OA_NS_INIT, 0, b->ip, ns_args,
+      [&](const InstPlan &p, int) { return oa_ns_items(OA_NS_INIT, p.n, 0); }, all, fix);
+  std::vector<Launch> ones, pairs;  // per tile: the launches repeated below
+  const size_t ns_at = b->seq.size(), fix_at = fix.size();
+  for (int phase : {OA_NS_B1, OA_NS_PAIR})
+    for (int wm : {4, 2})
+      add_group<oa_ns_args>(
+          blob, b->seq, LK_NS, phase, wm, b->ip, ns_args,
+          [&](const InstPlan &p, int) { return oa_ns_items(phase, p.n, wm); },
+          [wm](const InstPlan &p) { return p.wm == wm; }, fix);
+  for (size_t k = ns_at; k < b->seq.size(); k++)
+    (b->seq[k].phase == OA_NS_B1 ? ones : pairs).push_back(b->seq[k]);
+  b->seq.resize(ns_at);
+  fix.resize(fix_at);
+  auto repeat = [&](const std::vector<Launch> &ls, int phase, int it) {
+    for (Launch L : ls) {
+      L.phase = phase;
+      L.it = it;
       fix.push_back({b->seq.size(), 0});
       b->seq.push_back(L);
     }
-    ns_group(cur == 0 ? OA_NS_RESID0 : OA_NS_RESID1);
-    ns_group(OA_NS_UPDATE);
+  };
+  repeat(ones, OA_NS_B1, 1);
+  for (int it = 1; it < b->maxit; it++) {
+    repeat(ones, OA_NS_C, it);
+    repeat(pairs, OA_NS_PAIR, it);
   }
-  ns_group(OA_NS_FINISH);
+  if (b->maxit > 1) repeat(ones, OA_NS_C, b->maxit);
   if (split) {
     add_group<oa_rows_args>(
         blob, b->seq, LK_SPLIT, OA_SP_ROWS, 128, b->ip,

@@ -7,7 +7,9 @@
 //                       all tiles for the asymmetric Lambda product).
 //   ovl_reduce_kernel   fixed-order sum of the split-K partials with the kx=0
 //                       weight, mirror to the lower triangle, max|S - d I|.
-//   ns_* kernels        guarded Newton-Schulz S->T iteration (device flags).
+//   ns_* kernels        guarded Newton-Schulz S->T iteration: one elementwise
+//                       launch and one GEMM for the first iteration, two GEMM
+//                       launches for every later one.
 //
 // What bounds the products: v_mfma_f64_16x16x4f64 (78.6 TFLOP/s nominal).  A
 // register-only loop of independent MFMAs reaches 77 TF from two or four
@@ -405,9 +407,15 @@ __device__ __forceinline__ ProbRegs pick_problem(const oa_gemm_problem &p0,
   return r;
 }
 
-// One BM x BN output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I.
-template <bool TX, bool TY, class C>
-__device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double *smem) {
+struct NoEpi {
+  __device__ __forceinline__ void operator()(int, int, double) const {}
+};
+
+// One BM x BN output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I;
+// epi(m, n, value) sees every output stored.
+template <bool TX, bool TY, class C, class Epi>
+__device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double *smem,
+                                          Epi &&epi) {
   constexpr int WM = C::WM, WN = C::WN;
   typedef RowMap<WM, C::WR, !TX> RM;
   typedef RowMap<WN, C::WC, TY> CM;
@@ -465,11 +473,15 @@ __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double
               o[1] = fma(al1, acc[i * WN + jo][v], fma(beta, old[1], d1));
             }
             *reinterpret_cast<d2u *>(crow + n) = o;
+            epi(m, n, o[0]);
+            epi(m, n + 1, o[1]);
             continue;
           }
         }
-        crow[n] = (beta == 0.0) ? fma(al, acc[i * WN + j][v], d)
-                                : fma(al, acc[i * WN + j][v], fma(beta, crow[n], d));
+        const double o = (beta == 0.0) ? fma(al, acc[i * WN + j][v], d)
+                                       : fma(al, acc[i * WN + j][v], fma(beta, crow[n], d));
+        crow[n] = o;
+        epi(m, n, o);
       }
     }
 }
@@ -480,7 +492,7 @@ void gemm_f64_kernel(oa_gemm_problem p0, oa_gemm_problem p1, const int32_t *skip
   if (skip && *skip) return;
   const ProbRegs P = pick_problem(p0, p1);
   __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
-  gemm_body<TX, TY, C>(P, xcd_logical(blockIdx.x, gridDim.x), smem);
+  gemm_body<TX, TY, C>(P, xcd_logical(blockIdx.x, gridDim.x), smem, NoEpi{});
 }
 
 // ------------------------------------------------------------------ grouped
@@ -504,27 +516,6 @@ __device__ __forceinline__ void for_items(int total, F &&f) {
     const int item = x * per + pos;
     if (item < total) f(item);
   }
-}
-
-// Many row-major NN problems in one persistent launch; items are output
-// tiles; a problem whose skip flag is set contributes no work.
-template <class C>
-__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
-void gemm_f64_grouped(const oa_gemm_item *__restrict__ t, const int *__restrict__ prefix,
-                      int count) {
-  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
-  for_items(prefix[count], [&](int item) {
-    const int i = group_find(prefix, count, item);
-    const oa_gemm_item &it = t[i];
-    if (it.skip && *it.skip) return;
-    ProbRegs P;
-    P.M = it.p.M; P.N = it.p.N; P.K = it.p.K;
-    P.X = it.p.X; P.ldx = it.p.ldx; P.Y = it.p.Y; P.ldy = it.p.ldy;
-    P.C = it.p.C; P.ldc = it.p.ldc;
-    P.alpha = it.p.alpha; P.beta = it.p.beta; P.diag_add = it.p.diag_add;
-    P.cw = it.p.cw; P.alpha_w = it.p.alpha_w;
-    gemm_body<false, false, C>(P, item - prefix[i], smem);
-  });
 }
 
 // Split-K partial products over the plane-wave index.
@@ -689,164 +680,187 @@ __global__ void fill_u64_kernel(unsigned long long *p, unsigned long long v, int
 }
 
 // ------------------------------------------------------------------ S->T
-// Ping-pong buffers A[2], B[2] and C; iteration i reads index i%2 and writes
-// 1-i%2, so the final T sits in A[iterations % 2].
-struct NsBufs {
-  double *A[2];
-  double *B[2];
-  double *C;
-  double *partial;  // NS_RES_WG doubles
-};
-constexpr int NS_RES_WG = 128;
+// Ortho's iteration (ortho.C:848-971): C = 3I - A B, B' = B C / 2, A' = C A / 2
+// until sqrt(sum (A - A')^2 / n^2) <= tol or maxit (collect_error, :109-146).
+// The matrices live in buffers of np x np (n rounded up to 16, zero padding),
+// so every product runs whole 16-byte-aligned stages whatever n.  Iteration i
+// reads A[i%2], B[i%2] and writes the other pair.
+//
+// At n <= 1024 the iteration is bound by launches and their latency, not by
+// its products (n = 128: 3 x 4 MFLOP), so its launches are few:
+//   INIT  B = S/2 or S.  A = I makes the first iteration elementwise:
+//         C = 3I - B, A' = C/2, with the residual of A' - I.
+//   B1    B' = B C / 2.
+//   C     C = 3I - A B.
+//   PAIR  B' and A' side by side; A' tiles also sum (A - A')^2 and store T.
+// A residual left as partial sums by INIT or PAIR is added up by every
+// workgroup of the next launch (B1 or C), each of which then knows by itself
+// whether the loop has ended; the first one writes the report.  T holds the
+// latest iterate throughout.  Before: four launches an iteration, of which a
+// one-thread sum of 128 partials took 5 to 9 us, and a final copy to T.
+enum NsMode { NS_B1 = 0, NS_C = 1, NS_PAIR = 2 };
 
-__global__ void ns_init_kernel(const double *__restrict__ S, int n, int nspin, double *A,
-                               double *B, oa_ns_report *rep) {
-  const long nn = (long)n * n;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < nn;
-       idx += (long)gridDim.x * blockDim.x) {
-    const int i = (int)(idx / n), j = (int)(idx % n);
-    B[idx] = (nspin == 1) ? S[idx] / 2.0 : S[idx];
-    A[idx] = (i == j) ? 1.0 : 0.0;
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    rep->iterations = 0;
-    rep->done = 0;
-    rep->status = OA_SUCCESS;
-    rep->pad = 0;
-    rep->error = 0.0;
-  }
-}
-
-// Fixed-order partial sums of (Aold - Anew)^2 (ortho.C:949-953).
-__global__ __launch_bounds__(NT) void ns_resid_kernel(const double *__restrict__ Aold,
-                                                      const double *__restrict__ Anew, long nn,
-                                                      double *partial, const int32_t *skip) {
-  if (*skip) return;
-  __shared__ double red[NT];
-  double s = 0.0;
-  for (long idx = (long)blockIdx.x * NT + threadIdx.x; idx < nn; idx += (long)gridDim.x * NT) {
-    const double d = Aold[idx] - Anew[idx];
-    s += d * d;
-  }
-  red[threadIdx.x] = s;
+// Sum of v over the workgroup in a fixed order; `red` holds one double per
+// wave.  Every thread returns the sum.
+__device__ __forceinline__ double block_sum(double v, double *red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
   __syncthreads();
-  for (int o = NT / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// Ortho::collect_error (ortho.C:109-146) on the device.
-__global__ void ns_update_kernel(const double *__restrict__ partial, int nwg, int n,
-                                 double tol, int maxit, oa_ns_report *rep) {
-  if (threadIdx.x != 0 || rep->done) return;
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
   double s = 0.0;
-  for (int i = 0; i < nwg; i++) s += partial[i];
-  const double err = sqrt(s / ((double)n * (double)n));
-  const int it = rep->iterations + 1;
-  rep->iterations = it;
-  rep->error = err;
-  if (!(err > tol && it < maxit)) {
-    rep->done = 1;
-    rep->status = (it >= maxit) ? OA_ERR_NOT_CONVERGED : OA_SUCCESS;
-  }
+  for (int w = 0; w < (int)(blockDim.x >> 6); w++) s += red[w];
+  __syncthreads();
+  return s;
 }
 
-__global__ void ns_finish_kernel(const double *__restrict__ A0, const double *__restrict__ A1,
-                                 long nn, double *T, const oa_ns_report *rep) {
-  const double *src = (rep->iterations & 1) ? A1 : A0;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < nn;
-       idx += (long)gridDim.x * blockDim.x)
-    T[idx] = src[idx];
-}
-
-// Grouped S->T bookkeeping over many instances (oa_ns_args tables).
-//   INIT   items of NT elements: B = S/2 or S, A = I, report cleared.
-//   RESID  item w < nwg: partial[w] = sum of (Aold - Anew)^2 over elements
-//          w*NT + t + j*nwg*NT (a fixed order for a given nwg).
-//   UPDATE one item per instance: Ortho::collect_error (ortho.C:109-146).
-//   FINISH items of NT elements: T = A[iterations % 2].
-__global__ __launch_bounds__(NT) void ns_init_grouped(const oa_ns_args *__restrict__ t,
-                                                      const int *__restrict__ prefix,
-                                                      int count) {
-  for_items(prefix[count], [&](int item) {
-    const int i = group_find(prefix, count, item);
-    const oa_ns_args &a = t[i];
-    const int w = item - prefix[i];
-    const long nn = (long)a.n * a.n, idx = (long)w * NT + threadIdx.x;
-    if (idx < nn) {
-      const int r = (int)(idx / a.n), c = (int)(idx % a.n);
-      a.B[0][idx] = (a.nspin == 1) ? a.S[idx] / 2.0 : a.S[idx];
-      a.A[0][idx] = (r == c) ? 1.0 : 0.0;
+// Workgroup w of nwg of the first, elementwise iteration.  A non-finite S makes the
+// residual NaN (the products of the identity with it would spread NaN), which
+// ends the loop; see NS_B1.
+__device__ __forceinline__ void ns_init_body(const oa_ns_args &a, int w, int nwg, double *red) {
+  const unsigned n = a.n, np = a.np, nn = np * np;
+  double s = 0.0;
+  for (unsigned idx = w * NT + threadIdx.x; idx < nn; idx += nwg * NT) {
+    const unsigned i = idx / np, j = idx - i * np;
+    double b = 0.0, c = 0.0, x = 0.0;
+    if (i < n && j < n) {
+      const long k = (long)i * n + j;
+      b = (a.nspin == 1) ? a.S[k] / 2.0 : a.S[k];
+      c = (i == j ? 3.0 : 0.0) - b;
+      x = 0.5 * c;
+      a.T[k] = x;
+      const double d = (i == j ? 1.0 : 0.0) - x;
+      s += (isfinite(d) || n == 1) ? d * d : __longlong_as_double(0x7ff8000000000000ll);
     }
-    if (w == 0 && threadIdx.x == 0) {
+    a.B[0][idx] = b;
+    a.C[idx] = c;
+    a.A[1][idx] = x;
+  }
+  s = block_sum(s, red);
+  if (threadIdx.x == 0) {
+    a.partial[w] = s;
+    if (w == 0) {
       a.rep->iterations = 0;
       a.rep->done = 0;
       a.rep->status = OA_SUCCESS;
       a.rep->pad = 0;
       a.rep->error = 0.0;
     }
-  });
+  }
 }
 
-template <int PAR>
-__global__ __launch_bounds__(NT) void ns_resid_grouped(const oa_ns_args *__restrict__ t,
-                                                       const int *__restrict__ prefix,
-                                                       int count) {
-  __shared__ double red[NT];
-  for_items(prefix[count], [&](int item) {
-    const int i = group_find(prefix, count, item);
-    const oa_ns_args &a = t[i];
-    if (a.rep->done) return;
-    const int w = item - prefix[i];
-    const long nn = (long)a.n * a.n;
-    const double *Aold = a.A[PAR], *Anew = a.A[PAR ^ 1];
-    double s = 0.0;
-    for (long idx = (long)w * NT + threadIdx.x; idx < nn; idx += (long)a.nwg * NT) {
-      const double d = Aold[idx] - Anew[idx];
+// Residual of the iteration `it` (1-based) from its npart partial sums;
+// returns whether the loop ends there.  `writer` stores the report.
+__device__ __forceinline__ bool ns_update(const oa_ns_args &a, int it, int npart, bool writer,
+                                          double *red, double &err) {
+  double s = 0.0;
+  for (int i = threadIdx.x; i < npart; i += blockDim.x) s += a.partial[i];
+  s = block_sum(s, red);
+  err = sqrt(s / ((double)a.n * (double)a.n));
+  const bool done = !(err > a.tol && it < a.maxit);
+  if (writer && threadIdx.x == 0) {
+    oa_ns_report r;
+    r.iterations = it;
+    r.done = done ? 1 : 0;
+    r.status = (done && it >= a.maxit) ? OA_ERR_NOT_CONVERGED : OA_SUCCESS;
+    r.pad = 0;
+    r.error = err;
+    *a.rep = r;
+    if (a.mirror) *a.mirror = r;
+  }
+  return done;
+}
+
+// Output tile `logical` of an NS_B1, NS_C or NS_PAIR launch after `it` iterations
+// (`which` of a pair: 0 = B', 1 = A').
+template <class C>
+__device__ __forceinline__ void ns_gemm_body(const oa_ns_args &a, int mode, int it, int npart,
+                                             int which, int logical, double *smem) {
+  const int t = cdiv(a.np, C::BM);
+  if (logical >= t * t) return;
+  if (mode != NS_B1 && (a.rep->done || it > a.maxit)) return;
+  if (mode == NS_B1 || (mode == NS_C && it >= 2)) {
+    double err;
+    const bool done = ns_update(a, it, npart, logical == 0, smem, err);
+    if (mode == NS_B1 && isnan(err)) {
+      // the identity's product with a non-finite S is NaN everywhere
+      const int m0 = (logical % t) * C::BM, n0 = (logical / t) * C::BN;
+      for (int e = threadIdx.x; e < C::BM * C::BN; e += C::NTHR) {
+        const int m = m0 + e / C::BN, n = n0 + e % C::BN;
+        if (m < a.n && n < a.n) a.T[(long)m * a.n + n] = err;
+      }
+    }
+    if (done) return;
+  }
+  const int cur = it & 1, nxt = cur ^ 1;
+  ProbRegs P;
+  P.M = P.N = P.K = a.np;
+  P.ldx = P.ldy = P.ldc = a.np;
+  P.beta = 0.0;
+  P.diag_add = 0.0;
+  P.cw = 0;
+  P.alpha_w = 0.0;
+  P.alpha = 0.5;
+  if (mode == NS_C) {
+    P.X = a.A[cur]; P.Y = a.B[cur]; P.C = a.C;
+    P.alpha = -1.0;
+    P.diag_add = 3.0;
+  } else if (mode == NS_B1) {
+    P.X = a.B[0]; P.Y = a.C; P.C = a.B[1];
+  } else if (which == 0) {
+    P.X = a.B[cur]; P.Y = a.C; P.C = a.B[nxt];
+  } else {
+    P.X = a.C; P.Y = a.A[cur]; P.C = a.A[nxt];
+  }
+  const bool res = mode == NS_PAIR && which == 1;
+  double s = 0.0;
+  gemm_body<false, false, C>(P, logical, smem, [&](int m, int n, double x) {
+    if (res) {
+      const double d = P.Y[(long)m * a.np + n] - x;
       s += d * d;
+      if (m < a.n && n < a.n) a.T[(long)m * a.n + n] = x;
     }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = NT / 2; o > 0; o >>= 1) {
-      if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) a.partial[w] = red[0];
-    __syncthreads();
+  });
+  if (res) {
+    s = block_sum(s, smem);
+    if (threadIdx.x == 0) a.partial[logical] = s;
+  }
+}
+
+__global__ __launch_bounds__(NT) void ns_init_kernel(oa_ns_args a) {
+  __shared__ double red[NT / 64];
+  ns_init_body(a, blockIdx.x, gridDim.x, red);
+}
+
+template <class C>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
+void ns_gemm_kernel(oa_ns_args a, int mode, int it, int npart) {
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
+  ns_gemm_body<C>(a, mode, it, npart, blockIdx.y, xcd_logical(blockIdx.x, gridDim.x), smem);
+}
+
+// The same over many instances (oa_ns_args tables): items are a.nwg INIT
+// workgroups, or the output tiles of one problem (B1, C) or two (PAIR).
+__global__ __launch_bounds__(NT) void ns_init_grouped(const oa_ns_args *__restrict__ t,
+                                                      const int *__restrict__ prefix,
+                                                      int count) {
+  __shared__ double red[NT / 64];
+  for_items(prefix[count], [&](int item) {
+    const int i = group_find(prefix, count, item);
+    ns_init_body(t[i], item - prefix[i], t[i].nwg, red);
   });
 }
 
-__global__ __launch_bounds__(NT) void ns_update_grouped(const oa_ns_args *__restrict__ t,
-                                                        const int *__restrict__ prefix,
-                                                        int count) {
+template <class C>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
+void ns_gemm_grouped(const oa_ns_args *__restrict__ t, const int *__restrict__ prefix, int count,
+                     int mode, int it) {
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
   for_items(prefix[count], [&](int item) {
     const int i = group_find(prefix, count, item);
     const oa_ns_args &a = t[i];
-    if (threadIdx.x != 0 || a.rep->done) return;
-    double s = 0.0;
-    for (int w = 0; w < a.nwg; w++) s += a.partial[w];
-    const double err = sqrt(s / ((double)a.n * (double)a.n));
-    const int it = a.rep->iterations + 1;
-    a.rep->iterations = it;
-    a.rep->error = err;
-    if (!(err > a.tol && it < a.maxit)) {
-      a.rep->done = 1;
-      a.rep->status = (it >= a.maxit) ? OA_ERR_NOT_CONVERGED : OA_SUCCESS;
-    }
-  });
-}
-
-__global__ __launch_bounds__(NT) void ns_finish_grouped(const oa_ns_args *__restrict__ t,
-                                                        const int *__restrict__ prefix,
-                                                        int count) {
-  for_items(prefix[count], [&](int item) {
-    const int i = group_find(prefix, count, item);
-    const oa_ns_args &a = t[i];
-    const long nn = (long)a.n * a.n, idx = (long)(item - prefix[i]) * NT + threadIdx.x;
-    const double *src = (a.rep->iterations & 1) ? a.A[1] : a.A[0];
-    if (idx < nn) a.T[idx] = src[idx];
+    const int tiles = cdiv(a.np, C::BM) * cdiv(a.np, C::BM), k = item - prefix[i];
+    ns_gemm_body<C>(a, mode, it, mode == NS_B1 ? a.nwg : tiles, k / tiles, k % tiles, smem);
   });
 }
 
@@ -1074,120 +1088,124 @@ int oa_launch_overlap_xy_f64(hipStream_t s, int n, int K, const double *X, long 
   return launch_ovl<T64, true, true>(s, pl, a, n, n, 0, alpha, C, n, 0.0, nullptr);
 }
 
+// Workspace of one S->T: A[2], B[2], C and the partial sums.
+static long ns_np(int n) { return (long)cdiv(n, 16) * 16; }
+static int ns_init_wg(int n) {
+  const long b = (ns_np(n) * ns_np(n) + 4 * NT - 1) / (4 * NT);
+  return (int)(b > 256 ? 256 : b);
+}
+static size_t ns_partials(int n) {
+  const size_t t = (size_t)cdiv((int)ns_np(n), 32);
+  return t * t > 256 ? t * t : 256;
+}
+
 size_t oa_ns_ws_bytes(int n) {
-  return (size_t)5 * n * n * sizeof(double) + NS_RES_WG * sizeof(double) + 256;
+  return (size_t)(5 * ns_np(n) * ns_np(n)) * sizeof(double) + ns_partials(n) * sizeof(double) +
+         256;
 }
 
-// S->T on the device in three parts so a host loop can stop early:
-// begin (B = S/2 or S, A = I, report cleared), guarded iterations, finish.
-static void ns_bufs(void *ws, int n, NsBufs &b) {
-  const long nn = (long)n * n;
+void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double *T,
+                oa_ns_report *rep, oa_ns_report *mirror, void *ws, oa_ns_args *a) {
+  const long nn = ns_np(n) * ns_np(n);
   double *base = (double *)ws;
-  b.A[0] = base;
-  b.A[1] = base + nn;
-  b.B[0] = base + 2 * nn;
-  b.B[1] = base + 3 * nn;
-  b.C = base + 4 * nn;
-  b.partial = base + 5 * nn;
+  a->S = S;
+  a->n = n;
+  a->np = (int)ns_np(n);
+  a->nspin = nspin;
+  a->A[0] = base;
+  a->A[1] = base + nn;
+  a->B[0] = base + 2 * nn;
+  a->B[1] = base + 3 * nn;
+  a->C = base + 4 * nn;
+  a->partial = base + 5 * nn;
+  a->nwg = ns_init_wg(n);
+  a->maxit = maxit;
+  a->tol = tol;
+  a->T = T;
+  a->rep = rep;
+  a->mirror = mirror;
 }
 
-int oa_ns_begin(hipStream_t s, int n, const double *S, int nspin, oa_ns_report *rep, void *ws) {
-  NsBufs b;
-  ns_bufs(ws, n, b);
-  const long nn = (long)n * n;
-  const long nblk = (nn + NT - 1) / NT;
-  const int eb = (int)(nblk < 1 ? 1 : (nblk > 1024 ? 1024 : nblk));
-  hipLaunchKernelGGL(ns_init_kernel, dim3(eb), dim3(NT), 0, s, S, n, nspin, b.A[0], b.B[0], rep);
+template <class C>
+static void launch_ns_tile(hipStream_t s, const oa_ns_args &a, int mode, int it, int npart) {
+  const int t = cdiv(a.np, C::BM);
+  // a C launch after the last iteration only writes the report
+  const int nb = (mode == NS_C && it >= a.maxit) ? 1 : cdiv(t * t, 8) * 8;
+  hipLaunchKernelGGL(ns_gemm_kernel<C>, dim3(nb, mode == NS_PAIR ? 2 : 1), dim3(C::NTHR), 0, s,
+                     a, mode, it, npart);
+}
+
+// Tile of an S->T launch of nprob products, by the rule of launch_gemm; returns
+// its edge.
+static int ns_tile(int np, int nprob) {
+  const long t128 = (long)cdiv(np, 128) * cdiv(np, 128) * nprob;
+  const long t64 = (long)cdiv(np, 64) * cdiv(np, 64) * nprob;
+  return t128 >= 512 ? 128 : (t64 >= 192 ? 64 : 32);
+}
+
+static int launch_ns(hipStream_t s, const oa_ns_args &a, int mode, int it) {
+  const int pt = cdiv(a.np, ns_tile(a.np, 2));
+  const int npart = mode == NS_B1 ? a.nwg : pt * pt;
+  switch (ns_tile(a.np, mode == NS_PAIR ? 2 : 1)) {
+    case 128: launch_ns_tile<T128>(s, a, mode, it, npart); break;
+    case 64: launch_ns_tile<T64W>(s, a, mode, it, npart); break;
+    default: launch_ns_tile<T32>(s, a, mode, it, npart);
+  }
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
-// Iteration `it` (0-based) of Ortho::do_iteration .. collect_error; a no-op
-// once rep->done is set.
-int oa_ns_iterate(hipStream_t s, int n, int it, double tol, int maxit, oa_ns_report *rep,
-                  void *ws) {
-  NsBufs b;
-  ns_bufs(ws, n, b);
-  const long nn = (long)n * n;
-  const int32_t *skip = &rep->done;
-  const int cur = it & 1, nxt = cur ^ 1;
-  // do_iteration (ortho.C:848-870): C = 3I - A*B
-  oa_gemm_problem p1{n, n, n, b.A[cur], n, b.B[cur], n, b.C, n, -1.0, 0.0, 3.0};
-  int st = oa_launch_gemm_f64(s, false, false, &p1, 1, skip);
-  if (st) return st;
-  // step_2 / step_3 (ortho.C:880-929): B' = B*C/2 ; A' = C*A/2
-  oa_gemm_problem p2[2] = {{n, n, n, b.B[cur], n, b.C, n, b.B[nxt], n, 0.5, 0.0, 0.0},
-                           {n, n, n, b.C, n, b.A[cur], n, b.A[nxt], n, 0.5, 0.0, 0.0}};
-  st = oa_launch_gemm_f64(s, false, false, p2, 2, skip);
-  if (st) return st;
-  hipLaunchKernelGGL(ns_resid_kernel, dim3(NS_RES_WG), dim3(NT), 0, s, (const double *)b.A[cur],
-                     (const double *)b.A[nxt], nn, b.partial, skip);
-  hipLaunchKernelGGL(ns_update_kernel, dim3(1), dim3(64), 0, s, (const double *)b.partial,
-                     NS_RES_WG, n, tol, maxit, rep);
-  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+int oa_ns_begin(hipStream_t s, const oa_ns_args &a) {
+  hipLaunchKernelGGL(ns_init_kernel, dim3(a.nwg), dim3(NT), 0, s, a);
+  return launch_ns(s, a, NS_B1, 1);
 }
 
-int oa_ns_finish(hipStream_t s, int n, double *T, const oa_ns_report *rep, void *ws) {
-  NsBufs b;
-  ns_bufs(ws, n, b);
-  const long nn = (long)n * n;
-  const long nblk = (nn + NT - 1) / NT;
-  const int eb = (int)(nblk < 1 ? 1 : (nblk > 1024 ? 1024 : nblk));
-  hipLaunchKernelGGL(ns_finish_kernel, dim3(eb), dim3(NT), 0, s, (const double *)b.A[0],
-                     (const double *)b.A[1], nn, T, rep);
-  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+int oa_ns_check(hipStream_t s, const oa_ns_args &a, int it) { return launch_ns(s, a, NS_C, it); }
+
+int oa_ns_iterate(hipStream_t s, const oa_ns_args &a, int it) {
+  return launch_ns(s, a, NS_PAIR, it);
 }
 
 int oa_launch_s_to_t(hipStream_t s, int n, const double *S, int nspin, double tol, int maxit,
                      double *T, oa_ns_report *rep, void *ws) {
-  int st = oa_ns_begin(s, n, S, nspin, rep, ws);
-  for (int it = 0; it < maxit && st == OA_SUCCESS; it++)
-    st = oa_ns_iterate(s, n, it, tol, maxit, rep, ws);
-  if (st) return st;
-  return oa_ns_finish(s, n, T, rep, ws);
+  oa_ns_args a;
+  oa_ns_fill(n, S, nspin, tol, maxit, T, rep, nullptr, ws, &a);
+  int st = oa_ns_begin(s, a);
+  for (int it = 1; it < maxit && st == OA_SUCCESS; it++) {
+    st = oa_ns_check(s, a, it);
+    if (st == OA_SUCCESS) st = oa_ns_iterate(s, a, it);
+  }
+  if (st == OA_SUCCESS && maxit > 1) st = oa_ns_check(s, a, maxit);
+  return st;
 }
 
-int oa_gemm_grouped(hipStream_t s, int wm, const oa_group &g) {
-  if (g.count <= 0 || g.total <= 0) return OA_SUCCESS;
-  const oa_gemm_item *t = reinterpret_cast<const oa_gemm_item *>(g.args);
-  if (wm == 4)
-    hipLaunchKernelGGL(gemm_f64_grouped<T128>,
-                       dim3(grouped_grid(gemm_f64_grouped<T128>, g.total, T128::NTHR)),
-                       dim3(T128::NTHR), 0, s, t, g.prefix, g.count);
-  else if (wm == 2)
-    hipLaunchKernelGGL(gemm_f64_grouped<T64W>,
-                       dim3(grouped_grid(gemm_f64_grouped<T64W>, g.total, T64W::NTHR)),
-                       dim3(T64W::NTHR), 0, s, t, g.prefix, g.count);
-  else
-    return OA_ERR_UNSUPPORTED;
-  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
-}
-
-int oa_ns_items(int phase, int n, int nwg) {
-  const long nn = (long)n * n;
+int oa_ns_items(int phase, int n, int wm) {
+  if (phase == OA_NS_INIT) return ns_init_wg(n);  // has no tile
+  const int t = cdiv((int)ns_np(n), 32 * wm);
   switch (phase) {
-    case OA_NS_INIT:
-    case OA_NS_FINISH: return (int)((nn + NT - 1) / NT);
-    case OA_NS_RESID0:
-    case OA_NS_RESID1: return nwg;
-    case OA_NS_UPDATE: return 1;
+    case OA_NS_B1:
+    case OA_NS_C: return t * t;
+    case OA_NS_PAIR: return 2 * t * t;
   }
   return 0;
 }
 
-int oa_ns_grouped(hipStream_t s, int phase, const oa_group &g) {
+template <class C>
+static void launch_ns_grouped(hipStream_t s, const oa_group &g, int mode, int it) {
+  hipLaunchKernelGGL(ns_gemm_grouped<C>, dim3(grouped_grid(ns_gemm_grouped<C>, g.total, C::NTHR)),
+                     dim3(C::NTHR), 0, s, reinterpret_cast<const oa_ns_args *>(g.args), g.prefix,
+                     g.count, mode, it);
+}
+
+int oa_ns_grouped(hipStream_t s, int phase, int wm, int it, const oa_group &g) {
   if (g.count <= 0 || g.total <= 0) return OA_SUCCESS;
-  const oa_ns_args *t = reinterpret_cast<const oa_ns_args *>(g.args);
-#define OA_NSG(K)                                                                      \
-  hipLaunchKernelGGL(K, dim3(grouped_grid(K, g.total)), dim3(NT), 0, s, t, g.prefix, \
-                     g.count)
-  switch (phase) {
-    case OA_NS_INIT: OA_NSG(ns_init_grouped); break;
-    case OA_NS_RESID0: OA_NSG(ns_resid_grouped<0>); break;
-    case OA_NS_RESID1: OA_NSG(ns_resid_grouped<1>); break;
-    case OA_NS_UPDATE: OA_NSG(ns_update_grouped); break;
-    case OA_NS_FINISH: OA_NSG(ns_finish_grouped); break;
-    default: return OA_ERR_UNSUPPORTED;
+  if (phase == OA_NS_INIT) {
+    hipLaunchKernelGGL(ns_init_grouped, dim3(grouped_grid(ns_init_grouped, g.total)), dim3(NT), 0,
+                       s, reinterpret_cast<const oa_ns_args *>(g.args), g.prefix, g.count);
+  } else {
+    const int mode = phase == OA_NS_B1 ? NS_B1 : (phase == OA_NS_C ? NS_C : NS_PAIR);
+    if (wm == 4) launch_ns_grouped<T128>(s, g, mode, it);
+    else if (wm == 2) launch_ns_grouped<T64W>(s, g, mode, it);
+    else return OA_ERR_UNSUPPORTED;
   }
-#undef OA_NSG
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }

@@ -53,8 +53,9 @@ int oa_ws_require(oa_context *c, size_t bytes);
 int oa_noalloc_init(int device);
 
 // Synchronous S->T on the handle's stream with the buffers at ws
-// (oa_ns_ws_bytes(n)) and the device report rep; the host reads rep through
-// the handle's pinned mirror every two iterations.
+// (oa_ns_ws_bytes(n)) and the device report rep; the kernels write every report
+// to the handle's pinned mirror too, which the host reads after three
+// iterations and then after every two.
 int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
                    double *T, int *iters, double *err, void *ws, oa_ns_report *rep);
 
@@ -130,16 +131,30 @@ int oa_launch_overlap_xy_f64(hipStream_t s, int n, int K, const double *X, long 
                              const double *Y, long ldy, double alpha, double *C, void *ws,
                              size_t ws_bytes);
 
-// S->T on the device.  Workspace: oa_ns_ws_bytes(n).  begin / iterate /
-// finish let a host loop stop early; oa_launch_s_to_t enqueues `maxit`
-// guarded iterations (no host decision, capturable).
+// S->T on the device.  Workspace: oa_ns_ws_bytes(n).  begin runs the first
+// iteration; for it = 1, 2, ... check(it) settles the report of iteration it
+// (it = 1 is settled by begin) and forms C for the next one unless the loop
+// has ended, and iterate(it) completes iteration it + 1.  All are no-ops once
+// rep->done is set; T holds the latest iterate.  A host loop may stop after any
+// check; oa_launch_s_to_t enqueues `maxit` guarded iterations (no host
+// decision, capturable).  `mirror` (may be null): a second place, such as
+// pinned host memory, that every report is written to.
+struct oa_ns_args {
+  const double *S;
+  int n, np, nspin;
+  double *A[2], *B[2], *C;
+  double *partial;
+  int nwg, maxit;
+  double tol;
+  double *T;
+  oa_ns_report *rep, *mirror;
+};
 size_t oa_ns_ws_bytes(int n);
-int oa_ns_begin(hipStream_t s, int n, const double *S, int nspin,
-                oa_ns_report *rep, void *ws);
-int oa_ns_iterate(hipStream_t s, int n, int it, double tol, int maxit,
-                  oa_ns_report *rep, void *ws);
-int oa_ns_finish(hipStream_t s, int n, double *T, const oa_ns_report *rep,
-                 void *ws);
+void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double *T,
+                oa_ns_report *rep, oa_ns_report *mirror, void *ws, oa_ns_args *a);
+int oa_ns_begin(hipStream_t s, const oa_ns_args &a);
+int oa_ns_check(hipStream_t s, const oa_ns_args &a, int it);
+int oa_ns_iterate(hipStream_t s, const oa_ns_args &a, int it);
 int oa_launch_s_to_t(hipStream_t s, int n, const double *S, int nspin,
                      double tol, int maxit, double *T, oa_ns_report *report,
                      void *ws);
@@ -309,26 +324,13 @@ int oa_launch_slice_counts(hipStream_t s, int prec, int n, int K, const double *
                            int kx0_end, void *ws, size_t ws_bytes, const int **counts,
                            int *nz, int *kchunk);
 
-// FP64 grouped kernels: GEMM (row-major NN, per-problem skip flag) and the
-// S->T bookkeeping kernels.
-struct oa_gemm_item {
-  oa_gemm_problem p;
-  const int32_t *skip;  // may be null
-};
-struct oa_ns_args {
-  const double *S;
-  int n, nspin;
-  double *A[2], *B[2], *C;
-  double *partial;
-  int nwg, maxit;
-  double tol;
-  double *T;
-  oa_ns_report *rep;
-};
-enum oa_ns_phase { OA_NS_INIT = 0, OA_NS_RESID0, OA_NS_RESID1, OA_NS_UPDATE, OA_NS_FINISH };
-int oa_gemm_grouped(hipStream_t s, int wm, const oa_group &g);
-int oa_ns_grouped(hipStream_t s, int phase, const oa_group &g);
-int oa_ns_items(int phase, int n, int nwg);
+// S->T over many instances: tables of oa_ns_args, one for every instance
+// sharing a GEMM tile (wm 4: 128, wm 2: 64); B1, C and PAIR as in the single
+// launches, `it` as in oa_ns_check / oa_ns_iterate (an instance past its own
+// maxit contributes nothing).
+enum oa_ns_phase { OA_NS_INIT = 0, OA_NS_B1, OA_NS_C, OA_NS_PAIR };
+int oa_ns_grouped(hipStream_t s, int phase, int wm, int it, const oa_group &g);
+int oa_ns_items(int phase, int n, int wm);
 
 // ---------------------------------------------------------------- device
 // s_waitcnt with vmcnt = N and the other counters left at their maximum.

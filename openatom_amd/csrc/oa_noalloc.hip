@@ -69,10 +69,16 @@ int oa_ortho_step_noalloc(oa_handle_t c, int n, int npw, const double *psi, long
     base = static_cast<char *>(scratch_dev[c->device]);
   }
   if (!base) return OA_ERR_HIP;
-  // layout: report | S->T buffers | split-K partial tiles
+  // layout: report | S->T buffers ... split-K partial tiles at the end.  The
+  // two overlap in time never (the partial tiles are summed into S before S->T
+  // begins), so they may overlap in space: the room for the partial tiles, and
+  // with it the sizes accepted and the split depth, counts 5 n^2 doubles of
+  // S->T buffers, while their rows are padded to 16.
   const size_t off_ns = al256(sizeof(oa_ns_report));
-  const size_t off_part = off_ns + al256(oa_ns_ws_bytes(n));
-  if (off_part >= OA_NOALLOC_SCRATCH_BYTES) return OA_ERR_CAPACITY;
+  const size_t off_part = off_ns + al256((size_t)5 * n * n * sizeof(double) + 1280);
+  if (off_part >= OA_NOALLOC_SCRATCH_BYTES ||
+      off_ns + oa_ns_ws_bytes(n) > OA_NOALLOC_SCRATCH_BYTES)
+    return OA_ERR_CAPACITY;
   oa_ns_report *rep = reinterpret_cast<oa_ns_report *>(base);
   void *ns = base + off_ns;
   void *part = base + off_part;

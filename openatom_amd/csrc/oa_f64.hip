@@ -44,6 +44,8 @@
 // to the wave rows in turn, so a ragged last tile drops them from every wave
 // alike; the overlap deals the blocks of a ragged or diagonal tile to its
 // waves one by one.
+#include <math.h>
+
 #include <type_traits>
 
 #include "oa_internal.h"
@@ -542,6 +544,20 @@ __device__ __forceinline__ void upper_tile(int tile, int T, int &bi, int &bj) {
   bj = b + rem;
 }
 
+// Tile (bi, bj), bi <= bj, of an upper triangle of T x T tiles: the tiles off
+// the diagonal by rows, then the diagonal ones.  The tiles of one k chunk that
+// start together then run in step and share their panels in L2 (a diagonal
+// tile is done in 5/8 of the time; between the others it let them drift).
+__device__ __forceinline__ void sym_tile(int tile, int T, int &bi, int &bj) {
+  const int off = T * (T - 1) / 2;
+  if (tile >= off) {
+    bi = bj = tile - off;
+  } else {
+    upper_tile(tile, T - 1, bi, bj);
+    bj++;
+  }
+}
+
 // XY (with SYM): the upper-tile map of the symmetric product over two
 // distinct operands X and Y (the complex overlap's Im S = psi (J psi)^T,
 // whose strict upper triangle is all a Hermitian S needs).
@@ -571,7 +587,7 @@ void ovl_f64_kernel(OvlArgs a) {
     z = logical / ntiles + hx;
   }
   int bi, bj;
-  if (SYM) upper_tile(tile, Tm, bi, bj);
+  if (SYM) sym_tile(tile, Tm, bi, bj);
   else { bi = tile % Tm; bj = tile / Tm; }
   int ka, kb;
   if (a.kx0_end > 0) {
@@ -640,38 +656,72 @@ void ovl_f64_kernel(OvlArgs a) {
   });
 }
 
-template <int WM, bool SYM>
-__global__ __launch_bounds__(NT) void ovl_reduce_kernel(const double *__restrict__ part, int M,
-                                                       int N, int nz, int has_kx0,
-                                                       double alpha, double *C, long ldc,
-                                                       double diag,
-                                                       unsigned long long *maxdev) {
-  constexpr int BM = 32 * WM;
+// C = alpha * (sum over z of the partial tiles), in a fixed order: a workgroup
+// owns 16 x 16 outputs, the four waves of z group q add z = q, q + 4, ... and
+// the groups combine in order.  (One thread adding all z of an element, one
+// load in flight at a time, took 32 us at n = 128 with 128 partials and 83 us
+// over four uneven instances; this takes 6 and 20.)  The mirror tile is written
+// from LDS, 128 bytes a row.
+//   has_kx0: z = 0 holds the leading kx0 columns and counts half.
+//   kx0_sub: every z counts fully and half the product of the leading
+//            kx0_sub columns of psi is taken off here.
+template <int BM, bool SYM>
+__global__ __launch_bounds__(1024) void ovl_reduce_kernel(const double *__restrict__ part, int M,
+                                                         int N, int nz, int has_kx0,
+                                                         int kx0_sub, const double *psi, long ld,
+                                                         double alpha, double *C, long ldc,
+                                                         double diag,
+                                                         unsigned long long *maxdev) {
+  constexpr int PB = BM / 16;  // patches per tile edge
   const int Tm = cdiv(M, BM), Tn = cdiv(N, BM);
   const int ntiles = SYM ? Tm * (Tm + 1) / 2 : Tm * Tn;
-  const long idx = (long)blockIdx.x * NT + threadIdx.x;
-  const int tile = (int)(idx / (BM * BM));
-  if (tile >= ntiles) return;
-  const int e = (int)(idx % (BM * BM));
-  const int lm = e / BM, ln = e % BM;
+  const int tile = blockIdx.x / (PB * PB), patch = blockIdx.x % (PB * PB);
   int bi, bj;
-  if (SYM) upper_tile(tile, Tm, bi, bj);
+  if (SYM) sym_tile(tile, Tm, bi, bj);
   else { bi = tile % Tm; bj = tile / Tm; }
-  if (SYM && bi == bj && ln < lm) return;
-  const int i = bi * BM + lm, j = bj * BM + ln;
-  if (i >= M || j >= N) return;
+  const int pi = (patch / PB) * 16, pj = (patch % PB) * 16;
+  if (bi * BM + pi >= M || bj * BM + pj >= N || (SYM && bi == bj && pi > pj)) return;
+  __shared__ double sums[4][256];
+  __shared__ double out[16][17];
+  const int t = threadIdx.x & 255, q = threadIdx.x >> 8;
+  const int lr = t >> 4, lc = t & 15;
+  const double *p = part + (long)tile * (BM * BM) + (pi + lr) * BM + pj + lc;
+  const long zs = (long)ntiles * (BM * BM);
   double s = 0.0;
-  for (int z = 0; z < nz; z++) {
-    const double p = part[((long)z * ntiles + tile) * (BM * BM) + e];
-    s += (has_kx0 && z == 0) ? 0.5 * p : p;
+#pragma unroll 8
+  for (int z = q; z < nz; z += 4) {
+    const double x = p[z * zs];
+    s += (has_kx0 && z == 0) ? 0.5 * x : x;
   }
-  s *= alpha;
-  C[(long)i * ldc + j] = s;
-  if (SYM) C[(long)j * ldc + i] = s;
-  if (maxdev) {
-    const double dv = fabs(s - (i == j ? diag : 0.0));
-    atomicMax(maxdev, (unsigned long long)__double_as_longlong(dv));
+  sums[q][t] = s;
+  __syncthreads();
+  const bool dpatch = SYM && bi == bj && pi == pj;  // holds part of the diagonal
+  if (q == 0) {
+    const int i = bi * BM + pi + lr, j = bj * BM + pj + lc;
+    const bool in = i < M && j < N && !(dpatch && lc < lr);
+    s = ((sums[0][t] + sums[1][t]) + sums[2][t]) + sums[3][t];
+    if (in) {
+      double g = 0.0;
+      for (int k = 0; k < kx0_sub; k++) g = fma(psi[(long)i * ld + k], psi[(long)j * ld + k], g);
+      s = alpha * fma(-0.5, g, s);
+      C[(long)i * ldc + j] = s;
+    }
+    out[lr][lc] = s;
+    if (maxdev) {
+      // on the bits of non-negative doubles; a NaN's compare above all others
+      const double dv = fabs(s - (i == j ? diag : 0.0));
+      unsigned long long u = in ? (unsigned long long)__double_as_longlong(dv) : 0ull;
+      for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long w = __shfl_xor(u, o);
+        u = w > u ? w : u;
+      }
+      if ((t & 63) == 0) atomicMax(maxdev, u);
+    }
   }
+  if (!SYM) return;
+  __syncthreads();
+  const int mi = bi * BM + pi + lc, mj = bj * BM + pj + lr;  // C[mj][mi] = out[lc][lr]
+  if (q == 0 && mi < M && mj < N && !(dpatch && lr < lc)) C[(long)mj * ldc + mi] = out[lc][lr];
 }
 
 __global__ void fill_u64_kernel(unsigned long long *p, unsigned long long v, int n) {
@@ -911,45 +961,61 @@ int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_
 
 // Split-K plan for the plane-wave products.
 struct OvlPlan {
-  int WM, BM, ntiles, nz_main, kchunk, nz;
+  int BM, ntiles, nz_main, kchunk, nz;
+  int kx0_slice;  // columns of a kx = 0 slice (z = 0), 0 for none
 };
 
-// Split depth nz for ntiles output tiles over K columns.  The main chunks go
-// to the 8 XCDs in equal contiguous ranges of cdiv(ntiles*nz, 8) workgroups,
-// of which 32 CUs x wpc are resident at once (wpc = 2 for WM = 4, whose two
-// 74 KB LDS footprints fill a CU's 160 KB; 4 for WM = 2), so a depth costs
-// rounds x cdiv(K, nz) columns of one workgroup's MFMA time (2 flops per
-// output element and column on 1/wpc of a CU's share of the FP64 MFMA peak:
-// 6.5 ps x wpc) plus writing and re-reading the nz*ntiles partial tiles
-// (16 bytes per element at about 5 TB/s: 3.2 ps); both terms are per output
-// element of a tile.  The cheapest depth wins; chunks keep at least 8 BK
-// stages.  The choice depends on (M, N, K) only, so workspace sizing and
-// launch agree for any kx = 0 split.
-int ovl_depth(int ntiles, int K, int wpc) {
+// A kx = 0 plane of at most this many columns is multiplied with the rest and
+// half its product taken off in the reduce; a wider one is a z slice of its
+// own, weighted there.
+constexpr int KX0_SUB_MAX = 32;
+
+// Split depth nz for ntiles output tiles of BM over K columns, of which the
+// blocks inside the matrix (and above the diagonal) are the fraction `fill`.
+// The chunks go to the 8 XCDs in equal contiguous ranges of w workgroups; of a
+// range, 32 CUs x wpc are resident at once (wpc = 2 for BM = 128, whose 64 KB
+// LDS footprints share a CU's 160 KB; 4 for BM = 64).  The cost of a depth:
+//   MFMA time of a CU, 2 flops per output and column at 0.3 TF (6.5 ps):
+//   whole rounds cost the work they hold (partial tiles save about a quarter of
+//   what they leave out), the last one a full tile's path; few workgroups on
+//   a CU reach only part of its rate.
+//   3 us a workgroup (first loads, partial tile).
+//   16 bytes per element of the nz*ntiles partial tiles, partly in L2.
+// Measured depths: n = 1024, npw = 262144: 14 (one round) 9.57 ms, 35 9.60, 56
+// 8.92, 71 9.05, 113 8.87; n = 512, npw = 65536: 25 0.685, 38 0.853, 51 (one
+// round) 0.659, 102 0.675, 256 0.696; n = 301, npw = 20011: 42 142 us, 85 (one
+// round) 124, 106 155, 170 150; n = 128, npw = 8192: 85 19.7, 128 22.9.
+// Chunks keep at least 8 BK stages.  The choice depends on (M, N, K) only, so
+// workspace sizing and launch agree for any kx = 0 split.
+int ovl_depth(int ntiles, int K, int BM, double fill) {
   const int nzmax = max(1, min(512, cdiv(K, 8 * BK)));
-  const long slots = 32L * wpc;
+  const int wpc = BM == 128 ? 2 : 4;
+  const double lone = BM == 128 ? 1.15 : 2.3, el = (double)BM * BM, f = 0.25 * (3.0 + fill);
+  const int slots = 32 * wpc;
   int best = 1;
   double best_cost = 0.0;
   for (int nz = 1; nz <= nzmax; nz++) {
-    const long rounds = (cdiv(ntiles * nz, 8) + slots - 1) / slots;
-    const double cost = (double)rounds * cdiv(K, nz) * wpc * 6.5 + (double)nz * ntiles * 3.2;
+    const int w = cdiv(ntiles * nz, 8), full = w / slots, rest = w % slots;
+    const double last = rest > 0 ? fmax((double)cdiv(rest, 32), lone) : wpc * (1.0 - f);
+    const double cost = cdiv(K, nz) * (wpc * full * f + last) * 6.5 * el + cdiv(w, 32) * 3e6 +
+                        (double)nz * ntiles * el * 2.5;
     if (nz == 1 || cost < best_cost) { best = nz; best_cost = cost; }
   }
   return best;
 }
 
-// max_part_bytes > 0 caps the depth so that the partial tiles (the kx = 0
-// slice included) fit that many bytes; nz_main = 0 reports that even one
-// chunk does not fit.
+// max_part_bytes > 0 caps the depth so that the partial tiles (a kx = 0 slice
+// included, whatever its width) fit that many bytes; nz_main = 0 reports that
+// even one chunk does not fit.
 OvlPlan plan_ovl(int M, int N, int K, int kx0_end, bool sym, size_t max_part_bytes = 0) {
   OvlPlan pl;
   const int t128 = sym ? cdiv(M, 128) * (cdiv(M, 128) + 1) / 2 : cdiv(M, 128) * cdiv(N, 128);
-  pl.WM = (M >= 256 || t128 >= 16) ? 4 : 2;
-  pl.BM = 32 * pl.WM;
+  pl.BM = (M >= 256 || t128 >= 16) ? 128 : 64;
   const int Tm = cdiv(M, pl.BM), Tn = cdiv(N, pl.BM);
   pl.ntiles = sym ? Tm * (Tm + 1) / 2 : Tm * Tn;
-  const int Kmain = K - kx0_end;
-  int nz = ovl_depth(pl.ntiles, max(K, 1), pl.WM == 4 ? 2 : 4);
+  const long bm = cdiv(M, 16), bn = cdiv(N, 16), bt = pl.BM / 16;
+  const double fill = (double)(sym ? bm * (bm + 1) / 2 : bm * bn) / (pl.ntiles * bt * bt);
+  int nz = ovl_depth(pl.ntiles, max(K, 1), pl.BM, fill);
   if (max_part_bytes > 0) {
     const size_t per = (size_t)pl.ntiles * pl.BM * pl.BM * sizeof(double);
     const long fit = (long)(max_part_bytes / per) - (kx0_end > 0 ? 1 : 0);
@@ -961,11 +1027,11 @@ OvlPlan plan_ovl(int M, int N, int K, int kx0_end, bool sym, size_t max_part_byt
     }
     if (nz > fit) nz = (int)fit;
   }
-  int kchunk = cdiv(cdiv(max(Kmain, 1), nz), BK) * BK;
-  nz = max(1, cdiv(max(Kmain, 1), kchunk));
-  pl.nz_main = nz;
-  pl.kchunk = kchunk;
-  pl.nz = nz + (kx0_end > 0 ? 1 : 0);
+  // the chunk length comes from K: a slice never adds more than one z
+  pl.kchunk = cdiv(cdiv(max(K, 1), nz), BK) * BK;
+  pl.kx0_slice = kx0_end > KX0_SUB_MAX ? kx0_end : 0;
+  pl.nz_main = max(1, cdiv(max(K - pl.kx0_slice, 1), pl.kchunk));
+  pl.nz = pl.nz_main + (pl.kx0_slice > 0 ? 1 : 0);
   return pl;
 }
 
@@ -1003,7 +1069,7 @@ int oa_launch_gemm_f64(hipStream_t s, bool tx, bool ty, const oa_gemm_problem *p
 
 size_t oa_overlap_f64_ws_bytes(int n, int K) {
   const OvlPlan pl = plan_ovl(n, n, K, 0, true);
-  // kx0 chunk adds one more z slice at most; maxdev slot after the partials
+  // a kx0 slice adds one z
   return (size_t)(pl.nz + 1) * pl.ntiles * pl.BM * pl.BM * sizeof(double) + 256;
 }
 
@@ -1012,80 +1078,66 @@ size_t oa_ntsplit_f64_ws_bytes(int M, int N, int K) {
   return (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double) + 256;
 }
 
-template <class T, bool SYM, bool XY = false>
-static int launch_ovl(hipStream_t s, const OvlPlan &pl, OvlArgs a, int M, int N, int kx0_end,
-                      double alpha, double *C, long ldc, double diag,
-                      unsigned long long *maxdev) {
-  const int nkx = kx0_end > 0 ? cdiv(pl.ntiles, 8) * 8 : 0;
+template <class T, bool SYM, bool XY>
+static int launch_ovl_tile(hipStream_t s, const OvlPlan &pl, const OvlArgs &a, int kx0_end,
+                           double alpha, double *C, long ldc, double diag,
+                           unsigned long long *maxdev) {
+  const int nkx = pl.kx0_slice > 0 ? cdiv(pl.ntiles, 8) * 8 : 0;
   const int nb = nkx + cdiv(pl.ntiles * pl.nz_main, 8) * 8;
   hipLaunchKernelGGL((ovl_f64_kernel<T, SYM, XY>), dim3(nb), dim3(T::NTHR), 0, s, a);
   if (maxdev) hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(64), 0, s, maxdev, 0ull, 1);
-  const long total = (long)pl.ntiles * pl.BM * pl.BM;
-  hipLaunchKernelGGL((ovl_reduce_kernel<T::BM / 32, SYM>), dim3((unsigned)cdiv((int)total, NT)),
-                     dim3(NT), 0, s, (const double *)a.part, M, N, pl.nz,
-                     kx0_end > 0 ? 1 : 0, alpha, C, ldc, diag, maxdev);
+  hipLaunchKernelGGL((ovl_reduce_kernel<T::BM, SYM>), dim3(pl.ntiles * (T::BM / 16) * (T::BM / 16)),
+                     dim3(1024), 0, s, (const double *)a.part, a.M, a.N, pl.nz,
+                     pl.kx0_slice > 0 ? 1 : 0, pl.kx0_slice > 0 ? 0 : kx0_end, a.X, a.ldx, alpha,
+                     C, ldc, diag, maxdev);
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+}
+
+// C = alpha X Y^T by the plan, the leading kx0_end columns at half weight.
+template <bool SYM, bool XY>
+static int launch_ovl(hipStream_t s, const OvlPlan &pl, int M, int N, int K, const double *X,
+                      long ldx, const double *Y, long ldy, int kx0_end, double alpha, double *C,
+                      long ldc, double diag, double *maxdev, void *ws, size_t ws_bytes) {
+  if (pl.nz_main < 1 ||
+      (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double) > ws_bytes)
+    return OA_ERR_CAPACITY;
+  OvlArgs a;
+  a.X = X; a.ldx = ldx; a.Y = Y; a.ldy = ldy;
+  a.M = M; a.N = N; a.K = K;
+  a.kx0_end = pl.kx0_slice; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
+  a.part = (double *)ws;
+  unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
+  if (pl.BM == 128)
+    return launch_ovl_tile<T128, SYM, XY>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
+  return launch_ovl_tile<T64, SYM, XY>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
 }
 
 int oa_launch_overlap_f64(hipStream_t s, int n, int K, const double *psi, long ld, int kx0_end,
                           double alpha, double *S, double diag, double *maxdev, void *ws,
                           size_t ws_bytes) {
-  const OvlPlan pl = plan_ovl(n, n, K, kx0_end, true);
-  const size_t need = (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double);
-  if (need > ws_bytes) return OA_ERR_CAPACITY;
-  OvlArgs a;
-  a.X = psi; a.ldx = ld; a.Y = psi; a.ldy = ld;
-  a.M = n; a.N = n; a.K = K;
-  a.kx0_end = kx0_end; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
-  a.part = (double *)ws;
-  unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
-  if (pl.WM == 4) return launch_ovl<T128, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
-  return launch_ovl<T64, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
+  return launch_ovl<true, false>(s, plan_ovl(n, n, K, kx0_end, true), n, n, K, psi, ld, psi, ld,
+                                 kx0_end, alpha, S, n, diag, maxdev, ws, ws_bytes);
 }
 
 int oa_launch_overlap_f64_fit(hipStream_t s, int n, int K, const double *psi, long ld,
                               int kx0_end, double alpha, double *S, double diag,
                               double *maxdev, void *ws, size_t ws_bytes) {
-  const OvlPlan pl = plan_ovl(n, n, K, kx0_end, true, ws_bytes);
-  if (pl.nz_main < 1) return OA_ERR_CAPACITY;
-  OvlArgs a;
-  a.X = psi; a.ldx = ld; a.Y = psi; a.ldy = ld;
-  a.M = n; a.N = n; a.K = K;
-  a.kx0_end = kx0_end; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
-  a.part = (double *)ws;
-  unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
-  if (pl.WM == 4) return launch_ovl<T128, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
-  return launch_ovl<T64, true>(s, pl, a, n, n, kx0_end, alpha, S, n, diag, md);
+  return launch_ovl<true, false>(s, plan_ovl(n, n, K, kx0_end, true, ws_bytes), n, n, K, psi, ld,
+                                 psi, ld, kx0_end, alpha, S, n, diag, maxdev, ws, ws_bytes);
 }
 
 int oa_launch_ntsplit_f64(hipStream_t s, int M, int N, int K, const double *X, long ldx,
                           const double *Y, long ldy, double alpha, double *C, long ldc, void *ws,
                           size_t ws_bytes) {
-  const OvlPlan pl = plan_ovl(M, N, K, 0, false);
-  const size_t need = (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double);
-  if (need > ws_bytes) return OA_ERR_CAPACITY;
-  OvlArgs a;
-  a.X = X; a.ldx = ldx; a.Y = Y; a.ldy = ldy;
-  a.M = M; a.N = N; a.K = K;
-  a.kx0_end = 0; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
-  a.part = (double *)ws;
-  if (pl.WM == 4) return launch_ovl<T128, false>(s, pl, a, M, N, 0, alpha, C, ldc, 0.0, nullptr);
-  return launch_ovl<T64, false>(s, pl, a, M, N, 0, alpha, C, ldc, 0.0, nullptr);
+  return launch_ovl<false, false>(s, plan_ovl(M, N, K, 0, false), M, N, K, X, ldx, Y, ldy, 0,
+                                  alpha, C, ldc, 0.0, nullptr, ws, ws_bytes);
 }
 
 int oa_launch_overlap_xy_f64(hipStream_t s, int n, int K, const double *X, long ldx,
                              const double *Y, long ldy, double alpha, double *C, void *ws,
                              size_t ws_bytes) {
-  const OvlPlan pl = plan_ovl(n, n, K, 0, true);
-  const size_t need = (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double);
-  if (need > ws_bytes) return OA_ERR_CAPACITY;
-  OvlArgs a;
-  a.X = X; a.ldx = ldx; a.Y = Y; a.ldy = ldy;
-  a.M = n; a.N = n; a.K = K;
-  a.kx0_end = 0; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
-  a.part = (double *)ws;
-  if (pl.WM == 4) return launch_ovl<T128, true, true>(s, pl, a, n, n, 0, alpha, C, n, 0.0, nullptr);
-  return launch_ovl<T64, true, true>(s, pl, a, n, n, 0, alpha, C, n, 0.0, nullptr);
+  return launch_ovl<true, true>(s, plan_ovl(n, n, K, 0, true), n, n, K, X, ldx, Y, ldy, 0, alpha,
+                                C, n, 0.0, nullptr, ws, ws_bytes);
 }
 
 // Workspace of one S->T: A[2], B[2], C and the partial sums.

@@ -97,3 +97,26 @@ def test_tile_choice_keeps_the_sum_order(handle):
         part = handle.backmul(T, psi[:, :cols])
         torch.cuda.synchronize()
         assert torch.equal(part, full[:, :cols]), cols
+
+
+@pytest.mark.parametrize("n,npw,nkx0", [(40, 700, 0), (40, 700, 16), (40, 700, 17), (17, 90, 90),
+                                        (130, 1501, 16), (301, 20011, 17), (301, 20011, 413),
+                                        (300, 5000, 4999)])
+def test_overlap_kx0_plane_and_maxdev(handle, n, npw, nkx0):
+    """A kx = 0 plane of up to 32 columns comes off in the reduce, a wider one
+    is a slice of its own; max|S - d I| from the reduce.  The subtraction adds
+    one rounding of the half product to the bound."""
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(n + npw)
+    psi = torch.randn((n, 2 * npw), generator=gen, dtype=torch.float64, device=DEV)
+    md = torch.zeros(1, dtype=torch.float64, device=DEV)
+    S = handle.overlap_sym(psi, nkx0=nkx0, alpha=2.0, diag=1.5, maxdev=md)
+    torch.cuda.synchronize()
+    w = torch.full((2 * npw,), 2.0, dtype=torch.float64, device=DEV)
+    w[:2 * nkx0] = 1.0
+    want = (psi * w) @ psi.T
+    bound = (2 * npw + 10) * EPS * 2.0 * (psi.abs() @ psi.abs().T)
+    assert bool(((S - want).abs() <= bound).all()), float(((S - want).abs() / bound).max())
+    assert torch.equal(S, S.T)
+    eye = torch.eye(n, dtype=torch.float64, device=DEV)
+    assert float(md) == float((S - 1.5 * eye).abs().max())

@@ -945,14 +945,19 @@ void launch_gemm_tile(hipStream_t s, const oa_gemm_problem *p, int nprob, const 
 
 template <bool TX, bool TY>
 int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_t *skip) {
-  // the largest tile that still gives every CU its two workgroups (T128), then
-  // four (T64), then about one (T64W)
+  // The largest tile that still gives every CU its two workgroups (T128), then
+  // four (T64), then about one (T64W).  A ragged 128 tile costs almost a whole
+  // one (its shorter stages wait for their loads), a 64 tile's MFMAs 1.1 times
+  // as much: T psi at n = 301 (npw 20011) 161 us with T128, 142 with T64; n =
+  // 448 (40000) 555 / 523; n = 192 (30000) 106 / 79; but n = 384 (40000) 386 /
+  // 389; n = 777 (50021) 1946 / 2135; n = 96 (60000) 51 / 60.
   long t128 = 0, t64 = 0;
   for (int i = 0; i < nprob; i++) {
     t128 = max(t128, (long)cdiv(p[i].M, 128) * cdiv(p[i].N, 128));
     t64 = max(t64, (long)cdiv(p[i].M, 64) * cdiv(p[i].N, 64));
   }
-  if (t128 * nprob >= 512) launch_gemm_tile<TX, TY, T128>(s, p, nprob, skip);
+  const bool ragged = 40 * t128 > 11 * t64;  // 128^2 t128 > 1.1 * 64^2 t64
+  if (t128 * nprob >= 512 && !ragged) launch_gemm_tile<TX, TY, T128>(s, p, nprob, skip);
   else if (t64 * nprob >= 1024) launch_gemm_tile<TX, TY, T64>(s, p, nprob, skip);
   else if (t64 * nprob >= 192) launch_gemm_tile<TX, TY, T64W>(s, p, nprob, skip);
   else launch_gemm_tile<TX, TY, T32>(s, p, nprob, skip);
@@ -976,28 +981,30 @@ constexpr int KX0_SUB_MAX = 32;
 // range, 32 CUs x wpc are resident at once (wpc = 2 for BM = 128, whose 64 KB
 // LDS footprints share a CU's 160 KB; 4 for BM = 64).  The cost of a depth:
 //   MFMA time of a CU, 2 flops per output and column at 0.3 TF (6.5 ps):
-//   whole rounds cost the work they hold (partial tiles save about a quarter of
-//   what they leave out), the last one a full tile's path; few workgroups on
-//   a CU reach only part of its rate.
-//   3 us a workgroup (first loads, partial tile).
+//   whole rounds cost the work they hold (partial tiles save a quarter, at
+//   BM = 64 half, of what they leave out), the last one a full tile's path;
+//   few workgroups on a CU reach only part of its rate.
+//   2 to 3 us a workgroup (first loads, partial tile).
 //   16 bytes per element of the nz*ntiles partial tiles, partly in L2.
-// Measured depths: n = 1024, npw = 262144: 14 (one round) 9.57 ms, 35 9.60, 56
-// 8.92, 71 9.05, 113 8.87; n = 512, npw = 65536: 25 0.685, 38 0.853, 51 (one
-// round) 0.659, 102 0.675, 256 0.696; n = 301, npw = 20011: 42 142 us, 85 (one
-// round) 124, 106 155, 170 150; n = 128, npw = 8192: 85 19.7, 128 22.9.
+// Measured depths, 128 tiles: n = 1024, npw = 262144: 14 (one round) 9.57 ms,
+// 35 9.60, 56 8.92, 71 9.05, 113 8.87; n = 512, npw = 65536: 25 0.685, 38
+// 0.853, 51 (one round) 0.659, 102 0.675, 256 0.696.  64 tiles: n = 777, npw =
+// 50021: 11 1.247, 22 1.195, 45 1.131, 90 1.136; n = 301, npw = 20011: 34 93
+// us, 51 92, 68 89, 136 95; n = 128, npw = 8192: 85 19.7, 128 22.9.
 // Chunks keep at least 8 BK stages.  The choice depends on (M, N, K) only, so
 // workspace sizing and launch agree for any kx = 0 split.
 int ovl_depth(int ntiles, int K, int BM, double fill) {
   const int nzmax = max(1, min(512, cdiv(K, 8 * BK)));
-  const int wpc = BM == 128 ? 2 : 4;
-  const double lone = BM == 128 ? 1.15 : 2.3, el = (double)BM * BM, f = 0.25 * (3.0 + fill);
-  const int slots = 32 * wpc;
+  const bool big = BM == 128;
+  const int wpc = big ? 2 : 4, slots = 32 * wpc;
+  const double lone = big ? 1.15 : 2.6, el = (double)BM * BM, start = big ? 3e6 : 2e6;
+  const double f = 1.0 - (big ? 0.25 : 0.5) * (1.0 - fill);
   int best = 1;
   double best_cost = 0.0;
   for (int nz = 1; nz <= nzmax; nz++) {
     const int w = cdiv(ntiles * nz, 8), full = w / slots, rest = w % slots;
     const double last = rest > 0 ? fmax((double)cdiv(rest, 32), lone) : wpc * (1.0 - f);
-    const double cost = cdiv(K, nz) * (wpc * full * f + last) * 6.5 * el + cdiv(w, 32) * 3e6 +
+    const double cost = cdiv(K, nz) * (wpc * full * f + last) * 6.5 * el + cdiv(w, 32) * start +
                         (double)nz * ntiles * el * 2.5;
     if (nz == 1 || cost < best_cost) { best = nz; best_cost = cost; }
   }
@@ -1009,15 +1016,25 @@ int ovl_depth(int ntiles, int K, int BM, double fill) {
 // even one chunk does not fit.
 OvlPlan plan_ovl(int M, int N, int K, int kx0_end, bool sym, size_t max_part_bytes = 0) {
   OvlPlan pl;
-  const int t128 = sym ? cdiv(M, 128) * (cdiv(M, 128) + 1) / 2 : cdiv(M, 128) * cdiv(N, 128);
-  pl.BM = (M >= 256 || t128 >= 16) ? 128 : 64;
-  const int Tm = cdiv(M, pl.BM), Tn = cdiv(N, pl.BM);
-  pl.ntiles = sym ? Tm * (Tm + 1) / 2 : Tm * Tn;
+  auto tiles = [&](int bm) {
+    const int a = cdiv(M, bm), b = cdiv(N, bm);
+    return sym ? a * (a + 1) / 2 : a * b;
+  };
+  const int t128 = tiles(128), t64 = tiles(64);
+  // A partial 128 tile costs almost a whole one, the MFMAs of 64 tiles 1.1 to
+  // 1.2 times as much.  Overlap with 128 / 64 tiles: n = 301 (npw 20011) 124 /
+  // 92 us, n = 384 (40000) 261 / 234, n = 448 (40000) 410 / 306, n = 512
+  // (65536) 657 / 666, n = 777 (50021) 1363 / 1267, n = 1024 (262144) 9.0 / 12.9
+  // ms.  Lambda: 301 198 / 145, 384 386 / 390, 448 634 / 539, 777 2212 / 2452.
+  const bool small = M < 256 && t128 < 16;
+  pl.BM = (small || t64 * (sym ? 1.12 : 1.2) < t128 * 4) ? 64 : 128;
+  pl.ntiles = pl.BM == 128 ? t128 : t64;
   const long bm = cdiv(M, 16), bn = cdiv(N, 16), bt = pl.BM / 16;
   const double fill = (double)(sym ? bm * (bm + 1) / 2 : bm * bn) / (pl.ntiles * bt * bt);
   int nz = ovl_depth(pl.ntiles, max(K, 1), pl.BM, fill);
   if (max_part_bytes > 0) {
-    const size_t per = (size_t)pl.ntiles * pl.BM * pl.BM * sizeof(double);
+    // counted in 128 tiles from M = 256 on (64 tiles never need more)
+    const size_t per = (size_t)(small ? t64 * 4096 : t128 * 16384) * sizeof(double);
     const long fit = (long)(max_part_bytes / per) - (kx0_end > 0 ? 1 : 0);
     if (fit < 1) {
       pl.nz_main = 0;

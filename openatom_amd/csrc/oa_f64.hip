@@ -69,7 +69,8 @@ __device__ __forceinline__ int xcd_logical(int b, int nb) {
 }
 
 // Tile configurations.  WPE waves per SIMD are allowed (512 / WPE registers a
-// wave); NBUF stages rotate through LDS (NBUF - 1 in flight).
+// wave).  The LDS ring has NBUF slots of GRP stages each (NBUF - 1 slots in
+// flight, one barrier per slot).
 //   T128   the large products: 64 x 32 wave tiles, two workgroups per CU.  Two
 //          stages suffice: one stage is 8192 MFMA cycles of a SIMD.  T psi at
 //          n = 1024 / 512 / 301 (npw 262144 / 65536 / 20011): 15.5 / 1.05 /
@@ -78,19 +79,23 @@ __device__ __forceinline__ int xcd_logical(int b, int nb) {
 //   T64    many small tiles: 32 x 32 wave tiles, four workgroups per CU.
 //   T64W   few tiles (about one per CU): 16 x 32 wave tiles, so that a lone
 //          workgroup still puts two waves on a SIMD.
-//   T32    fewer still: a quarter of the tile, four times the workgroups.
-template <int BM_, int BN_, int WR_, int WC_, int WPE_, int NBUF_>
+//   T32    fewer still: a quarter of the tile, four times the workgroups.  Each
+//          wave is one chain of MFMAs, of which a stage holds four: the LDS
+//          latency and the barrier are paid once per GRP stages.
+template <int BM_, int BN_, int WR_, int WC_, int WPE_, int NBUF_, int GRP_ = 1>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, WR = WR_, WC = WC_, WPE = WPE_, NBUF = NBUF_;
+  static constexpr int GRP = GRP_;
   static constexpr int NW = WR * WC, NTHR = 64 * NW;
   static constexpr int WM = BM / (16 * WR), WN = BN / (16 * WC);
   static constexpr int STAGE = (BM + BN) * BK;  // doubles of one stage, X panel then Y
-  static constexpr int SMEM = NBUF * STAGE;
+  static constexpr int SMEM = NBUF * GRP * STAGE;
+  static_assert(NBUF * GRP >= 2 && NBUF <= 4, "waits below");
 };
 typedef Tile<128, 128, 2, 4, 4, 2> T128;
 typedef Tile<64, 64, 2, 2, 4, 2> T64;
-typedef Tile<64, 64, 4, 2, 4, 4> T64W;
-typedef Tile<32, 32, 2, 2, 4, 4> T32;
+typedef Tile<64, 64, 4, 2, 4, 2, 2> T64W;
+typedef Tile<32, 32, 2, 2, 4, 2, 4> T32;
 
 __device__ __forceinline__ bool aligned16(const void *p) {
   return ((uintptr_t)p & 15) == 0;
@@ -302,25 +307,41 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
   if (!YSAME) ly.init(Y, ldy, n0, nlim, ka, w, lane);
   const bool dx = lx.dmaok, dy = YSAME || ly.dmaok;
   if (dx && dy) {
-    constexpr int PER = PX::CH + (YSAME ? 0 : PY::CH);  // loads of a stage per wave
-    auto issue = [&](int s) {
-      double *buf = smem + (s % NBUF) * C::STAGE;
-      lx.dma(buf, w);
-      if (!YSAME) ly.dma(buf + YOFF, w);
+    constexpr int G = C::GRP;
+    constexpr int PER = G * (PX::CH + (YSAME ? 0 : PY::CH));  // loads of a slot per wave
+    const int ngrp = nfull / G, rem = nfull % G;  // whole slots, then one of rem stages
+    auto issue = [&](int s, int m) {
+      double *buf = smem + (s % NBUF) * (G * C::STAGE);
+#pragma unroll
+      for (int j = 0; j < G; j++)
+        if (j < m) {
+          lx.dma(buf + j * C::STAGE, w);
+          if (!YSAME) ly.dma(buf + j * C::STAGE + YOFF, w);
+        }
+    };
+    auto next = [&](int s) {
+      if (s < ngrp) issue(s, G);
+      else if (G > 1 && s == ngrp && rem > 0) issue(s, rem);
     };
 #pragma unroll
-    for (int s = 0; s < NBUF - 1; s++)
-      if (s < nfull) issue(s);
-    for (int s = 0; s < nfull; s++) {
-      // stages s + 1 .. min(nfull - 1, s + NBUF - 2) may stay in flight
-      const int ahead = min(nfull - 1, s + NBUF - 2) - s;
+    for (int s = 0; s < NBUF - 1; s++) next(s);
+    for (int s = 0; s < ngrp; s++) {
+      // slots s + 1 .. min(ngrp - 1, s + NBUF - 2) may stay in flight
+      const int ahead = min(ngrp - 1, s + NBUF - 2) - s;
       if (NBUF >= 4 && ahead >= 2) wait_vm<2 * PER>();
       else if (NBUF >= 3 && ahead >= 1) wait_vm<PER>();
       else wait_vm<0>();
       ring_barrier();
-      if (s + NBUF - 1 < nfull) issue(s + NBUF - 1);
-      const double *cur = smem + (s % NBUF) * C::STAGE;
-      mma(cur, cur + YOFF);
+      next(s + NBUF - 1);
+      const double *cur = smem + (s % NBUF) * (G * C::STAGE);
+#pragma unroll
+      for (int j = 0; j < G; j++) mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF);
+    }
+    if (G > 1 && rem > 0) {
+      wait_vm<0>();
+      ring_barrier();
+      const double *cur = smem + (ngrp % NBUF) * (G * C::STAGE);
+      for (int j = 0; j < rem; j++) mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF);
     }
   } else {
     // one operand at least goes through registers: loaded while the stage

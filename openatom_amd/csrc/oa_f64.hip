@@ -837,7 +837,18 @@ __device__ __forceinline__ bool ns_update(const oa_ns_args &a, int it, int npart
     r.pad = 0;
     r.error = err;
     *a.rep = r;
-    if (a.mirror) *a.mirror = r;
+    if (a.mirror) {
+      // host memory; `pad` is the word the host polls, stored when the rest
+      // has arrived
+      __hip_atomic_store(&a.mirror->error, err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&a.mirror->status, r.status, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&a.mirror->done, r.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&a.mirror->iterations, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      wait_vm<0>();
+      __hip_atomic_store(&a.mirror->pad, 2 * it + r.done, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
   return done;
 }

@@ -52,12 +52,16 @@ int oa_ws_require(oa_context *c, size_t bytes);
 // (once per device; the device is current).
 int oa_noalloc_init(int device);
 
-// Synchronous S->T on the handle's stream with the buffers at ws
-// (oa_ns_ws_bytes(n)) and the device report rep; the kernels write every report
-// to the handle's pinned mirror too, which the host reads after three
-// iterations and then after every two.
+// S->T on the handle's stream with the buffers at ws (oa_ns_ws_bytes(n)) and
+// the device report rep; returns when the loop's outcome is known (iterations
+// that do nothing may still be enqueued, and T is complete for later work on
+// the stream).  The kernels write every report to the handle's pinned mirror
+// too, where the host waits for it.
 int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
                    double *T, int *iters, double *err, void *ws, oa_ns_report *rep);
+
+// Waits for the report of iteration `upto` (or the last one) in the mirror.
+int oa_ns_wait(oa_context *c, int upto);
 
 // Makes the handle's device current for the scope of an API call and
 // restores the caller's device afterwards.

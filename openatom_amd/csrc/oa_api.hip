@@ -467,9 +467,10 @@ int oa_ns_wait(oa_context *c, int upto) {
 }
 
 int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
-                   double *T, int *iters, double *err, void *ws, oa_ns_report *rep) {
+                   double *T, int *iters, double *err, void *ws, oa_ns_report *rep, bool z,
+                   int modulus) {
   oa_ns_args a;
-  oa_ns_fill(n, S, nspin, tol, maxit, T, rep, c->host_report, ws, &a);
+  oa_ns_fill(n, S, nspin, tol, maxit, T, rep, c->host_report, ws, &a, z, modulus);
   *c->host_report = oa_ns_report{};
   int st = oa_ns_begin(c->stream, a);
   if (st == OA_SUCCESS && maxit > 1) st = oa_ns_check(c->stream, a, 1);

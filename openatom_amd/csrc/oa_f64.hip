@@ -101,6 +101,13 @@ __device__ __forceinline__ bool aligned16(const void *p) {
   return ((uintptr_t)p & 15) == 0;
 }
 
+// c + (NEGB ? -1 : 1) a b.  The FP64 MFMAs take their operands' sign bits in the
+// field that selects a lane group elsewhere (bit 1: B).
+template <bool NEGB>
+__device__ __forceinline__ d4 mfma(double a, double b, d4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, NEGB ? 2 : 0);
+}
+
 // Position of block i (16 rows) of a wave inside its panel, and the panel row
 // of the block's operand lane idx.  PAIR: blocks 2b, 2b + 1 interleave the
 // rows of one 32-row span.
@@ -192,9 +199,22 @@ struct Panel {
   }
 };
 
+// The products a tile sums: op(X) op(Y) alone, with +-op(X1) op(Y1) before it
+// (one part of a complex product), or with +-op(X1) (J Y1) before it (a real
+// matrix times interleaved complex rows).
+enum Seg { SEG_ONE = 0, SEG_TWO = 1, SEG_J = 2 };
+
+__device__ __forceinline__ double flip_sign(double x, unsigned bit) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+  return __builtin_bit_cast(double, u ^ ((unsigned long long)bit << 32));
+}
+
 // One operand's fragments of k step kk of a stage: get(e, i) is this lane's
 // value of block i (of the first NI) for MFMA e.
-template <int R, bool KC, int W, int NWAVE, int NI>
+// J (KC): the operand's k are interleaved (re, im) pairs and J y = i y = (-im,
+// re) of it is multiplied: a fragment read holds a pair, so J is a swap of
+// registers and the MFMA's negation of its B operand where neg(e).
+template <int R, bool KC, int W, int NWAVE, int NI, bool J = false>
 struct Frags {
   static constexpr bool PAIR = RowMap<W, NWAVE, KC>::PAIR;
   static constexpr int NF = PAIR ? (NI + 1) / 2 : NI;
@@ -224,41 +244,66 @@ struct Frags {
     }
   }
   __device__ __forceinline__ double get(int e, int i) const {
-    if constexpr (KC) return f[i][e];
+    if constexpr (KC) return f[i][J ? e ^ 1 : e];
     else if constexpr (PAIR) return f[e * NF + i / 2][i & 1];
     else return f[e * NF + i][0];
   }
+  __device__ __forceinline__ static constexpr bool neg(int e) { return J && e == 0; }
+  // Turns the fragments of Y1 (`first`) into those of +-Y1 or +-J Y1, J along the
+  // rows: a few vector instructions beside MFMAs of 64 cycles.  (A loop of its
+  // own per product made the compiler keep two sets of accumulators.)
+  template <Seg SEG>
+  __device__ __forceinline__ void sign(bool first, bool minus, int lane) {
+    static_assert(!KC || SEG != SEG_J, "J along the rows");
+    const unsigned m = first && minus ? 0x80000000u : 0u;
+    const unsigned jm = m ^ (first ? 0x80000000u : 0u);
+#pragma unroll
+    for (int i = 0; i < (KC ? NI : 2 * NF); i++) {
+      const d2v x = f[i];
+      if constexpr (SEG == SEG_TWO || KC) {
+        f[i] = d2v{flip_sign(x[0], m), flip_sign(x[1], m)};
+      } else if constexpr (PAIR) {
+        f[i] = d2v{flip_sign(first ? x[1] : x[0], jm), flip_sign(first ? x[0] : x[1], m)};
+      } else {
+        const double y = __shfl_xor(x[0], 1);  // the pair's other half
+        f[i][0] = first ? flip_sign(y, lane & 1 ? m : jm) : x[0];
+      }
+    }
+  }
+  static_assert(KC || !J, "J along k only");
 };
 
 // The MFMAs of one stage over the first NI row blocks of the wave.  (A count
 // tested per MFMA made the compiler copy the accumulators at every branch, so
 // the count is a template argument and the choice lies outside the k loop.)
-template <class C, bool XKC, bool YKC, int NI>
+template <class C, bool XKC, bool YKC, int NI, bool YJ = false, Seg SEG = SEG_ONE>
 __device__ __forceinline__ void mma_rows(const double *Xs, const double *Ys, int wr, int wc,
-                                         int lane, d4 (&acc)[C::WM * C::WN]) {
+                                         int lane, d4 (&acc)[C::WM * C::WN], bool first = false,
+                                         bool minus = false) {
   constexpr int WN = C::WN;
   if constexpr (NI > 0) {
 #pragma unroll
     for (int kk = 0; kk < BK / 8; kk++) {
       Frags<C::BM, XKC, C::WM, C::WR, NI> a;
-      Frags<C::BN, YKC, WN, C::WC, WN> b;
+      Frags<C::BN, YKC, WN, C::WC, WN, YJ> b;
       a.load(Xs, wr, kk, lane);
       b.load(Ys, wc, kk, lane);
+      if constexpr (SEG != SEG_ONE) b.template sign<SEG>(first, minus, lane);
 #pragma unroll
       for (int e = 0; e < 2; e++)
 #pragma unroll
         for (int i = 0; i < NI; i++)
 #pragma unroll
           for (int j = 0; j < WN; j++)
-            acc[i * WN + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.get(e, i), b.get(e, j),
-                                                                   acc[i * WN + j], 0, 0, 0);
+            acc[i * WN + j] = b.neg(e) ? mfma<true>(a.get(e, i), b.get(e, j), acc[i * WN + j])
+                                          : mfma<false>(a.get(e, i), b.get(e, j), acc[i * WN + j]);
     }
   }
 }
 
 // The MFMAs of one stage over NB single blocks (KC operands): block t has its
 // operand rows at panel rows xr[t] and yr[t].
-template <int NB, int CAP>
+template <int NB, bool YJ, int CAP>
 __device__ __forceinline__ void mma_list(const double *Xs, const double *Ys,
                                          const int (&xr)[NB], const int (&yr)[NB], int lane,
                                          d4 (&acc)[CAP]) {
@@ -271,9 +316,8 @@ __device__ __forceinline__ void mma_list(const double *Xs, const double *Ys,
     for (int t = 0; t < NB; t++) {
       const d2v a = *reinterpret_cast<const d2v *>(Xs + xr[t] * BK + off);
       const d2v b = *reinterpret_cast<const d2v *>(Ys + yr[t] * BK + off);
-#pragma unroll
-      for (int e = 0; e < 2; e++)
-        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], b[e], acc[t], 0, 0, 0);
+      acc[t] = mfma<YJ>(a[0], b[YJ ? 1 : 0], acc[t]);
+      acc[t] = mfma<false>(a[1], b[YJ ? 0 : 1], acc[t]);
     }
   }
 }
@@ -289,45 +333,56 @@ __device__ __forceinline__ void count_switch(int v, F &&f) {
   }
 }
 
-// Runs mma(X panel, Y panel) over the stages of k in [ka, kb) of one tile.
-// YSAME: the Y panel is the X panel (diagonal tile of a symmetric product),
-// loaded once.
-template <class C, bool XKC, bool YKC, bool YSAME, class Mma>
+// Runs mma(X panel, Y panel, first) over the stages of k in [ka, kb) of one
+// tile; with SEG over those of (X1, Y1) first.  YSAME: the Y panel is the X
+// panel (diagonal tile of a symmetric product), loaded once.
+template <class C, bool XKC, bool YKC, bool YSAME, Seg SEG = SEG_ONE, class Mma>
 __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mlim,
                                       const double *Y, long ldy, int n0, int nlim, int ka,
-                                      int kb, double *smem, Mma &&mma) {
-  constexpr int NBUF = C::NBUF, YOFF = YSAME ? 0 : C::BM * BK;
+                                      int kb, double *smem, Mma &&mma,
+                                      const double *X1 = nullptr, const double *Y1 = nullptr) {
+  constexpr int NBUF = C::NBUF, G = C::GRP, YOFF = YSAME ? 0 : C::BM * BK;
+  constexpr bool TWO = SEG != SEG_ONE;
   typedef Panel<C::BM, XKC, C::NW> PX;
   typedef Panel<C::BN, YKC, C::NW> PY;
   const int nfull = (kb - ka) / BK;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   PX lx;
   PY ly;
-  lx.init(X, ldx, m0, mlim, ka, w, lane);
-  if (!YSAME) ly.init(Y, ldy, n0, nlim, ka, w, lane);
-  const bool dx = lx.dmaok, dy = YSAME || ly.dmaok;
+  auto start = [&](bool first, int k0) {
+    lx.init(TWO && first ? X1 : X, ldx, m0, mlim, k0, w, lane);
+    if (!YSAME) ly.init(TWO && first ? Y1 : Y, ldy, n0, nlim, k0, w, lane);
+  };
+  start(TWO, ka);
+  const bool dx = lx.dmaok && !(TWO && !aligned16(X));
+  const bool dy = YSAME || (ly.dmaok && !(TWO && !aligned16(Y)));
+  auto dma = [&](double *buf) {
+    lx.dma(buf, w);
+    if (!YSAME) ly.dma(buf + YOFF, w);
+  };
   if (dx && dy) {
-    constexpr int G = C::GRP;
     constexpr int PER = G * (PX::CH + (YSAME ? 0 : PY::CH));  // loads of a slot per wave
-    const int ngrp = nfull / G, rem = nfull % G;  // whole slots, then one of rem stages
+    const int ngrp = nfull / G, rem = nfull % G;  // whole slots, then rem stages
+    const int total = TWO ? 2 * ngrp : ngrp;
     auto issue = [&](int s, int m) {
       double *buf = smem + (s % NBUF) * (G * C::STAGE);
 #pragma unroll
       for (int j = 0; j < G; j++)
-        if (j < m) {
-          lx.dma(buf + j * C::STAGE, w);
-          if (!YSAME) ly.dma(buf + j * C::STAGE + YOFF, w);
-        }
+        if (j < m) dma(buf + j * C::STAGE);
     };
     auto next = [&](int s) {
-      if (s < ngrp) issue(s, G);
-      else if (G > 1 && s == ngrp && rem > 0) issue(s, rem);
+      if (s < total) {
+        if (TWO && s == ngrp) start(false, ka);
+        issue(s, G);
+      } else if (!TWO && G > 1 && s == ngrp && rem > 0) {
+        issue(s, rem);
+      }
     };
 #pragma unroll
     for (int s = 0; s < NBUF - 1; s++) next(s);
-    for (int s = 0; s < ngrp; s++) {
-      // slots s + 1 .. min(ngrp - 1, s + NBUF - 2) may stay in flight
-      const int ahead = min(ngrp - 1, s + NBUF - 2) - s;
+    for (int s = 0; s < total; s++) {
+      // slots s + 1 .. min(total - 1, s + NBUF - 2) may stay in flight
+      const int ahead = min(total - 1, s + NBUF - 2) - s;
       if (NBUF >= 4 && ahead >= 2) wait_vm<2 * PER>();
       else if (NBUF >= 3 && ahead >= 1) wait_vm<PER>();
       else wait_vm<0>();
@@ -335,21 +390,33 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
       next(s + NBUF - 1);
       const double *cur = smem + (s % NBUF) * (G * C::STAGE);
 #pragma unroll
-      for (int j = 0; j < G; j++) mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF);
+      for (int j = 0; j < G; j++)
+        mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF, TWO && s < ngrp);
     }
     if (G > 1 && rem > 0) {
-      wait_vm<0>();
-      ring_barrier();
-      const double *cur = smem + (ngrp % NBUF) * (G * C::STAGE);
-      for (int j = 0; j < rem; j++) mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF);
+#pragma nounroll
+      for (int seg = TWO ? 0 : 1; seg < 2; seg++) {
+        if (TWO) {
+          ring_barrier();
+          start(seg == 0, ka + ngrp * G * BK);
+          issue(ngrp, rem);
+        }
+        wait_vm<0>();
+        ring_barrier();
+        const double *cur = smem + (ngrp % NBUF) * (G * C::STAGE);
+        for (int j = 0; j < rem; j++)
+          mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF, seg == 0);
+      }
     }
   } else {
     // one operand at least goes through registers: loaded while the stage
     // before it is multiplied, stored after it
     const bool px = !dx && lx.pairok, py = !dy && ly.pairok;
+    const int total = TWO ? 2 * nfull : nfull;
     d2v vx[PX::CH], vy[PY::CH];
     auto load = [&](int s) {
       double *buf = smem + (s & 1) * C::STAGE;
+      if (TWO && s == nfull) start(false, ka);
       if (dx) lx.dma(buf, w);
       else if (px) lx.pair(vx);
       if (!YSAME) {
@@ -359,37 +426,41 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
     };
     auto finish = [&](int s) {
       double *buf = smem + (s & 1) * C::STAGE;
-      const int k0 = ka + s * BK;
+      const bool first = TWO && s < nfull;
+      const int k0 = ka + (TWO && !first ? s - nfull : s) * BK;
       if (!dx) {
         if (px) PX::put(vx, buf, w, lane);
-        else PX::masked(X, ldx, m0, mlim, k0, kb, buf, w, lane);
+        else PX::masked(first ? X1 : X, ldx, m0, mlim, k0, kb, buf, w, lane);
       }
       if (!YSAME && !dy) {
         if (py) PY::put(vy, buf + YOFF, w, lane);
-        else PY::masked(Y, ldy, n0, nlim, k0, kb, buf + YOFF, w, lane);
+        else PY::masked(first ? Y1 : Y, ldy, n0, nlim, k0, kb, buf + YOFF, w, lane);
       }
     };
-    if (nfull > 0) {
+    if (total > 0) {
       load(0);
       finish(0);
     }
-    for (int s = 0; s < nfull; s++) {
+    for (int s = 0; s < total; s++) {
       wait_vm<0>();
       ring_barrier();
-      if (s + 1 < nfull) load(s + 1);
+      if (s + 1 < total) load(s + 1);
       const double *cur = smem + (s & 1) * C::STAGE;
-      mma(cur, cur + YOFF);
-      if (s + 1 < nfull) finish(s + 1);
+      mma(cur, cur + YOFF, TWO && s < nfull);
+      if (s + 1 < total) finish(s + 1);
     }
   }
   // the rest of a contraction that is no multiple of BK
   const int k0 = ka + nfull * BK;
   if (k0 < kb) {
-    ring_barrier();
-    PX::masked(X, ldx, m0, mlim, k0, kb, smem, w, lane);
-    if (!YSAME) PY::masked(Y, ldy, n0, nlim, k0, kb, smem + YOFF, w, lane);
-    ring_barrier();
-    mma(smem, smem + YOFF);
+#pragma nounroll
+    for (int seg = TWO ? 0 : 1; seg < 2; seg++) {
+      ring_barrier();
+      PX::masked(TWO && !seg ? X1 : X, ldx, m0, mlim, k0, kb, smem, w, lane);
+      if (!YSAME) PY::masked(TWO && !seg ? Y1 : Y, ldy, n0, nlim, k0, kb, smem + YOFF, w, lane);
+      ring_barrier();
+      mma(smem, smem + YOFF, TWO && !seg);
+    }
   }
   ring_barrier();  // the ring may be refilled (a workgroup's next item)
 }
@@ -407,6 +478,9 @@ struct ProbRegs {
   double alpha, beta, diag_add;
   int cw;
   double alpha_w;
+  // second product of the same shape and layouts (SEG): (neg1 ? -1 : 1) X1 Y1
+  const double *X1, *Y1;
+  bool neg1;
 };
 
 __device__ __forceinline__ ProbRegs pick_problem(const oa_gemm_problem &p0,
@@ -427,6 +501,8 @@ __device__ __forceinline__ ProbRegs pick_problem(const oa_gemm_problem &p0,
   r.diag_add = y ? p1.diag_add : p0.diag_add;
   r.cw = y ? p1.cw : p0.cw;
   r.alpha_w = y ? p1.alpha_w : p0.alpha_w;
+  r.X1 = r.Y1 = nullptr;
+  r.neg1 = false;
   return r;
 }
 
@@ -434,9 +510,9 @@ struct NoEpi {
   __device__ __forceinline__ void operator()(int, int, double) const {}
 };
 
-// One BM x BN output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I;
-// epi(m, n, value) sees every output stored.
-template <bool TX, bool TY, class C, class Epi>
+// One BM x BN output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I (the
+// product by SEG); epi(m, n, value) sees every output stored.
+template <bool TX, bool TY, class C, Seg SEG, class Epi>
 __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double *smem,
                                           Epi &&epi) {
   constexpr int WM = C::WM, WN = C::WN;
@@ -456,11 +532,13 @@ __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double
 #pragma unroll
   for (int i = 0; i < WM * WN; i++) acc[i] = d4{0, 0, 0, 0};
   count_switch<0, WM>(ni, [&](auto c) {
-    kloop<C, !TX, TY, false>(P.X, P.ldx, m0, P.M, P.Y, P.ldy, n0, P.N, 0, P.K, smem,
-                             [&](const double *Xs, const double *Ys) {
-                               mma_rows<C, !TX, TY, decltype(c)::value>(Xs, Ys, wr, wc, lane,
-                                                                        acc);
-                             });
+    constexpr int NI = decltype(c)::value;
+    kloop<C, !TX, TY, false, SEG>(P.X, P.ldx, m0, P.M, P.Y, P.ldy, n0, P.N, 0, P.K, smem,
+                                  [&](const double *Xs, const double *Ys, bool first) {
+                                    mma_rows<C, !TX, TY, NI, false, SEG>(
+                                        Xs, Ys, wr, wc, lane, acc, first, P.neg1);
+                                  },
+                                  P.X1, P.Y1);
   });
 
   const int r = lane & 15, g = lane >> 4;
@@ -515,7 +593,20 @@ void gemm_f64_kernel(oa_gemm_problem p0, oa_gemm_problem p1, const int32_t *skip
   if (skip && *skip) return;
   const ProbRegs P = pick_problem(p0, p1);
   __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
-  gemm_body<TX, TY, C>(P, xcd_logical(blockIdx.x, gridDim.x), smem, NoEpi{});
+  gemm_body<TX, TY, C, SEG_ONE>(P, xcd_logical(blockIdx.x, gridDim.x), smem, NoEpi{});
+}
+
+// out = alpha (op(Mr) psi +- op(Mi) J psi) + beta out: the complex back-multiply
+// in one pass over out, J psi never formed.
+template <bool TX, class C>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
+void zback_f64_kernel(oa_gemm_problem p, const double *Mi, int neg) {
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
+  ProbRegs P = pick_problem(p, p);
+  P.X1 = Mi;
+  P.Y1 = p.Y;
+  P.neg1 = neg != 0;
+  gemm_body<TX, false, C, SEG_J>(P, xcd_logical(blockIdx.x, gridDim.x), smem, NoEpi{});
 }
 
 // ------------------------------------------------------------------ grouped
@@ -579,10 +670,10 @@ __device__ __forceinline__ void sym_tile(int tile, int T, int &bi, int &bj) {
   }
 }
 
-// XY (with SYM): the upper-tile map of the symmetric product over two
-// distinct operands X and Y (the complex overlap's Im S = psi (J psi)^T,
-// whose strict upper triangle is all a Hermitian S needs).
-template <class C, bool SYM, bool XY = false>
+// YJ: the product is X (J Y)^T.  With SYM that is the complex overlap's Im S =
+// psi (J psi)^T on the upper tiles, whose strict upper triangle is all a
+// Hermitian S needs.
+template <class C, bool SYM, bool YJ>
 __global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 void ovl_f64_kernel(OvlArgs a) {
   constexpr int BM = C::BM, WM = C::WM, WN = C::WN;
@@ -622,8 +713,6 @@ void ovl_f64_kernel(OvlArgs a) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = w / C::WC, wc = w % C::WC;
   const int r = lane & 15, g = lane >> 4;
-  const double *Yp = (SYM && !XY) ? a.X : a.Y;
-  const long ldy = (SYM && !XY) ? a.ldx : a.ldy;
   double *pt = a.part + ((long)z * ntiles + tile) * (BM * BM);
   // blocks inside the matrix; a symmetric diagonal tile needs those on or
   // above its diagonal
@@ -634,9 +723,9 @@ void ovl_f64_kernel(OvlArgs a) {
 #pragma unroll
   for (int i = 0; i < WM * WN; i++) acc[i] = d4{0, 0, 0, 0};
   if (nblk == (BM / 16) * (BM / 16)) {
-    kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, Yp, ldy, n0, a.N, ka, kb, smem,
-                                [&](const double *Xs, const double *Ys) {
-                                  mma_rows<C, true, true, WM>(Xs, Ys, wr, wc, lane, acc);
+    kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, a.Y, a.ldy, n0, a.N, ka, kb, smem,
+                                [&](const double *Xs, const double *Ys, bool) {
+                                  mma_rows<C, true, true, WM, YJ>(Xs, Ys, wr, wc, lane, acc);
                                 });
 #pragma unroll
     for (int i = 0; i < WM; i++)
@@ -662,13 +751,13 @@ void ovl_f64_kernel(OvlArgs a) {
       xr[t] = rb * 16;
       yr[t] = cb * 16;
     }
-    auto mma = [&](const double *Xs, const double *Ys) {
-      mma_list<NB>(Xs, Ys, xr, yr, lane, acc);
+    auto mma = [&](const double *Xs, const double *Ys, bool) {
+      mma_list<NB, YJ>(Xs, Ys, xr, yr, lane, acc);
     };
-    if (diag && !XY)
+    if (diag)
       kloop<C, true, true, true>(a.X, a.ldx, m0, a.M, a.X, a.ldx, n0, a.N, ka, kb, smem, mma);
     else
-      kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, Yp, ldy, n0, a.N, ka, kb, smem, mma);
+      kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, a.Y, a.ldy, n0, a.N, ka, kb, smem, mma);
 #pragma unroll
     for (int t = 0; t < NB; t++)
       if (w + C::NW * t < nblk)
@@ -787,29 +876,49 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
 
 // Workgroup w of nwg of the first, elementwise iteration.  A non-finite S makes the
 // residual NaN (the products of the identity with it would spread NaN), which
-// ends the loop; see NS_B1.
+// ends the loop; see NS_B1.  Z: S and T hold complex pairs, the buffers a real
+// and an imaginary plane (a.zs apart); the residual has two sums.
+template <bool Z>
 __device__ __forceinline__ void ns_init_body(const oa_ns_args &a, int w, int nwg, double *red) {
   const unsigned n = a.n, np = a.np, nn = np * np;
-  double s = 0.0;
+  const double half = (a.nspin == 1) ? 0.5 : 1.0, nan = __longlong_as_double(0x7ff8000000000000ll);
+  double s = 0.0, si = 0.0;
   for (unsigned idx = w * NT + threadIdx.x; idx < nn; idx += nwg * NT) {
     const unsigned i = idx / np, j = idx - i * np;
-    double b = 0.0, c = 0.0, x = 0.0;
+    double b = 0.0, c = 0.0, x = 0.0, bi = 0.0, xi = 0.0;
     if (i < n && j < n) {
       const long k = (long)i * n + j;
-      b = (a.nspin == 1) ? a.S[k] / 2.0 : a.S[k];
+      b = half * a.S[Z ? 2 * k : k];
       c = (i == j ? 3.0 : 0.0) - b;
       x = 0.5 * c;
-      a.T[k] = x;
       const double d = (i == j ? 1.0 : 0.0) - x;
-      s += (isfinite(d) || n == 1) ? d * d : __longlong_as_double(0x7ff8000000000000ll);
+      if (Z) {
+        bi = half * a.S[2 * k + 1];
+        xi = -0.5 * bi;
+        a.T[2 * k] = x;
+        a.T[2 * k + 1] = xi;
+        const bool ok = isfinite(d) && isfinite(xi);
+        s += ok ? d * d : nan;
+        si += ok ? xi * xi : nan;
+      } else {
+        a.T[k] = x;
+        s += (isfinite(d) || n == 1) ? d * d : nan;
+      }
     }
     a.B[0][idx] = b;
     a.C[idx] = c;
     a.A[1][idx] = x;
+    if (Z) {
+      a.B[0][a.zs + idx] = bi;
+      a.C[a.zs + idx] = -bi;
+      a.A[1][a.zs + idx] = xi;
+    }
   }
   s = block_sum(s, red);
+  if (Z) si = block_sum(si, red);
   if (threadIdx.x == 0) {
     a.partial[w] = s;
+    if (Z) a.partial[nwg + w] = si;
     if (w == 0) {
       a.rep->iterations = 0;
       a.rep->done = 0;
@@ -820,13 +929,22 @@ __device__ __forceinline__ void ns_init_body(const oa_ns_args &a, int w, int nwg
   }
 }
 
-// Residual of the iteration `it` (1-based) from its npart partial sums;
-// returns whether the loop ends there.  `writer` stores the report.
+// Residual of the iteration `it` (1-based) from its npart partial sums (Z: of
+// either part); returns whether the loop ends there.  `writer` stores the
+// report.  The complex rule is the reference's Re sum (dA)^2, NaN where that is
+// negative, or sum |dA|^2 (modulus).
+template <bool Z>
 __device__ __forceinline__ bool ns_update(const oa_ns_args &a, int it, int npart, bool writer,
                                           double *red, double &err) {
   double s = 0.0;
   for (int i = threadIdx.x; i < npart; i += blockDim.x) s += a.partial[i];
   s = block_sum(s, red);
+  if (Z) {
+    double si = 0.0;
+    for (int i = threadIdx.x; i < npart; i += blockDim.x) si += a.partial[npart + i];
+    si = block_sum(si, red);
+    s = a.modulus ? s + si : s - si;
+  }
   err = sqrt(s / ((double)a.n * (double)a.n));
   const bool done = !(err > a.tol && it < a.maxit);
   if (writer && threadIdx.x == 0) {
@@ -853,75 +971,98 @@ __device__ __forceinline__ bool ns_update(const oa_ns_args &a, int it, int npart
   return done;
 }
 
-// Output tile `logical` of an NS_B1, NS_C or NS_PAIR launch after `it` iterations
-// (`which` of a pair: 0 = B', 1 = A').
-template <class C>
+// Output tile `logical` of an NS_B1, NS_C or NS_PAIR launch after `it` iterations.
+// `which` of the launch's products: 0 = B', 1 = A' of a pair; with Z the real
+// and the imaginary part of each in turn (four real products in two sums).
+template <class C, bool Z>
 __device__ __forceinline__ void ns_gemm_body(const oa_ns_args &a, int mode, int it, int npart,
                                              int which, int logical, double *smem) {
   const int t = cdiv(a.np, C::BM);
   if (logical >= t * t) return;
   if (mode != NS_B1 && (a.rep->done || it > a.maxit)) return;
+  const int part = Z ? which & 1 : 0;
+  const bool second = (Z ? which >> 1 : which) != 0;
   if (mode == NS_B1 || (mode == NS_C && it >= 2)) {
     double err;
-    const bool done = ns_update(a, it, npart, logical == 0, smem, err);
+    const bool done = ns_update<Z>(a, it, npart, logical == 0 && which == 0, smem, err);
     if (mode == NS_B1 && isnan(err)) {
-      // the identity's product with a non-finite S is NaN everywhere
+      // S's identity product with a non-finite S is NaN everywhere (a complex
+      // residual may also be NaN by its rule: then T stands)
+      bool bad = !Z;
+      if (Z) {
+        double s = 0.0;
+        for (int i = threadIdx.x; i < npart; i += blockDim.x) s += a.partial[i];
+        bad = isnan(block_sum(s, smem));
+      }
       const int m0 = (logical % t) * C::BM, n0 = (logical / t) * C::BN;
-      for (int e = threadIdx.x; e < C::BM * C::BN; e += C::NTHR) {
+      for (int e = threadIdx.x; bad && e < C::BM * C::BN; e += C::NTHR) {
         const int m = m0 + e / C::BN, n = n0 + e % C::BN;
-        if (m < a.n && n < a.n) a.T[(long)m * a.n + n] = err;
+        if (m < a.n && n < a.n) a.T[Z ? 2 * ((long)m * a.n + n) + part : (long)m * a.n + n] = err;
       }
     }
     if (done) return;
   }
   const int cur = it & 1, nxt = cur ^ 1;
+  const double *X, *Y;
+  double *O;
   ProbRegs P;
+  P.alpha = 0.5;
+  P.diag_add = 0.0;
+  if (mode == NS_C) {
+    X = a.A[cur]; Y = a.B[cur]; O = a.C;
+    P.alpha = -1.0;
+    P.diag_add = part ? 0.0 : 3.0;
+  } else if (mode == NS_B1) {
+    X = a.B[0]; Y = a.C; O = a.B[1];
+  } else if (!second) {
+    X = a.B[cur]; Y = a.C; O = a.B[nxt];
+  } else {
+    X = a.C; Y = a.A[cur]; O = a.A[nxt];
+  }
+  const long im = Z ? a.zs : 0;
   P.M = P.N = P.K = a.np;
   P.ldx = P.ldy = P.ldc = a.np;
   P.beta = 0.0;
-  P.diag_add = 0.0;
   P.cw = 0;
   P.alpha_w = 0.0;
-  P.alpha = 0.5;
-  if (mode == NS_C) {
-    P.X = a.A[cur]; P.Y = a.B[cur]; P.C = a.C;
-    P.alpha = -1.0;
-    P.diag_add = 3.0;
-  } else if (mode == NS_B1) {
-    P.X = a.B[0]; P.Y = a.C; P.C = a.B[1];
-  } else if (which == 0) {
-    P.X = a.B[cur]; P.Y = a.C; P.C = a.B[nxt];
-  } else {
-    P.X = a.C; P.Y = a.A[cur]; P.C = a.A[nxt];
-  }
-  const bool res = mode == NS_PAIR && which == 1;
+  P.X = X;
+  P.Y = part ? Y + im : Y;
+  P.C = part ? O + im : O;
+  // re: Xr Yr - Xi Yi, im: Xr Yi + Xi Yr
+  P.X1 = X + im;
+  P.Y1 = part ? Y : Y + im;
+  P.neg1 = part == 0;
+  const bool res = mode == NS_PAIR && second;
+  const double *old = part ? Y + im : Y;
   double s = 0.0;
-  gemm_body<false, false, C>(P, logical, smem, [&](int m, int n, double x) {
+  gemm_body<false, false, C, Z ? SEG_TWO : SEG_ONE>(P, logical, smem, [&](int m, int n, double x) {
     if (res) {
-      const double d = P.Y[(long)m * a.np + n] - x;
+      const double d = old[(long)m * a.np + n] - x;
       s += d * d;
-      if (m < a.n && n < a.n) a.T[(long)m * a.n + n] = x;
+      if (m < a.n && n < a.n)
+        a.T[Z ? 2 * ((long)m * a.n + n) + part : (long)m * a.n + n] = x;
     }
   });
   if (res) {
     s = block_sum(s, smem);
-    if (threadIdx.x == 0) a.partial[logical] = s;
+    if (threadIdx.x == 0) a.partial[part * t * t + logical] = s;
   }
 }
 
+template <bool Z>
 __global__ __launch_bounds__(NT) void ns_init_kernel(oa_ns_args a) {
   __shared__ double red[NT / 64];
-  ns_init_body(a, blockIdx.x, gridDim.x, red);
+  ns_init_body<Z>(a, blockIdx.x, gridDim.x, red);
 }
 
-template <class C>
+template <class C, bool Z>
 __global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 void ns_gemm_kernel(oa_ns_args a, int mode, int it, int npart) {
   __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
-  ns_gemm_body<C>(a, mode, it, npart, blockIdx.y, xcd_logical(blockIdx.x, gridDim.x), smem);
+  ns_gemm_body<C, Z>(a, mode, it, npart, blockIdx.y, xcd_logical(blockIdx.x, gridDim.x), smem);
 }
 
-// The same over many instances (oa_ns_args tables): items are a.nwg INIT
+// The same over many real instances (oa_ns_args tables): items are a.nwg INIT
 // workgroups, or the output tiles of one problem (B1, C) or two (PAIR).
 __global__ __launch_bounds__(NT) void ns_init_grouped(const oa_ns_args *__restrict__ t,
                                                       const int *__restrict__ prefix,
@@ -929,7 +1070,7 @@ __global__ __launch_bounds__(NT) void ns_init_grouped(const oa_ns_args *__restri
   __shared__ double red[NT / 64];
   for_items(prefix[count], [&](int item) {
     const int i = group_find(prefix, count, item);
-    ns_init_body(t[i], item - prefix[i], t[i].nwg, red);
+    ns_init_body<false>(t[i], item - prefix[i], t[i].nwg, red);
   });
 }
 
@@ -942,7 +1083,8 @@ void ns_gemm_grouped(const oa_ns_args *__restrict__ t, const int *__restrict__ p
     const int i = group_find(prefix, count, item);
     const oa_ns_args &a = t[i];
     const int tiles = cdiv(a.np, C::BM) * cdiv(a.np, C::BM), k = item - prefix[i];
-    ns_gemm_body<C>(a, mode, it, mode == NS_B1 ? a.nwg : tiles, k / tiles, k % tiles, smem);
+    ns_gemm_body<C, false>(a, mode, it, mode == NS_B1 ? a.nwg : tiles, k / tiles, k % tiles,
+                           smem);
   });
 }
 
@@ -966,33 +1108,56 @@ int grouped_grid(K kernel, int total, int threads = NT) {
   return g < cap ? g : cap;
 }
 
-template <bool TX, bool TY, class C>
-void launch_gemm_tile(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_t *skip) {
-  int tiles = 0;
-  for (int i = 0; i < nprob; i++)
-    tiles = max(tiles, cdiv(p[i].M, C::BM) * cdiv(p[i].N, C::BN));
-  hipLaunchKernelGGL((gemm_f64_kernel<TX, TY, C>), dim3(cdiv(tiles, 8) * 8, nprob),
-                     dim3(C::NTHR), 0, s, p[0], p[nprob > 1 ? 1 : 0], skip);
+// The largest tile that still gives every CU its two workgroups (T128), then
+// four (T64), then about one (T64W).  A ragged 128 tile costs almost a whole
+// one (its shorter stages wait for their loads), a 64 tile's MFMAs 1.1 times
+// as much: T psi at n = 301 (npw 20011) 161 us with T128, 142 with T64; n =
+// 448 (40000) 555 / 523; n = 192 (30000) 106 / 79; but n = 384 (40000) 386 /
+// 389; n = 777 (50021) 1946 / 2135; n = 96 (60000) 51 / 60.
+enum TilePick { PICK_128, PICK_64, PICK_64W, PICK_32 };
+TilePick pick_tile(long t128, long t64, int nprob) {
+  const bool ragged = 40 * t128 > 11 * t64;  // 128^2 t128 > 1.1 * 64^2 t64
+  if (t128 * nprob >= 512 && !ragged) return PICK_128;
+  if (t64 * nprob >= 1024) return PICK_64;
+  return t64 * nprob >= 192 ? PICK_64W : PICK_32;
+}
+
+// Calls f(tile configuration).
+template <class F>
+void with_tile(TilePick t, F &&f) {
+  switch (t) {
+    case PICK_128: f(T128{}); break;
+    case PICK_64: f(T64{}); break;
+    case PICK_64W: f(T64W{}); break;
+    case PICK_32: f(T32{}); break;
+  }
 }
 
 template <bool TX, bool TY>
 int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_t *skip) {
-  // The largest tile that still gives every CU its two workgroups (T128), then
-  // four (T64), then about one (T64W).  A ragged 128 tile costs almost a whole
-  // one (its shorter stages wait for their loads), a 64 tile's MFMAs 1.1 times
-  // as much: T psi at n = 301 (npw 20011) 161 us with T128, 142 with T64; n =
-  // 448 (40000) 555 / 523; n = 192 (30000) 106 / 79; but n = 384 (40000) 386 /
-  // 389; n = 777 (50021) 1946 / 2135; n = 96 (60000) 51 / 60.
-  long t128 = 0, t64 = 0;
-  for (int i = 0; i < nprob; i++) {
-    t128 = max(t128, (long)cdiv(p[i].M, 128) * cdiv(p[i].N, 128));
-    t64 = max(t64, (long)cdiv(p[i].M, 64) * cdiv(p[i].N, 64));
-  }
-  const bool ragged = 40 * t128 > 11 * t64;  // 128^2 t128 > 1.1 * 64^2 t64
-  if (t128 * nprob >= 512 && !ragged) launch_gemm_tile<TX, TY, T128>(s, p, nprob, skip);
-  else if (t64 * nprob >= 1024) launch_gemm_tile<TX, TY, T64>(s, p, nprob, skip);
-  else if (t64 * nprob >= 192) launch_gemm_tile<TX, TY, T64W>(s, p, nprob, skip);
-  else launch_gemm_tile<TX, TY, T32>(s, p, nprob, skip);
+  auto tiles = [&](int bm, int bn) {
+    long t = 0;
+    for (int i = 0; i < nprob; i++) t = max(t, (long)cdiv(p[i].M, bm) * cdiv(p[i].N, bn));
+    return t;
+  };
+  with_tile(pick_tile(tiles(128, 128), tiles(64, 64), nprob), [&](auto c) {
+    typedef decltype(c) C;
+    hipLaunchKernelGGL((gemm_f64_kernel<TX, TY, C>),
+                       dim3((unsigned)((tiles(C::BM, C::BN) + 7) / 8 * 8), nprob),
+                       dim3(C::NTHR), 0, s, p[0], p[nprob > 1 ? 1 : 0], skip);
+  });
+  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+}
+
+template <bool TX>
+int launch_zback(hipStream_t s, const oa_gemm_problem &p, const double *Mi, bool neg) {
+  auto tiles = [&](int bm, int bn) { return (long)cdiv(p.M, bm) * cdiv(p.N, bn); };
+  with_tile(pick_tile(tiles(128, 128), tiles(64, 64), 1), [&](auto c) {
+    typedef decltype(c) C;
+    hipLaunchKernelGGL((zback_f64_kernel<TX, C>),
+                       dim3((unsigned)((tiles(C::BM, C::BN) + 7) / 8 * 8)), dim3(C::NTHR), 0, s,
+                       p, Mi, neg ? 1 : 0);
+  });
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
@@ -1116,6 +1281,13 @@ int oa_launch_gemm_f64(hipStream_t s, bool tx, bool ty, const oa_gemm_problem *p
   return launch_gemm<true, true>(s, p, nprob, skip);
 }
 
+int oa_launch_zback_f64(hipStream_t s, bool tx, int n, int K, const double *Mr, const double *Mi,
+                        long ldm, bool neg, const double *psi, long ld, double alpha, double beta,
+                        double *out, long ldo) {
+  const oa_gemm_problem p{n, K, n, Mr, ldm, psi, ld, out, ldo, alpha, beta, 0.0};
+  return tx ? launch_zback<true>(s, p, Mi, neg) : launch_zback<false>(s, p, Mi, neg);
+}
+
 size_t oa_overlap_f64_ws_bytes(int n, int K) {
   const OvlPlan pl = plan_ovl(n, n, K, 0, true);
   // a kx0 slice adds one z
@@ -1127,13 +1299,13 @@ size_t oa_ntsplit_f64_ws_bytes(int M, int N, int K) {
   return (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double) + 256;
 }
 
-template <class T, bool SYM, bool XY>
+template <class T, bool SYM, bool YJ>
 static int launch_ovl_tile(hipStream_t s, const OvlPlan &pl, const OvlArgs &a, int kx0_end,
                            double alpha, double *C, long ldc, double diag,
                            unsigned long long *maxdev) {
   const int nkx = pl.kx0_slice > 0 ? cdiv(pl.ntiles, 8) * 8 : 0;
   const int nb = nkx + cdiv(pl.ntiles * pl.nz_main, 8) * 8;
-  hipLaunchKernelGGL((ovl_f64_kernel<T, SYM, XY>), dim3(nb), dim3(T::NTHR), 0, s, a);
+  hipLaunchKernelGGL((ovl_f64_kernel<T, SYM, YJ>), dim3(nb), dim3(T::NTHR), 0, s, a);
   if (maxdev) hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(64), 0, s, maxdev, 0ull, 1);
   hipLaunchKernelGGL((ovl_reduce_kernel<T::BM, SYM>), dim3(pl.ntiles * (T::BM / 16) * (T::BM / 16)),
                      dim3(1024), 0, s, (const double *)a.part, a.M, a.N, pl.nz,
@@ -1142,8 +1314,9 @@ static int launch_ovl_tile(hipStream_t s, const OvlPlan &pl, const OvlArgs &a, i
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
-// C = alpha X Y^T by the plan, the leading kx0_end columns at half weight.
-template <bool SYM, bool XY>
+// C = alpha X Y^T (YJ: X (J Y)^T) by the plan, the leading kx0_end columns at half
+// weight.
+template <bool SYM, bool YJ>
 static int launch_ovl(hipStream_t s, const OvlPlan &pl, int M, int N, int K, const double *X,
                       long ldx, const double *Y, long ldy, int kx0_end, double alpha, double *C,
                       long ldc, double diag, double *maxdev, void *ws, size_t ws_bytes) {
@@ -1157,8 +1330,8 @@ static int launch_ovl(hipStream_t s, const OvlPlan &pl, int M, int N, int K, con
   a.part = (double *)ws;
   unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
   if (pl.BM == 128)
-    return launch_ovl_tile<T128, SYM, XY>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
-  return launch_ovl_tile<T64, SYM, XY>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
+    return launch_ovl_tile<T128, SYM, YJ>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
+  return launch_ovl_tile<T64, SYM, YJ>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
 }
 
 int oa_launch_overlap_f64(hipStream_t s, int n, int K, const double *psi, long ld, int kx0_end,
@@ -1177,15 +1350,18 @@ int oa_launch_overlap_f64_fit(hipStream_t s, int n, int K, const double *psi, lo
 
 int oa_launch_ntsplit_f64(hipStream_t s, int M, int N, int K, const double *X, long ldx,
                           const double *Y, long ldy, double alpha, double *C, long ldc, void *ws,
-                          size_t ws_bytes) {
-  return launch_ovl<false, false>(s, plan_ovl(M, N, K, 0, false), M, N, K, X, ldx, Y, ldy, 0,
-                                  alpha, C, ldc, 0.0, nullptr, ws, ws_bytes);
+                          size_t ws_bytes, bool yj) {
+  const OvlPlan pl = plan_ovl(M, N, K, 0, false);
+  if (yj)
+    return launch_ovl<false, true>(s, pl, M, N, K, X, ldx, Y, ldy, 0, alpha, C, ldc, 0.0, nullptr,
+                                   ws, ws_bytes);
+  return launch_ovl<false, false>(s, pl, M, N, K, X, ldx, Y, ldy, 0, alpha, C, ldc, 0.0, nullptr,
+                                  ws, ws_bytes);
 }
 
-int oa_launch_overlap_xy_f64(hipStream_t s, int n, int K, const double *X, long ldx,
-                             const double *Y, long ldy, double alpha, double *C, void *ws,
-                             size_t ws_bytes) {
-  return launch_ovl<true, true>(s, plan_ovl(n, n, K, 0, true), n, n, K, X, ldx, Y, ldy, 0, alpha,
+int oa_launch_overlap_j_f64(hipStream_t s, int n, int K, const double *psi, long ld, double alpha,
+                            double *C, void *ws, size_t ws_bytes) {
+  return launch_ovl<true, true>(s, plan_ovl(n, n, K, 0, true), n, n, K, psi, ld, psi, ld, 0, alpha,
                                 C, n, 0.0, nullptr, ws, ws_bytes);
 }
 
@@ -1200,14 +1376,14 @@ static size_t ns_partials(int n) {
   return t * t > 256 ? t * t : 256;
 }
 
-size_t oa_ns_ws_bytes(int n) {
-  return (size_t)(5 * ns_np(n) * ns_np(n)) * sizeof(double) + ns_partials(n) * sizeof(double) +
-         256;
+size_t oa_ns_ws_bytes(int n, bool z) {
+  return (z ? 2 : 1) * ((size_t)(5 * ns_np(n) * ns_np(n)) + ns_partials(n)) * sizeof(double) + 256;
 }
 
 void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double *T,
-                oa_ns_report *rep, oa_ns_report *mirror, void *ws, oa_ns_args *a) {
-  const long nn = ns_np(n) * ns_np(n);
+                oa_ns_report *rep, oa_ns_report *mirror, void *ws, oa_ns_args *a, bool z,
+                int modulus) {
+  const long nn = (z ? 2 : 1) * ns_np(n) * ns_np(n);
   double *base = (double *)ws;
   a->S = S;
   a->n = n;
@@ -1225,19 +1401,11 @@ void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double
   a->T = T;
   a->rep = rep;
   a->mirror = mirror;
+  a->zs = z ? nn / 2 : 0;
+  a->modulus = modulus;
 }
 
-template <class C>
-static void launch_ns_tile(hipStream_t s, const oa_ns_args &a, int mode, int it, int npart) {
-  const int t = cdiv(a.np, C::BM);
-  // a C launch after the last iteration only writes the report
-  const int nb = (mode == NS_C && it >= a.maxit) ? 1 : cdiv(t * t, 8) * 8;
-  hipLaunchKernelGGL(ns_gemm_kernel<C>, dim3(nb, mode == NS_PAIR ? 2 : 1), dim3(C::NTHR), 0, s,
-                     a, mode, it, npart);
-}
-
-// Tile of an S->T launch of nprob products, by the rule of launch_gemm; returns
-// its edge.
+// Edge of the tile of an S->T launch of nprob products.
 static int ns_tile(int np, int nprob) {
   const long t128 = (long)cdiv(np, 128) * cdiv(np, 128) * nprob;
   const long t64 = (long)cdiv(np, 64) * cdiv(np, 64) * nprob;
@@ -1245,18 +1413,27 @@ static int ns_tile(int np, int nprob) {
 }
 
 static int launch_ns(hipStream_t s, const oa_ns_args &a, int mode, int it) {
-  const int pt = cdiv(a.np, ns_tile(a.np, 2));
+  const int z = a.zs ? 2 : 1, nprob = z * (mode == NS_PAIR ? 2 : 1);
+  const int pt = cdiv(a.np, ns_tile(a.np, 2 * z));
   const int npart = mode == NS_B1 ? a.nwg : pt * pt;
-  switch (ns_tile(a.np, mode == NS_PAIR ? 2 : 1)) {
-    case 128: launch_ns_tile<T128>(s, a, mode, it, npart); break;
-    case 64: launch_ns_tile<T64W>(s, a, mode, it, npart); break;
-    default: launch_ns_tile<T32>(s, a, mode, it, npart);
-  }
+  const int edge = ns_tile(a.np, nprob);
+  with_tile(edge == 128 ? PICK_128 : (edge == 64 ? PICK_64W : PICK_32), [&](auto c) {
+    typedef decltype(c) C;
+    const int t = cdiv(a.np, C::BM);
+    // a C launch after the last iteration only writes the report
+    const bool last = mode == NS_C && it >= a.maxit;
+    const dim3 g(last ? 1 : cdiv(t * t, 8) * 8, last ? 1 : nprob);
+    if (a.zs)
+      hipLaunchKernelGGL((ns_gemm_kernel<C, true>), g, dim3(C::NTHR), 0, s, a, mode, it, npart);
+    else
+      hipLaunchKernelGGL((ns_gemm_kernel<C, false>), g, dim3(C::NTHR), 0, s, a, mode, it, npart);
+  });
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
 int oa_ns_begin(hipStream_t s, const oa_ns_args &a) {
-  hipLaunchKernelGGL(ns_init_kernel, dim3(a.nwg), dim3(NT), 0, s, a);
+  if (a.zs) hipLaunchKernelGGL(ns_init_kernel<true>, dim3(a.nwg), dim3(NT), 0, s, a);
+  else hipLaunchKernelGGL(ns_init_kernel<false>, dim3(a.nwg), dim3(NT), 0, s, a);
   return launch_ns(s, a, NS_B1, 1);
 }
 

@@ -58,7 +58,8 @@ int oa_noalloc_init(int device);
 // the stream).  The kernels write every report to the handle's pinned mirror
 // too, where the host waits for it.
 int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
-                   double *T, int *iters, double *err, void *ws, oa_ns_report *rep);
+                   double *T, int *iters, double *err, void *ws, oa_ns_report *rep,
+                   bool z = false, int modulus = 0);
 
 // Waits for the report of iteration `upto` (or the last one) in the mirror.
 int oa_ns_wait(oa_context *c, int upto);
@@ -125,15 +126,21 @@ int oa_launch_overlap_f64_fit(hipStream_t s, int n, int K, const double *psi, lo
 
 // Rectangular split-K product C[M][N] = alpha * X[M][K] * Y[N][K]^T (Lambda).
 size_t oa_ntsplit_f64_ws_bytes(int M, int N, int K);
+// yj: alpha * X (J Y)^T, J (re, im) = (-im, re) on Y's interleaved pairs.
 int oa_launch_ntsplit_f64(hipStream_t s, int M, int N, int K, const double *X,
                           long ldx, const double *Y, long ldy, double alpha,
-                          double *C, long ldc, void *ws, size_t ws_bytes);
-// Upper tiles of C = alpha X Y^T (n x n) for two distinct [n][K] operands,
-// the rest of C the mirror (the strict upper triangle is the product); same
-// workspace as oa_launch_overlap_f64.
-int oa_launch_overlap_xy_f64(hipStream_t s, int n, int K, const double *X, long ldx,
-                             const double *Y, long ldy, double alpha, double *C, void *ws,
-                             size_t ws_bytes);
+                          double *C, long ldc, void *ws, size_t ws_bytes, bool yj = false);
+// Upper tiles of C = alpha psi (J psi)^T (n x n), the rest of C the mirror (the
+// strict upper triangle is the product); same workspace as
+// oa_launch_overlap_f64.
+int oa_launch_overlap_j_f64(hipStream_t s, int n, int K, const double *psi, long ld, double alpha,
+                            double *C, void *ws, size_t ws_bytes);
+// out = alpha (op(Mr) psi + sign op(Mi) J psi) + beta out over K columns of
+// interleaved pairs; Mr and Mi n x n with leading dimension ldm, op the
+// transpose when tx, sign -1 when neg.
+int oa_launch_zback_f64(hipStream_t s, bool tx, int n, int K, const double *Mr, const double *Mi,
+                        long ldm, bool neg, const double *psi, long ld, double alpha, double beta,
+                        double *out, long ldo);
 
 // S->T on the device.  Workspace: oa_ns_ws_bytes(n).  begin runs the first
 // iteration; for it = 1, 2, ... check(it) settles the report of iteration it
@@ -152,10 +159,13 @@ struct oa_ns_args {
   double tol;
   double *T;
   oa_ns_report *rep, *mirror;
+  long zs;      // complex S and T: elements from a buffer's real to its imaginary plane
+  int modulus;  // complex: stop on sum |dA|^2 instead of Re sum (dA)^2
 };
-size_t oa_ns_ws_bytes(int n);
+size_t oa_ns_ws_bytes(int n, bool z = false);
 void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double *T,
-                oa_ns_report *rep, oa_ns_report *mirror, void *ws, oa_ns_args *a);
+                oa_ns_report *rep, oa_ns_report *mirror, void *ws, oa_ns_args *a, bool z = false,
+                int modulus = 0);
 int oa_ns_begin(hipStream_t s, const oa_ns_args &a);
 int oa_ns_check(hipStream_t s, const oa_ns_args &a, int it);
 int oa_ns_iterate(hipStream_t s, const oa_ns_args &a, int it);

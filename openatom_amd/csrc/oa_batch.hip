@@ -13,8 +13,10 @@
 //   S->T init and B' = BC/2 (the first iteration) -> (maxit - 1) x (residual
 //   check with GEMM C = 3I - AB, GEMM pair B' = BC/2, A' = CA/2) -> last
 //   check -> slice T -> back-multiply digit products.
-// FP64: the overlap and the back-multiply are per-instance FP64-MFMA launches
-// inside the same sequence; S->T is grouped as above.
+// FP64: overlap (one launch per tile edge) -> reduce -> S->T as above ->
+// back-multiply (one launch per tile).  Instances whose buffers overlap, so
+// that one could read what another writes, go to launches of their own, in
+// order.
 // Every launch reads device tables built at plan time; the sequence performs
 // no allocation, no memset and no host synchronisation, so it captures into
 // a graph as is.
@@ -50,13 +52,12 @@ struct DevGuard {
   }
 };
 
-enum LaunchKind { LK_FILL = 0, LK_SPLIT, LK_NS, LK_F64_OVL, LK_F64_BACK };
+enum LaunchKind { LK_FILL = 0, LK_SPLIT, LK_NS, LK_F64_OVL, LK_F64_REDUCE, LK_F64_BACK };
 
 struct Launch {
   int kind, phase, variant;
   int it;         // LK_NS: iterations done
   oa_group g;     // device tables (grouped kinds)
-  int inst;       // per-instance kinds
 };
 
 struct InstPlan {
@@ -160,13 +161,17 @@ int validate(int count, const oa_instance *in) {
 }
 
 // Group the instances with variant v (digit tile or WM) into one table.
+// (the table in the given order of instances, or as they come).
 template <class T, class GetArgs, class GetItems, class Sel>
 void add_group(Blob &blob, std::vector<Launch> &seq, int kind, int phase, int variant,
                const std::vector<InstPlan> &ip, GetArgs args, GetItems items, Sel sel,
-               std::vector<std::pair<size_t, size_t>> &fix) {
+               std::vector<std::pair<size_t, size_t>> &fix,
+               const std::vector<int> *order = nullptr) {
   std::vector<T> a;
   std::vector<int> prefix(1, 0);
-  for (size_t i = 0; i < ip.size(); i++) {
+  const size_t cnt = order ? order->size() : ip.size();
+  for (size_t k = 0; k < cnt; k++) {
+    const size_t i = order ? (size_t)(*order)[k] : k;
     if (!sel(ip[i])) continue;
     const int it = items(ip[i], (int)i);
     if (it <= 0) continue;
@@ -189,6 +194,32 @@ void add_group(Blob &blob, std::vector<Launch> &seq, int kind, int phase, int va
   seq.push_back(L);
 }
 
+// Address range of a matrix.
+struct Range {
+  const double *lo, *hi;
+  Range(const double *p, int rows, long ld, int cols) : lo(p), hi(p + (rows - 1) * ld + cols) {}
+  bool meets(const Range &o) const { return lo < o.hi && o.lo < hi; }
+};
+
+// Splits the instances, in order, into runs that may execute at once: no
+// member writes what another one reads or writes.
+template <class Reads, class Writes>
+std::vector<std::vector<int>> runs(int count, Reads reads, Writes writes) {
+  std::vector<std::vector<int>> out;
+  for (int i = 0; i < count; i++) {
+    bool fits = !out.empty();
+    for (size_t k = 0; fits && k < out.back().size(); k++) {
+      const int j = out.back()[k];
+      fits = !writes(i).meets(writes(j));
+      for (const Range &r : reads(j)) fits = fits && !writes(i).meets(r);
+      for (const Range &r : reads(i)) fits = fits && !writes(j).meets(r);
+    }
+    if (!fits) out.emplace_back();
+    out.back().push_back(i);
+  }
+  return out;
+}
+
 int run_seq(oa_batch *b, hipStream_t s) {
   int st = OA_SUCCESS;
   for (const Launch &L : b->seq) {
@@ -196,18 +227,9 @@ int run_seq(oa_batch *b, hipStream_t s) {
       case LK_FILL: st = oa_fill_u64(s, b->counters, b->ncounters); break;
       case LK_SPLIT: st = oa_split_grouped(s, b->prec, L.variant, L.phase, L.g); break;
       case LK_NS: st = oa_ns_grouped(s, L.phase, L.variant, L.it, L.g); break;
-      case LK_F64_OVL: {
-        const InstPlan &p = b->ip[L.inst];
-        st = oa_launch_overlap_f64(s, p.n, p.K, p.psi, p.ld, p.kx0_end, 2.0, p.S, 0.0, nullptr,
-                                   p.ovl_ws, p.ovl_bytes);
-        break;
-      }
-      case LK_F64_BACK: {
-        const InstPlan &p = b->ip[L.inst];
-        oa_gemm_problem g{p.n, p.K, p.n, p.T, p.n, p.psi, p.ld, p.out, p.ldout, 1.0, 0.0, 0.0};
-        st = oa_launch_gemm_f64(s, false, false, &g, 1, nullptr);
-        break;
-      }
+      case LK_F64_OVL: st = oa_ovl_grouped(s, L.variant, L.g); break;
+      case LK_F64_REDUCE: st = oa_ovl_reduce_grouped(s, L.g); break;
+      case LK_F64_BACK: st = oa_gemm_f64_grouped(s, L.variant, L.g); break;
       default: st = OA_ERR_UNSUPPORTED;
     }
     if (st) return st;
@@ -308,6 +330,9 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
   auto dcnt = [&](long k) { return (unsigned long long *)(dbase + off_cnt) + k; };
   oa_ns_report *drep = (oa_ns_report *)(dbase + off_rep);
   auto all = [](const InstPlan &) { return true; };
+  auto psi_range = [&](int i) {
+    return Range(b->ip[i].psi, b->ip[i].n, b->ip[i].ld, b->ip[i].K);
+  };
   if (split) {
     for (int i = 0; i < count; i++) {
       InstPlan &p = b->ip[i];
@@ -346,11 +371,31 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
           [&](const InstPlan &, int i) { return sa[i].items_rd; }, sel, fix);
     }
   } else {
+    std::vector<oa_ovl_args> oa(count);
+    std::vector<int> blocks(count), rblocks(count);
     for (int i = 0; i < count; i++) {
-      Launch L{};
-      L.kind = LK_F64_OVL;
-      L.inst = i;
-      b->seq.push_back(L);
+      const InstPlan &p = b->ip[i];
+      st = oa_ovl_fill(p.n, p.K, p.psi, p.ld, p.kx0_end, 2.0, p.S, p.ovl_ws, p.ovl_bytes, &oa[i],
+                       &blocks[i], &rblocks[i]);
+      if (st) return st;
+    }
+    auto args = [&](const InstPlan &, int i) { return oa[i]; };
+    for (std::vector<int> &run : runs(
+             count, [&](int i) { return std::vector<Range>{psi_range(i)}; },
+             [&](int i) { return Range(b->ip[i].S, b->ip[i].n, b->ip[i].n, b->ip[i].n); })) {
+      std::stable_sort(run.begin(), run.end(),
+                       [&](int i, int j) { return oa[i].kchunk > oa[j].kchunk; });
+      for (int bm : {128, 64}) {
+        std::vector<int> sub;
+        for (int i : run)
+          if (oa[i].bm == bm) sub.push_back(i);
+        add_group<oa_ovl_args>(
+            blob, b->seq, LK_F64_OVL, 0, bm, b->ip, args,
+            [&](const InstPlan &, int i) { return blocks[i]; }, all, fix, &sub);
+      }
+      add_group<oa_ovl_args>(
+          blob, b->seq, LK_F64_REDUCE, 0, 0, b->ip, args,
+          [&](const InstPlan &, int i) { return rblocks[i]; }, all, fix, &run);
     }
   }
   // S->T, grouped for both precisions: one table for INIT, and per GEMM tile
@@ -403,11 +448,32 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
           [&](const InstPlan &, int i) { return sa[i].items_d1; }, sel, fix);
     }
   } else {
-    for (int i = 0; i < count; i++) {
-      Launch L{};
-      L.kind = LK_F64_BACK;
-      L.inst = i;
-      b->seq.push_back(L);
+    for (std::vector<int> &run : runs(
+             count,
+             [&](int i) {
+               const InstPlan &p = b->ip[i];
+               return std::vector<Range>{psi_range(i), Range(p.T, p.n, p.n, p.n)};
+             },
+             [&](int i) { return Range(b->ip[i].out, b->ip[i].n, b->ip[i].ldout, b->ip[i].K); })) {
+      std::stable_sort(run.begin(), run.end(),
+                       [&](int i, int j) { return b->ip[i].n > b->ip[j].n; });
+      std::vector<oa_gemm_problem> gp;
+      for (int i : run) {
+        const InstPlan &p = b->ip[i];
+        gp.push_back({p.n, p.K, p.n, p.T, p.n, p.psi, p.ld, p.out, p.ldout, 1.0, 0.0, 0.0});
+      }
+      std::vector<int> tile(run.size()), blocks(run.size()), at(count);
+      oa_gemm_f64_group(gp.data(), (int)run.size(), tile.data(), blocks.data());
+      for (size_t k = 0; k < run.size(); k++) at[run[k]] = (int)k;
+      for (int v = 0; v < OA_GEMM_TILES; v++) {
+        std::vector<int> sub;
+        for (int i : run)
+          if (tile[at[i]] == v) sub.push_back(i);
+        add_group<oa_gemm_problem>(
+            blob, b->seq, LK_F64_BACK, 0, v, b->ip,
+            [&](const InstPlan &, int i) { return gp[at[i]]; },
+            [&](const InstPlan &, int i) { return blocks[at[i]]; }, all, fix, &sub);
+      }
     }
   }
   // the table region: grow (and rebuild the address-carrying structs) if the

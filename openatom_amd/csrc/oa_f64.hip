@@ -303,10 +303,10 @@ __device__ __forceinline__ void mma_rows(const double *Xs, const double *Ys, int
 
 // The MFMAs of one stage over NB single blocks (KC operands): block t has its
 // operand rows at panel rows xr[t] and yr[t].
-template <int NB, bool YJ, int CAP>
+template <int NB, bool YJ>
 __device__ __forceinline__ void mma_list(const double *Xs, const double *Ys,
                                          const int (&xr)[NB], const int (&yr)[NB], int lane,
-                                         d4 (&acc)[CAP]) {
+                                         d4 (&acc)[NB]) {
   const int r = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int kk = 0; kk < BK / 8; kk++) {
@@ -632,20 +632,6 @@ __device__ __forceinline__ void for_items(int total, F &&f) {
   }
 }
 
-// Split-K partial products over the plane-wave index.
-//   SYM: tiles (bi <= bj) of X X^T; else all tiles of X Y^T.
-//   Chunk 0 covers [0, kx0_end) when kx0_end > 0 (weighted 1/2 later).
-struct OvlArgs {
-  const double *X;
-  long ldx;
-  const double *Y;
-  long ldy;
-  int M, N, K;
-  int kx0_end;
-  int nz_main, kchunk;
-  double *part;  // [nz][ntiles][BM][BM]
-};
-
 __device__ __forceinline__ void upper_tile(int tile, int T, int &bi, int &bj) {
   int b = 0, rem = tile;
   while (rem >= T - b) {
@@ -672,15 +658,14 @@ __device__ __forceinline__ void sym_tile(int tile, int T, int &bi, int &bj) {
 
 // YJ: the product is X (J Y)^T.  With SYM that is the complex overlap's Im S =
 // psi (J psi)^T on the upper tiles, whose strict upper triangle is all a
-// Hermitian S needs.
+// Hermitian S needs.  Workgroup `block` of nblocks.
 template <class C, bool SYM, bool YJ>
-__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
-void ovl_f64_kernel(OvlArgs a) {
+__device__ __forceinline__ void ovl_body(const oa_ovl_args &a, int block, int nblocks,
+                                         double *smem) {
   constexpr int BM = C::BM, WM = C::WM, WN = C::WN;
   static_assert(C::BM == C::BN, "square tiles");
   typedef RowMap<WM, C::WR, true> RM;
   typedef RowMap<WN, C::WC, true> CM;
-  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
   const int Tm = cdiv(a.M, BM), Tn = cdiv(a.N, BM);
   const int ntiles = SYM ? Tm * (Tm + 1) / 2 : Tm * Tn;
   // The short kx = 0 slice (z = 0) takes the leading workgroups, which the
@@ -688,12 +673,12 @@ void ovl_f64_kernel(OvlArgs a) {
   const int hx = a.kx0_end > 0 ? 1 : 0;
   const int nkx = hx ? cdiv(ntiles, 8) * 8 : 0;
   int tile, z;
-  if ((int)blockIdx.x < nkx) {
-    if ((int)blockIdx.x >= ntiles) return;
-    tile = blockIdx.x;
+  if (block < nkx) {
+    if (block >= ntiles) return;
+    tile = block;
     z = 0;
   } else {
-    const int logical = xcd_logical(blockIdx.x - nkx, gridDim.x - nkx);
+    const int logical = xcd_logical(block - nkx, nblocks - nkx);
     if (logical >= ntiles * a.nz_main) return;
     tile = logical % ntiles;
     z = logical / ntiles + hx;
@@ -719,10 +704,10 @@ void ovl_f64_kernel(OvlArgs a) {
   const bool diag = SYM && bi == bj;
   const int nbr = min(BM / 16, cdiv(a.M - m0, 16)), nbc = min(BM / 16, cdiv(a.N - n0, 16));
   const int nblk = diag ? nbr * (nbr + 1) / 2 : nbr * nbc;
-  d4 acc[WM * WN];
-#pragma unroll
-  for (int i = 0; i < WM * WN; i++) acc[i] = d4{0, 0, 0, 0};
   if (nblk == (BM / 16) * (BM / 16)) {
+    d4 acc[WM * WN];
+#pragma unroll
+    for (int i = 0; i < WM * WN; i++) acc[i] = d4{0, 0, 0, 0};
     kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, a.Y, a.ldy, n0, a.N, ka, kb, smem,
                                 [&](const double *Xs, const double *Ys, bool) {
                                   mma_rows<C, true, true, WM, YJ>(Xs, Ys, wr, wc, lane, acc);
@@ -741,9 +726,11 @@ void ovl_f64_kernel(OvlArgs a) {
   // one repeats the last, unstored
   count_switch<1, WM * WN>(cdiv(nblk, C::NW), [&](auto c) {
     constexpr int NB = decltype(c)::value;
+    d4 acc[NB];
     int xr[NB], yr[NB];
 #pragma unroll
     for (int t = 0; t < NB; t++) {
+      acc[t] = d4{0, 0, 0, 0};
       const int idx = min(w + C::NW * t, nblk - 1);
       int rb, cb;
       if (diag) upper_tile(idx, nbr, rb, cb);
@@ -766,6 +753,13 @@ void ovl_f64_kernel(OvlArgs a) {
   });
 }
 
+template <class C, bool SYM, bool YJ>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
+void ovl_f64_kernel(oa_ovl_args a) {
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
+  ovl_body<C, SYM, YJ>(a, blockIdx.x, gridDim.x, smem);
+}
+
 // C = alpha * (sum over z of the partial tiles), in a fixed order: a workgroup
 // owns 16 x 16 outputs, the four waves of z group q add z = q, q + 4, ... and
 // the groups combine in order.  (One thread adding all z of an element, one
@@ -776,26 +770,25 @@ void ovl_f64_kernel(OvlArgs a) {
 //   kx0_sub: every z counts fully and half the product of the leading
 //            kx0_sub columns of psi is taken off here.
 template <int BM, bool SYM>
-__global__ __launch_bounds__(1024) void ovl_reduce_kernel(const double *__restrict__ part, int M,
-                                                         int N, int nz, int has_kx0,
-                                                         int kx0_sub, const double *psi, long ld,
-                                                         double alpha, double *C, long ldc,
-                                                         double diag,
-                                                         unsigned long long *maxdev) {
+__device__ __forceinline__ void ovl_reduce_body(const oa_ovl_args &a, int block,
+                                                double (&sums)[4][256], double (&out)[16][17]) {
   constexpr int PB = BM / 16;  // patches per tile edge
+  const int M = a.M, N = a.N, nz = a.nz;
+  const bool has_kx0 = a.kx0_end > 0;
+  const double *psi = a.X;
+  const long ld = a.ldx, ldc = a.ldc;
+  double *C = a.C;
   const int Tm = cdiv(M, BM), Tn = cdiv(N, BM);
   const int ntiles = SYM ? Tm * (Tm + 1) / 2 : Tm * Tn;
-  const int tile = blockIdx.x / (PB * PB), patch = blockIdx.x % (PB * PB);
+  const int tile = block / (PB * PB), patch = block % (PB * PB);
   int bi, bj;
   if (SYM) sym_tile(tile, Tm, bi, bj);
   else { bi = tile % Tm; bj = tile / Tm; }
   const int pi = (patch / PB) * 16, pj = (patch % PB) * 16;
   if (bi * BM + pi >= M || bj * BM + pj >= N || (SYM && bi == bj && pi > pj)) return;
-  __shared__ double sums[4][256];
-  __shared__ double out[16][17];
   const int t = threadIdx.x & 255, q = threadIdx.x >> 8;
   const int lr = t >> 4, lc = t & 15;
-  const double *p = part + (long)tile * (BM * BM) + (pi + lr) * BM + pj + lc;
+  const double *p = a.part + (long)tile * (BM * BM) + (pi + lr) * BM + pj + lc;
   const long zs = (long)ntiles * (BM * BM);
   double s = 0.0;
 #pragma unroll 8
@@ -812,26 +805,73 @@ __global__ __launch_bounds__(1024) void ovl_reduce_kernel(const double *__restri
     s = ((sums[0][t] + sums[1][t]) + sums[2][t]) + sums[3][t];
     if (in) {
       double g = 0.0;
-      for (int k = 0; k < kx0_sub; k++) g = fma(psi[(long)i * ld + k], psi[(long)j * ld + k], g);
-      s = alpha * fma(-0.5, g, s);
+      for (int k = 0; k < a.kx0_sub; k++) g = fma(psi[(long)i * ld + k], psi[(long)j * ld + k], g);
+      s = a.alpha * fma(-0.5, g, s);
       C[(long)i * ldc + j] = s;
     }
     out[lr][lc] = s;
-    if (maxdev) {
+    if (a.maxdev) {
       // on the bits of non-negative doubles; a NaN's compare above all others
-      const double dv = fabs(s - (i == j ? diag : 0.0));
+      const double dv = fabs(s - (i == j ? a.diag : 0.0));
       unsigned long long u = in ? (unsigned long long)__double_as_longlong(dv) : 0ull;
       for (int o = 32; o > 0; o >>= 1) {
         const unsigned long long w = __shfl_xor(u, o);
         u = w > u ? w : u;
       }
-      if ((t & 63) == 0) atomicMax(maxdev, u);
+      if ((t & 63) == 0) atomicMax(a.maxdev, u);
     }
   }
   if (!SYM) return;
   __syncthreads();
   const int mi = bi * BM + pi + lc, mj = bj * BM + pj + lr;  // C[mj][mi] = out[lc][lr]
   if (q == 0 && mi < M && mj < N && !(dpatch && lr < lc)) C[(long)mj * ldc + mi] = out[lc][lr];
+}
+
+template <int BM, bool SYM>
+__global__ __launch_bounds__(1024) void ovl_reduce_kernel(oa_ovl_args a) {
+  __shared__ double sums[4][256];
+  __shared__ double out[16][17];
+  ovl_reduce_body<BM, SYM>(a, blockIdx.x, sums, out);
+}
+
+// The same over many instances: workgroups prefix[i] .. prefix[i + 1] - 1 are
+// those of instance i's own launch, so the sums are the single launches' bit
+// for bit.  Instances one after another leave the chip partly idle at both ends
+// of every launch: twelve of n = 64 to 512 (npw 8192 to 65536) took 5.45 ms a
+// step, together 4.91.
+// The table is in order of falling work per workgroup, so the short ones fill
+// the end.
+template <class C>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
+void ovl_f64_grouped(const oa_ovl_args *__restrict__ t, const int *__restrict__ prefix,
+                     int count) {
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
+  const int i = group_find(prefix, count, blockIdx.x);
+  const oa_ovl_args a = t[i];
+  ovl_body<C, true, false>(a, blockIdx.x - prefix[i], prefix[i + 1] - prefix[i], smem);
+}
+
+__global__ __launch_bounds__(1024) void ovl_reduce_grouped(const oa_ovl_args *__restrict__ t,
+                                                           const int *__restrict__ prefix,
+                                                           int count) {
+  __shared__ double sums[4][256];
+  __shared__ double out[16][17];
+  const int i = group_find(prefix, count, blockIdx.x);
+  const int block = blockIdx.x - prefix[i];
+  if (t[i].bm == 128) ovl_reduce_body<128, true>(t[i], block, sums, out);
+  else ovl_reduce_body<64, true>(t[i], block, sums, out);
+}
+
+template <class C>
+__global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
+void gemm_f64_grouped(const oa_gemm_problem *__restrict__ t, const int *__restrict__ prefix,
+                      int count) {
+  __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
+  const int i = group_find(prefix, count, blockIdx.x);
+  const oa_gemm_problem &p = t[i];
+  gemm_body<false, false, C, SEG_ONE>(
+      pick_problem(p, p), xcd_logical(blockIdx.x - prefix[i], prefix[i + 1] - prefix[i]), smem,
+      NoEpi{});
 }
 
 __global__ void fill_u64_kernel(unsigned long long *p, unsigned long long v, int n) {
@@ -1115,11 +1155,15 @@ int grouped_grid(K kernel, int total, int threads = NT) {
 // 448 (40000) 555 / 523; n = 192 (30000) 106 / 79; but n = 384 (40000) 386 /
 // 389; n = 777 (50021) 1946 / 2135; n = 96 (60000) 51 / 60.
 enum TilePick { PICK_128, PICK_64, PICK_64W, PICK_32 };
-TilePick pick_tile(long t128, long t64, int nprob) {
+// (t128, t64): tiles of the product; (all128, all64): those of the whole launch.
+TilePick pick_tile(long t128, long t64, long all128, long all64) {
   const bool ragged = 40 * t128 > 11 * t64;  // 128^2 t128 > 1.1 * 64^2 t64
-  if (t128 * nprob >= 512 && !ragged) return PICK_128;
-  if (t64 * nprob >= 1024) return PICK_64;
-  return t64 * nprob >= 192 ? PICK_64W : PICK_32;
+  if (all128 >= 512 && !ragged) return PICK_128;
+  if (all64 >= 1024) return PICK_64;
+  return all64 >= 192 ? PICK_64W : PICK_32;
+}
+long gemm_tiles(const oa_gemm_problem &p, int bm, int bn) {
+  return (long)cdiv(p.M, bm) * cdiv(p.N, bn);
 }
 
 // Calls f(tile configuration).
@@ -1137,10 +1181,11 @@ template <bool TX, bool TY>
 int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_t *skip) {
   auto tiles = [&](int bm, int bn) {
     long t = 0;
-    for (int i = 0; i < nprob; i++) t = max(t, (long)cdiv(p[i].M, bm) * cdiv(p[i].N, bn));
+    for (int i = 0; i < nprob; i++) t = max(t, gemm_tiles(p[i], bm, bn));
     return t;
   };
-  with_tile(pick_tile(tiles(128, 128), tiles(64, 64), nprob), [&](auto c) {
+  const long t128 = tiles(128, 128), t64 = tiles(64, 64);
+  with_tile(pick_tile(t128, t64, t128 * nprob, t64 * nprob), [&](auto c) {
     typedef decltype(c) C;
     hipLaunchKernelGGL((gemm_f64_kernel<TX, TY, C>),
                        dim3((unsigned)((tiles(C::BM, C::BN) + 7) / 8 * 8), nprob),
@@ -1151,12 +1196,12 @@ int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_
 
 template <bool TX>
 int launch_zback(hipStream_t s, const oa_gemm_problem &p, const double *Mi, bool neg) {
-  auto tiles = [&](int bm, int bn) { return (long)cdiv(p.M, bm) * cdiv(p.N, bn); };
-  with_tile(pick_tile(tiles(128, 128), tiles(64, 64), 1), [&](auto c) {
+  const long t128 = gemm_tiles(p, 128, 128), t64 = gemm_tiles(p, 64, 64);
+  with_tile(pick_tile(t128, t64, t128, t64), [&](auto c) {
     typedef decltype(c) C;
     hipLaunchKernelGGL((zback_f64_kernel<TX, C>),
-                       dim3((unsigned)((tiles(C::BM, C::BN) + 7) / 8 * 8)), dim3(C::NTHR), 0, s,
-                       p, Mi, neg ? 1 : 0);
+                       dim3((unsigned)((gemm_tiles(p, C::BM, C::BN) + 7) / 8 * 8)), dim3(C::NTHR), 0,
+                       s, p, Mi, neg ? 1 : 0);
   });
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
@@ -1299,39 +1344,97 @@ size_t oa_ntsplit_f64_ws_bytes(int M, int N, int K) {
   return (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double) + 256;
 }
 
-template <class T, bool SYM, bool YJ>
-static int launch_ovl_tile(hipStream_t s, const OvlPlan &pl, const OvlArgs &a, int kx0_end,
-                           double alpha, double *C, long ldc, double diag,
-                           unsigned long long *maxdev) {
-  const int nkx = pl.kx0_slice > 0 ? cdiv(pl.ntiles, 8) * 8 : 0;
-  const int nb = nkx + cdiv(pl.ntiles * pl.nz_main, 8) * 8;
-  hipLaunchKernelGGL((ovl_f64_kernel<T, SYM, YJ>), dim3(nb), dim3(T::NTHR), 0, s, a);
-  if (maxdev) hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(64), 0, s, maxdev, 0ull, 1);
-  hipLaunchKernelGGL((ovl_reduce_kernel<T::BM, SYM>), dim3(pl.ntiles * (T::BM / 16) * (T::BM / 16)),
-                     dim3(1024), 0, s, (const double *)a.part, a.M, a.N, pl.nz,
-                     pl.kx0_slice > 0 ? 1 : 0, pl.kx0_slice > 0 ? 0 : kx0_end, a.X, a.ldx, alpha,
-                     C, ldc, diag, maxdev);
-  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+// Workgroups of a plan's launches.
+static int ovl_blocks(const OvlPlan &pl) {
+  return (pl.kx0_slice > 0 ? cdiv(pl.ntiles, 8) * 8 : 0) + cdiv(pl.ntiles * pl.nz_main, 8) * 8;
+}
+static int reduce_blocks(const OvlPlan &pl) {
+  return pl.ntiles * (pl.BM / 16) * (pl.BM / 16);
 }
 
-// C = alpha X Y^T (YJ: X (J Y)^T) by the plan, the leading kx0_end columns at half
-// weight.
+// C = alpha X Y^T by the plan, the leading kx0_end columns at half weight.
+static int fill_ovl(const OvlPlan &pl, int M, int N, int K, const double *X, long ldx,
+                    const double *Y, long ldy, int kx0_end, double alpha, double *C, long ldc,
+                    double diag, double *maxdev, void *ws, size_t ws_bytes, oa_ovl_args *a) {
+  if (pl.nz_main < 1 ||
+      (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double) > ws_bytes)
+    return OA_ERR_CAPACITY;
+  *a = oa_ovl_args{X, ldx, Y, ldy, M, N, K, pl.kx0_slice, pl.nz_main, pl.kchunk, (double *)ws,
+                   pl.BM, pl.nz, pl.kx0_slice > 0 ? 0 : kx0_end, alpha, C, ldc, diag,
+                   reinterpret_cast<unsigned long long *>(maxdev)};
+  return OA_SUCCESS;
+}
+
+template <class T, bool SYM, bool YJ>
+static void launch_ovl_tile(hipStream_t s, const OvlPlan &pl, const oa_ovl_args &a) {
+  hipLaunchKernelGGL((ovl_f64_kernel<T, SYM, YJ>), dim3(ovl_blocks(pl)), dim3(T::NTHR), 0, s, a);
+  if (a.maxdev) hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(64), 0, s, a.maxdev, 0ull, 1);
+  hipLaunchKernelGGL((ovl_reduce_kernel<T::BM, SYM>), dim3(reduce_blocks(pl)), dim3(1024), 0, s,
+                     a);
+}
+
+// YJ: X (J Y)^T.
 template <bool SYM, bool YJ>
 static int launch_ovl(hipStream_t s, const OvlPlan &pl, int M, int N, int K, const double *X,
                       long ldx, const double *Y, long ldy, int kx0_end, double alpha, double *C,
                       long ldc, double diag, double *maxdev, void *ws, size_t ws_bytes) {
-  if (pl.nz_main < 1 ||
-      (size_t)pl.nz * pl.ntiles * pl.BM * pl.BM * sizeof(double) > ws_bytes)
-    return OA_ERR_CAPACITY;
-  OvlArgs a;
-  a.X = X; a.ldx = ldx; a.Y = Y; a.ldy = ldy;
-  a.M = M; a.N = N; a.K = K;
-  a.kx0_end = pl.kx0_slice; a.nz_main = pl.nz_main; a.kchunk = pl.kchunk;
-  a.part = (double *)ws;
-  unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
-  if (pl.BM == 128)
-    return launch_ovl_tile<T128, SYM, YJ>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
-  return launch_ovl_tile<T64, SYM, YJ>(s, pl, a, kx0_end, alpha, C, ldc, diag, md);
+  oa_ovl_args a;
+  const int st = fill_ovl(pl, M, N, K, X, ldx, Y, ldy, kx0_end, alpha, C, ldc, diag, maxdev, ws,
+                          ws_bytes, &a);
+  if (st) return st;
+  if (pl.BM == 128) launch_ovl_tile<T128, SYM, YJ>(s, pl, a);
+  else launch_ovl_tile<T64, SYM, YJ>(s, pl, a);
+  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+}
+
+int oa_ovl_fill(int n, int K, const double *psi, long ld, int kx0_end, double alpha, double *S,
+                void *ws, size_t ws_bytes, oa_ovl_args *a, int *blocks, int *rblocks) {
+  const OvlPlan pl = plan_ovl(n, n, K, kx0_end, true);
+  *blocks = ovl_blocks(pl);
+  *rblocks = reduce_blocks(pl);
+  return fill_ovl(pl, n, n, K, psi, ld, psi, ld, kx0_end, alpha, S, n, 0.0, nullptr, ws, ws_bytes,
+                  a);
+}
+
+int oa_ovl_grouped(hipStream_t s, int bm, const oa_group &g) {
+  const oa_ovl_args *t = reinterpret_cast<const oa_ovl_args *>(g.args);
+  if (bm == 128)
+    hipLaunchKernelGGL(ovl_f64_grouped<T128>, dim3(g.total), dim3(T128::NTHR), 0, s, t, g.prefix,
+                       g.count);
+  else
+    hipLaunchKernelGGL(ovl_f64_grouped<T64>, dim3(g.total), dim3(T64::NTHR), 0, s, t, g.prefix,
+                       g.count);
+  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+}
+
+int oa_ovl_reduce_grouped(hipStream_t s, const oa_group &g) {
+  hipLaunchKernelGGL(ovl_reduce_grouped, dim3(g.total), dim3(1024), 0, s,
+                     reinterpret_cast<const oa_ovl_args *>(g.args), g.prefix, g.count);
+  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
+}
+
+void oa_gemm_f64_group(const oa_gemm_problem *p, int count, int *tile, int *blocks) {
+  long all128 = 0, all64 = 0;
+  for (int i = 0; i < count; i++) {
+    all128 += gemm_tiles(p[i], 128, 128);
+    all64 += gemm_tiles(p[i], 64, 64);
+  }
+  for (int i = 0; i < count; i++) {
+    tile[i] = pick_tile(gemm_tiles(p[i], 128, 128), gemm_tiles(p[i], 64, 64), all128, all64);
+    with_tile((TilePick)tile[i], [&](auto c) {
+      typedef decltype(c) C;
+      blocks[i] = (int)((gemm_tiles(p[i], C::BM, C::BN) + 7) / 8 * 8);
+    });
+  }
+}
+
+int oa_gemm_f64_grouped(hipStream_t s, int tile, const oa_group &g) {
+  with_tile((TilePick)tile, [&](auto c) {
+    typedef decltype(c) C;
+    hipLaunchKernelGGL(gemm_f64_grouped<C>, dim3(g.total), dim3(C::NTHR), 0, s,
+                       reinterpret_cast<const oa_gemm_problem *>(g.args), g.prefix, g.count);
+  });
+  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
 int oa_launch_overlap_f64(hipStream_t s, int n, int K, const double *psi, long ld, int kx0_end,

@@ -291,6 +291,39 @@ struct oa_rows_args {
   double *diagv;
 };
 
+// FP64 split-K product over the plane-wave index: partial tiles, and their sum
+// C = alpha X Y^T.
+struct oa_ovl_args {
+  const double *X;
+  long ldx;
+  const double *Y;
+  long ldy;
+  int M, N, K;
+  int kx0_end;          // > 0: z = 0 covers [0, kx0_end) and counts half
+  int nz_main, kchunk;
+  double *part;         // [nz][ntiles][bm][bm]
+  int bm, nz;
+  int kx0_sub;          // columns of X whose product is taken off by half
+  double alpha;
+  double *C;
+  long ldc;
+  double diag;
+  unsigned long long *maxdev;  // max |C - diag I| as bits, or null
+};
+// The overlap of one instance by the single launch's plan, with the workgroups
+// of its two launches; then tables of such instances (one tile edge bm a
+// launch; any in the reduce).  prefix counts workgroups: these grids are exact,
+// not persistent.
+int oa_ovl_fill(int n, int K, const double *psi, long ld, int kx0_end, double alpha, double *S,
+                void *ws, size_t ws_bytes, oa_ovl_args *a, int *blocks, int *rblocks);
+int oa_ovl_grouped(hipStream_t s, int bm, const oa_group &g);
+int oa_ovl_reduce_grouped(hipStream_t s, const oa_group &g);
+// Plain products (no transposes) launched together: the tile (0 .. 3) and the
+// workgroups of each; then a table of those that share a tile.
+constexpr int OA_GEMM_TILES = 4;
+void oa_gemm_f64_group(const oa_gemm_problem *p, int count, int *tile, int *blocks);
+int oa_gemm_f64_grouped(hipStream_t s, int tile, const oa_group &g);
+
 // Split-precision layout of one instance (digit workspace offsets).
 struct oa_split_plan {
   int dt, S, es, tile;

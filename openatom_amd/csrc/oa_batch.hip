@@ -194,6 +194,15 @@ void add_group(Blob &blob, std::vector<Launch> &seq, int kind, int phase, int va
   seq.push_back(L);
 }
 
+// 0 .. count - 1 by falling key.
+template <class Key>
+std::vector<int> sorted(int count, Key key) {
+  std::vector<int> v(count);
+  for (int i = 0; i < count; i++) v[i] = i;
+  std::stable_sort(v.begin(), v.end(), [&](int i, int j) { return key(i) > key(j); });
+  return v;
+}
+
 // Address range of a matrix.
 struct Range {
   const double *lo, *hi;
@@ -356,12 +365,14 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
         blob, b->seq, LK_SPLIT, OA_SP_SLICE, 128, b->ip,
         [&](const InstPlan &, int i) { return sa[i].sl; },
         [&](const InstPlan &, int i) { return sa[i].items_sl; }, all, fix);
+    // long items first: short ones fill the end of the launch
+    std::vector<int> order = sorted(count, [&](int i) { return b->ip[i].sp.ksub; });
     for (int tile : {128, 64}) {
       auto sel = [tile](const InstPlan &p) { return p.tile == tile; };
       add_group<oa_digit_args>(
           blob, b->seq, LK_SPLIT, OA_SP_DIGIT0, tile, b->ip,
           [&](const InstPlan &, int i) { return sa[i].d0; },
-          [&](const InstPlan &, int i) { return sa[i].items_d0; }, sel, fix);
+          [&](const InstPlan &, int i) { return sa[i].items_d0; }, sel, fix, &order);
     }
     for (int tile : {128, 64}) {
       auto sel = [tile](const InstPlan &p) { return p.tile == tile; };
@@ -440,12 +451,13 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
         blob, b->seq, LK_SPLIT, OA_SP_ROWS, 128, b->ip,
         [&](const InstPlan &, int i) { return sa[i].rows; },
         [&](const InstPlan &, int i) { return sa[i].items_rows; }, all, fix);
+    std::vector<int> order = sorted(count, [&](int i) { return b->ip[i].n; });
     for (int tile : {128, 64}) {
       auto sel = [tile](const InstPlan &p) { return p.tile == tile; };
       add_group<oa_digit_args>(
           blob, b->seq, LK_SPLIT, OA_SP_DIGIT1, tile, b->ip,
           [&](const InstPlan &, int i) { return sa[i].d1; },
-          [&](const InstPlan &, int i) { return sa[i].items_d1; }, sel, fix);
+          [&](const InstPlan &, int i) { return sa[i].items_d1; }, sel, fix, &order);
     }
   } else {
     for (std::vector<int> &run : runs(

@@ -252,10 +252,11 @@ struct oa_digit_args {
   const void *Y;  // k-blocked digits, rows n
   long ldy, sy;
   int M, N;       // output extent
-  int kc;         // contraction length per split (elements) or total
+  int kc;         // contraction length of a chunk (elements) or total
   int kfull;      // contraction extent of the digit arrays (padded)
-  int ntiles, nz; // MODE 0: symmetric tiles, splits
-  double *part;   // MODE 0 output
+  int ntiles, nz; // MODES 0 and 2: tiles, chunks
+  int nsub, ksub; // and parts of a chunk, columns of one
+  double *part;   // MODES 0 and 2: output
   const unsigned long long *chunk_max;  // MODE 0: per chunk scale source
   double *out;    // MODE 1 output
   long ldo;
@@ -329,7 +330,8 @@ struct oa_split_plan {
   int dt, S, es, tile;
   int adaptive;     // per chunk slice counts (OA_PREC_ADAPTIVE)
   int np, Kp;       // padded rows / columns (multiples of the tile)
-  int kchunk, nz;   // psi chunks: scale blocks and split-K units
+  int kchunk, nz;   // psi chunks: scale blocks
+  int nsub, ksub;   // parts of a chunk and their columns: split-K units
   int ntiles;       // upper-triangle tiles of S
   size_t off_ds, off_db, off_dt, off_maxS, off_maxB, off_fexp, off_diag, off_part, off_md,
       off_sl;

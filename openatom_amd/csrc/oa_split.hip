@@ -638,15 +638,32 @@ __device__ __forceinline__ void upper_tile_d(int tile, int T, int &bi, int &bj) 
 // Panels hold TILE rows x 32 bytes per slice with the two 16-byte halves of
 // row r swapped when bit 3 of r is set, which spreads any 16 consecutive
 // lanes' 16-byte fragment reads over all 64 LDS banks.
-template <int DT, int NL, int WI, int WJ, int TILE, int TN = TILE>
+// dma(q) issues the part q of NL of the wave's loads of a later stage.  From 4
+// int8 levels on they go between the MFMAs of the Y slices, and the next slice
+// is read ahead of the current one's MFMAs: with all loads at the head of the
+// stage eight waves queued for the address unit while the matrix cores waited
+// (overlap n = 777 int8x5 740 -> 691 us, n = 1024 int8x6a 3.02 -> 2.84 ms; at 3
+// levels, where memory bounds the stage, no gain).
+template <int DT, int NL, int WI, int WJ, int TILE, int TN, class Dma>
 __device__ __forceinline__ void digit_stage(const char *Xs, const char *Ys, int xrow, int yrow,
                                             int lane,
-                                            typename DTraits<DT>::acc_t (&acc)[NL][WI][WJ]) {
+                                            typename DTraits<DT>::acc_t (&acc)[NL][WI][WJ],
+                                            Dma &&dma) {
   constexpr int PANEL = TILE * 32;   // X slice panel (TILE rows of 32 bytes)
   constexpr int YPANEL = TN * 32;    // Y slice panel (TN rows)
+  constexpr bool AHEAD = DT == DT_I8 && NL >= 4;
   const int r = lane & 31;
   const int boff = r * 32 + 16 * ((lane >> 5) ^ ((r >> 3) & 1));
-  i4v a[NL][WI];
+  i4v a[NL][WI], b[WJ], next[WJ];
+  auto read_b = [&](int q, i4v(&d)[WJ]) {
+#pragma unroll
+    for (int j = 0; j < WJ; j++)
+      d[j] = *reinterpret_cast<const i4v *>(Ys + q * YPANEL + (yrow + j * 32) * 32 + boff);
+  };
+  if (!AHEAD)
+#pragma unroll
+    for (int q = 0; q < NL; q++) dma(q);
+  if (AHEAD) read_b(0, next);
 #pragma unroll
   for (int p = 0; p < NL; p++)
 #pragma unroll
@@ -654,10 +671,16 @@ __device__ __forceinline__ void digit_stage(const char *Xs, const char *Ys, int 
       a[p][i] = *reinterpret_cast<const i4v *>(Xs + p * PANEL + (xrow + i * 32) * 32 + boff);
 #pragma unroll
   for (int q = 0; q < NL; q++) {
-    i4v b[WJ];
+    if (AHEAD) {
 #pragma unroll
-    for (int j = 0; j < WJ; j++)
-      b[j] = *reinterpret_cast<const i4v *>(Ys + q * YPANEL + (yrow + j * 32) * 32 + boff);
+      for (int j = 0; j < WJ; j++) b[j] = next[j];
+      if (q + 1 < NL) read_b(q + 1, next);
+      __builtin_amdgcn_sched_barrier(0);
+      dma(q);
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      read_b(q, b);
+    }
 #pragma unroll
     for (int p = 0; p + q < NL; p++)
 #pragma unroll
@@ -665,6 +688,7 @@ __device__ __forceinline__ void digit_stage(const char *Xs, const char *Ys, int 
 #pragma unroll
         for (int j = 0; j < WJ; j++)
           acc[p + q][i][j] = mfma_digit<DT>(a[p][i], b[j], acc[p + q][i][j]);
+    if (AHEAD) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -716,7 +740,7 @@ struct DigitCfg {
 };
 
 // C[m][n] = sum over the contraction of level-grouped digit products, for one
-// output tile (bi, bj) and, in MODES 0 and 2, one chunk z.
+// output tile (bi, bj) and, in MODES 0 and 2, unit u: part u % nsub of chunk z.
 //   MODE 0: symmetric split-K partial tiles of S; NLR slices, levels < NLR.
 //   MODE 1: back-multiply with T = D + X: out[m][n] = alpha (D_m psi~[m][n]
 //           + 2^(f_m + e(n) - 14) C) + beta out, where C uses NLR slices of
@@ -730,7 +754,7 @@ struct DigitCfg {
 //   TN: output columns of the tile (TILE, or 2 TILE for the wide back-multiply
 //       tile of 64 x 64 wave tiles, used at two levels or fewer).
 template <int DT, int S, int MODE, int NLB, int TILE, int NLR, int TN = TILE>
-__device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int bj, int z,
+__device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int bj, int z, int u,
                                            int tile, int SD, char *smem) {
   typedef typename DTraits<DT>::acc_t ACC;
   typedef DigitCfg<DT, S, MODE, NLB, TILE> C;
@@ -764,8 +788,8 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
   constexpr int PROMOTE = (DT == DT_I8) ? (1 << 30) : 128 / SK;
 
   const int m0 = bi * TILE, n0 = bj * TN;
-  const int ka = (MODE != 1) ? z * a.kc : 0;
-  const int kb = (MODE != 1) ? min(a.kfull, ka + a.kc) : a.kfull;
+  const int ka = (MODE != 1) ? z * a.kc + (u - z * a.nsub) * a.ksub : 0;
+  const int kb = (MODE != 1) ? min(min(a.kfull, (z + 1) * a.kc), ka + a.ksub) : a.kfull;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int xrow = (w / WC) * 32 * WI, yrow = (w % WC) * 32 * WJ;
 
@@ -787,7 +811,7 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
   const char *Xg = reinterpret_cast<const char *>(a.X);
   const char *Yg = reinterpret_cast<const char *>(a.Y);
   const size_t sx = a.sx, sy = a.sy, ldx = a.ldx, ldy = a.ldy;
-  const int nst = (kb - ka) / SK;
+  const int nst = max(0, kb - ka) / SK;
   // MODE 1 with int8 digits contracts the tile's own ND row blocks last, so
   // their NL slices are still in the ring when the epilogue rebuilds psi~
   // (those blocks of DB are the psi digits of the tile's output rows).  The
@@ -822,12 +846,13 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
     voff[j] = (unsigned)(r * SK * ES + h * 16);
     loff[j] = x ? p * PANEL + q * 1024 : NL * PANEL + p * YPANEL + q * 1024;
   }
-  auto issue = [&](int st) {
+  // part q of NL of the wave's loads of stage st
+  auto issue = [&](int st, int q) {
     int kblk = DIAG_LDS ? st + rot : (ka + st * SK) / SK;
     if (DIAG_LDS && kblk >= nst) kblk -= nst;
     char *buf = smem + (st % NBUF) * STAGE;
 #pragma unroll
-    for (int j = 0; j < PERW; j++) {
+    for (int j = q * PERW / NL; j < (q + 1) * PERW / NL; j++) {
       if (NHI != 0 && j == PERW - 1 && !whi) break;
       const char *g = sbase[j] + (size_t)kblk * spitch[j] + voff[j];
       __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void *)(buf + loff[j]),
@@ -851,14 +876,19 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
   };
 #pragma unroll
   for (int st = 0; st < NBUF - 1; st++)
-    if (st < nst) issue(st);
+#pragma unroll
+    for (int q = 0; q < NL; q++)
+      if (st < nst) issue(st, q);
   for (int s = 0; s < nst; s++) {
     // stages s+1 .. min(nst-1, s+NBUF-2) may stay in flight
     wait_stages(min(nst - 1 - s, NBUF - 2));
     ring_barrier();
-    if (s + NBUF - 1 < nst) issue(s + NBUF - 1);
+    const bool more = s + NBUF - 1 < nst;
     const char *cur = smem + (s % NBUF) * STAGE;
-    digit_stage<DT, NL, WI, WJ, TILE, TN>(cur, cur + NL * PANEL, xrow, yrow, lane, acc);
+    digit_stage<DT, NL, WI, WJ, TILE, TN>(cur, cur + NL * PANEL, xrow, yrow, lane, acc,
+                                          [&](int q) {
+                                            if (more) issue(s + NBUF - 1, q);
+                                          });
     if (DT != DT_I8 && ((s + 1) % PROMOTE == 0 || s + 1 == nst)) {
 #pragma unroll
       for (int i = 0; i < WI; i++)
@@ -918,7 +948,7 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
       const int ex = chunk_exp(__longlong_as_double((long long)a.chunk_max[z]));
       const int sc = (MODE == 0) ? 2 * (ex - 7)
                                  : ex + chunk_exp(__longlong_as_double((long long)a.colmax[z])) - 14;
-      double *pt = a.part + ((size_t)z * a.ntiles + tile) * (TILE * TILE) + ln;
+      double *pt = a.part + ((size_t)u * a.ntiles + tile) * (TILE * TILE) + ln;
 #pragma unroll
       for (int v = 0; v < 16; v++) {
         const int lm = xr + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
@@ -1025,52 +1055,47 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
 }
 
 
-// Item decoding.  An adaptive split spreads the chunks over the XCDs: the
-// dispatcher gives XCD x the contiguous item range x*per .. (x+1)*per - 1,
-// which covers consecutive chunks; with nz = 8c the chunk order is permuted
-// so that XCD x takes chunks x, x + 8, ..., and every XCD gets a like mix of
-// heavy (leading, more slices) and light chunks.  Tiles of one chunk stay on
-// one XCD (their operand panels share its L2).
+// Item decoding.  XCD x of 8 gets the items x*per .. (x+1)*per - 1.  Where the
+// number of units (chunks, or their parts) is a multiple of 8 they are dealt to
+// the XCDs in turn, so that each gets a like mix of heavy (leading, more slices)
+// and light chunks.  The tiles of a unit share its operand panels in one L2.
+__device__ __forceinline__ int deal8(int pos, int units) {
+  return (units & 7) ? pos : (pos % (units >> 3)) * 8 + pos / (units >> 3);
+}
+
 template <int DT, int S, int MODE, int NLB, int TILE>
 __device__ __forceinline__ void digit_body(const oa_digit_args &a, int logical, char *smem) {
   constexpr int NL = DigitCfg<DT, S, MODE, NLB, TILE>::NL;
   constexpr bool ADA_OK = (DT == DT_I8) && (MODE != 2) && (S >= ADA_SMIN_MAX);
   const bool ada = ADA_OK && a.slices != nullptr;
-  int bi, bj, z = 0, tile = logical;
-  if (MODE == 0) {
+  int bi, bj, z, u = 0, tile = logical;
+  if (MODE != 1) {
+    const int units = a.nz * a.nsub;
+    if (logical >= units * a.ntiles) return;
     tile = logical % a.ntiles;
-    z = logical / a.ntiles;
-    if (ada && (a.nz & 7) == 0) {
-      const int c = a.nz >> 3;
-      z = (z % c) * 8 + z / c;
+    u = deal8(logical / a.ntiles, units);
+    z = u / a.nsub;
+    if (MODE == 0) {
+      upper_tile_d(tile, cdv(a.M, TILE), bi, bj);
+    } else {
+      const int T = cdv(a.M, TILE);
+      bi = tile % T;
+      bj = tile / T;
     }
-    upper_tile_d(tile, cdv(a.M, TILE), bi, bj);
-  } else if (MODE == 2) {
-    const int T = cdv(a.M, TILE);
-    tile = logical % a.ntiles;
-    z = logical / a.ntiles;
-    bi = tile % T;
-    bj = tile / T;
   } else {
-    const int tm = cdv(a.M, TILE);
+    const int tm = cdv(a.M, TILE), cpt = a.kchunk / TILE;  // kchunk: a multiple of TILE
     bi = logical % tm;
     bj = logical / tm;
-    if (ada) {
-      // chunk of the output columns (kchunk is a multiple of TILE)
-      const int cpt = a.kchunk / TILE;
-      if ((a.nz & 7) == 0 && cdv(a.N, TILE) == a.nz * cpt) {
-        const int c = a.nz >> 3, zl = bj / cpt;
-        bj = ((zl % c) * 8 + zl / c) * cpt + bj % cpt;
-      }
-      z = bj / cpt;
-    }
+    if (bj >= cdv(a.N, TILE)) return;
+    if (ada && cdv(a.N, TILE) == a.nz * cpt) bj = deal8(bj / cpt, a.nz) * cpt + bj % cpt;
+    z = bj / cpt;
   }
   if constexpr (ADA_OK) {
     if (ada) {
       const int sz = a.slices[z];
       if constexpr (MODE == 0) {
         level_switch<ADA_SMIN, NL>(sz, [&](auto c) {
-          digit_core<DT, S, MODE, NLB, TILE, decltype(c)::value>(a, bi, bj, z, tile, S, smem);
+          digit_core<DT, S, MODE, NLB, TILE, decltype(c)::value>(a, bi, bj, z, u, tile, S, smem);
         });
       } else {
         constexpr int LO = (NLB - (S - ADA_SMIN) > 1) ? NLB - (S - ADA_SMIN) : 1;
@@ -1086,19 +1111,19 @@ __device__ __forceinline__ void digit_body(const oa_digit_args &a, int logical, 
             if (bj & 1) return;
             level_switch<LO, (NLB < 2 ? NLB : 2)>(nlr, [&](auto c) {
               digit_core<DT, S, MODE, NLB, TILE, decltype(c)::value, 2 * TILE>(
-                  a, bi, bj >> 1, z, tile, sz, smem);
+                  a, bi, bj >> 1, z, u, tile, sz, smem);
             });
             return;
           }
         }
         level_switch<LO, NLB>(nlr, [&](auto c) {
-          digit_core<DT, S, MODE, NLB, TILE, decltype(c)::value>(a, bi, bj, z, tile, sz, smem);
+          digit_core<DT, S, MODE, NLB, TILE, decltype(c)::value>(a, bi, bj, z, u, tile, sz, smem);
         });
       }
       return;
     }
   }
-  digit_core<DT, S, MODE, NLB, TILE, NL>(a, bi, bj, z, tile, S, smem);
+  digit_core<DT, S, MODE, NLB, TILE, NL>(a, bi, bj, z, u, tile, S, smem);
 }
 
 template <int DT, int S, int MODE, int NLB, int TILE>
@@ -1119,64 +1144,87 @@ __attribute__((amdgpu_waves_per_eu(DigitCfg<DT, S, MODE, NLB, TILE>::WPE,
                                    DigitCfg<DT, S, MODE, NLB, TILE>::WPE))) void digit_nt_grouped(
     const oa_digit_args *__restrict__ t, const int *__restrict__ prefix, int count) {
   __shared__ __attribute__((aligned(1024))) char smem[DigitCfg<DT, S, MODE, NLB, TILE>::SMEM];
-  for_items(prefix[count], [&](int item) {
-    const int i = group_find(prefix, count, item);
-    digit_body<DT, S, MODE, NLB, TILE>(t[i], item - prefix[i], smem);
-  });
-}
-
-// ------------------------------------------------------------ reduce
-// Item = 256 consecutive elements of the upper-triangle partial tiles: fixed
-// order sum over the splits, the FP64 kx0 term (weight 1/2) of a plane of
-// at most KX0_FP64_MAX columns (a wider one is in the digits), mirror,
-// max|S - d I|.
-template <int TILE>
-__device__ __forceinline__ void split_reduce_body(const oa_sreduce_args &a, int item) {
-  const int n = a.n;
-  const int T = cdv(n, TILE);
-  const int ntiles = T * (T + 1) / 2;
-  const long idx = (long)item * 256 + threadIdx.x;
-  const int tile = (int)(idx / (TILE * TILE));
-  if (tile >= ntiles) return;
-  const int e = (int)(idx % (TILE * TILE));
-  const int lm = e / TILE, ln = e % TILE;
-  int bi, bj;
-  upper_tile_d(tile, T, bi, bj);
-  if (bi == bj && ln < lm) return;
-  const int i = bi * TILE + lm, j = bj * TILE + ln;
-  if (i >= n || j >= n) return;
-  double s = 0.0;
-  for (int z = 0; z < a.nz; z++) s += a.part[((long)z * ntiles + tile) * (TILE * TILE) + e];
-  double g = 0.0;
-  if (a.kx0_end <= KX0_FP64_MAX)
-    for (int k = 0; k < a.kx0_end; k++)
-      g = fma(a.psi[(long)i * a.ld + k], a.psi[(long)j * a.ld + k], g);
-  s = fma(a.alpha, s, __dmul_rn(0.5 * a.alpha, g));
-  a.S[(long)i * n + j] = s;
-  a.S[(long)j * n + i] = s;
-  if (a.maxdev) {
-    const double dv = fabs(s - (i == j ? a.diag : 0.0));
-    atomicMax(a.maxdev, (unsigned long long)__double_as_longlong(dv));
+  // prefix counts multiples of 8: every XCD takes an eighth of each instance
+  // (ranges of items over all instances gave one XCD the large ones)
+  const int x = blockIdx.x & 7, per = prefix[count] >> 3, slots = (int)gridDim.x >> 3;
+  for (int pos = blockIdx.x >> 3; pos < per; pos += slots) {
+    const int i = group_find(prefix, count, pos << 3);
+    const int each = (prefix[i + 1] - prefix[i]) >> 3;
+    digit_body<DT, S, MODE, NLB, TILE>(t[i], x * each + pos - (prefix[i] >> 3), smem);
   }
 }
 
+// ------------------------------------------------------------ reduce
+// Item = 16 x 16 outputs of the upper-triangle partial tiles.  The four waves of
+// group q of 1024 threads add units q, q + 4, ... in order, then the groups
+// combine: a fixed order with more loads in flight (one thread a sum took 18 us
+// at n = 512 with 32 partials, 91 at 1024; this 10 and 64).  Then the FP64 kx0 term (weight
+// 1/2) of a plane of at most KX0_FP64_MAX columns (a wider one is in the
+// digits), the mirror from LDS, and max|S - d I|.
 template <int TILE>
-__global__ __launch_bounds__(256) void split_reduce_kernel(oa_sreduce_args a, int total) {
+__device__ __forceinline__ void split_reduce_body(const oa_sreduce_args &a, int item) {
+  constexpr int PB = TILE / 16;
+  __shared__ double sums[4][256];
+  __shared__ double out[16][17];
+  const int n = a.n;
+  const int T = cdv(n, TILE);
+  const int ntiles = T * (T + 1) / 2;
+  const int tile = item / (PB * PB), patch = item % (PB * PB);
+  if (tile >= ntiles) return;
+  int bi, bj;
+  upper_tile_d(tile, T, bi, bj);
+  const int pi = (patch / PB) * 16, pj = (patch % PB) * 16;
+  if (bi * TILE + pi >= n || bj * TILE + pj >= n || (bi == bj && pi > pj)) return;
+  const int t = threadIdx.x & 255, q = threadIdx.x >> 8, lr = t >> 4, lc = t & 15;
+  const double *p = a.part + (long)tile * (TILE * TILE) + (pi + lr) * TILE + pj + lc;
+  const long zs = (long)ntiles * (TILE * TILE);
+  double s = 0.0;
+#pragma unroll 4
+  for (int z = q; z < a.nz; z += 4) s += p[z * zs];
+  sums[q][t] = s;
+  __syncthreads();
+  const bool diag = bi == bj && pi == pj;
+  if (q == 0) {
+    const int i = bi * TILE + pi + lr, j = bj * TILE + pj + lc;
+    const bool in = i < n && j < n && !(diag && lc < lr);
+    s = ((sums[0][t] + sums[1][t]) + sums[2][t]) + sums[3][t];
+    if (in) {
+      double g = 0.0;
+      if (a.kx0_end <= KX0_FP64_MAX)
+        for (int k = 0; k < a.kx0_end; k++)
+          g = fma(a.psi[(long)i * a.ld + k], a.psi[(long)j * a.ld + k], g);
+      s = fma(a.alpha, s, __dmul_rn(0.5 * a.alpha, g));
+      a.S[(long)i * n + j] = s;
+      if (a.maxdev) {
+        const double dv = fabs(s - (i == j ? a.diag : 0.0));
+        atomicMax(a.maxdev, (unsigned long long)__double_as_longlong(dv));
+      }
+    }
+    out[lr][lc] = s;
+  }
+  __syncthreads();
+  const int mi = bi * TILE + pi + lc, mj = bj * TILE + pj + lr;  // S[mj][mi] = out[lc][lr]
+  if (q == 0 && mi < n && mj < n && !(diag && lr < lc)) a.S[(long)mj * n + mi] = out[lc][lr];
+  __syncthreads();  // the next item overwrites `out`
+}
+
+template <int TILE>
+__global__ __launch_bounds__(1024) void split_reduce_kernel(oa_sreduce_args a, int total) {
   const int item = single_item(total);
   if (item < total) split_reduce_body<TILE>(a, item);
 }
 
 template <int TILE>
-__global__ __launch_bounds__(256) void split_reduce_grouped(const oa_sreduce_args *__restrict__ t,
-                                                            const int *__restrict__ prefix,
-                                                            int count) {
+__global__ __launch_bounds__(1024) void split_reduce_grouped(
+    const oa_sreduce_args *__restrict__ t, const int *__restrict__ prefix, int count) {
   for_items(prefix[count], [&](int item) {
     const int i = group_find(prefix, count, item);
     split_reduce_body<TILE>(t[i], item - prefix[i]);
   });
 }
 
-// Asymmetric reduce: L[i][j] = alpha * sum_z part (fixed order), all tiles.
+// Asymmetric reduce: L[i][j] = alpha * sum_z part, all tiles, in the symmetric
+// reduce's order.
 template <int TILE>
 __global__ __launch_bounds__(256) void lambda_reduce_kernel(const double *__restrict__ part,
                                                             int n, int nz, double alpha,
@@ -1189,8 +1237,12 @@ __global__ __launch_bounds__(256) void lambda_reduce_kernel(const double *__rest
   const int e = (int)(idx % (TILE * TILE));
   const int i = (tile % T) * TILE + e / TILE, j = (tile / T) * TILE + e % TILE;
   if (i >= n || j >= n) return;
-  double s = 0.0;
-  for (int z = 0; z < nz; z++) s += part[((long)z * ntiles + tile) * (TILE * TILE) + e];
+  double q[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int z = 0; z < nz; z += 4)
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (z + k < nz) q[k] += part[((long)(z + k) * ntiles + tile) * (TILE * TILE) + e];
+  const double s = ((q[0] + q[1]) + q[2]) + q[3];
   L[(long)i * n + j] = alpha * s;
 }
 
@@ -1246,6 +1298,33 @@ int chunk_len(int dt, int S, int n, int K) {
   return max(128, kchunk / 128 * 128);
 }
 
+// Parts of a chunk in the split-K products over ntiles 128-tiles (any tile
+// shape and launch form: the parts decide the rounding of S).  32 CUs of an XCD
+// each take one item at a time, so a count that fills them a little over once
+// leaves most idle half of the time.  The cost of a depth: rounds of items, each
+// of stages at 0.35 us and 0.061 us per level product (measured at 10 and 15
+// products) and 5 us of first loads and partial tile, and the partial tiles
+// written and read.  Measured with 1, 2, 3, 4 parts (overlap / reduce, us): n =
+// 512 (npw 65536) int8x6a 336, 236, 234, 226 / 10, 17, 26, 34; n = 777 (50021)
+// int8x5 688, 570, 627, 586 / 15, 20, 24, 33; n = 1024 (262144) int8x6a 2777,
+// 2624, 2630, 2658 / 64, 123, 178, 233.  (One workgroup per item, as they come
+// free, against resident workgroups with fixed shares: 249 -> 237 us at 512,
+// 598 -> 564 at 777.)
+int chunk_parts(int dt, int S, bool adaptive, int ntiles, int nz, int kchunk) {
+  const int stages = kchunk / (dt == DT_I8 ? 32 : (dt == DT_F32 ? 8 : 16));
+  const int lv = adaptive && S > 3 ? S - 2 : S;  // most chunks drop slices
+  const double stage_us = 0.35 + lv * (lv + 1) / 2 * 0.061;
+  int best = 1;
+  double best_cost = 0.0;
+  for (int p = 1; p <= 8 && 2 * p <= stages; p++) {
+    const int rounds = cdv(cdv(nz * p * ntiles, 8), 32);
+    const double cost = rounds * (cdv(stages, p) * stage_us + 5.0) +
+                        (double)nz * p * ntiles * 0.06;
+    if (p == 1 || cost < best_cost) { best = p; best_cost = cost; }
+  }
+  return best;
+}
+
 // Levels the back-multiply's X psi products keep (MODE 1).
 int backmul_levels(int S, bool lean) {
   const int nl = lean ? S - 2 : S - 1;
@@ -1273,6 +1352,9 @@ oa_split_plan make_plan(int prec, int n, int K, int tile) {
   pl.kchunk = chunk_len(pl.dt, pl.S, n, K);
   pl.nz = cdv(pl.Kp, pl.kchunk);
   pl.adaptive = (prec & OA_PREC_ADAPTIVE) ? 1 : 0;
+  const int T128 = cdv(n, 128);
+  pl.nsub = chunk_parts(pl.dt, pl.S, pl.adaptive != 0, T128 * (T128 + 1) / 2, pl.nz, pl.kchunk);
+  pl.ksub = cdv(cdv(pl.kchunk, pl.nsub), DBK) * DBK;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -1287,7 +1369,7 @@ oa_split_plan make_plan(int prec, int n, int K, int tile) {
   pl.off_fexp = take((size_t)pl.np * 4);
   pl.off_diag = take((size_t)pl.np * 8);
   pl.off_md = take(8);
-  pl.off_part = take((size_t)pl.nz * pl.ntiles * tile * tile * 8);
+  pl.off_part = take((size_t)pl.nz * pl.nsub * pl.ntiles * tile * tile * 8);
   pl.off_sl = take((size_t)pl.nz * 4);
   pl.total = off;
   return pl;
@@ -1379,12 +1461,14 @@ void fill_inst(const oa_split_plan &pl, int n, int K, const double *psi, long ld
   a.kfull = pl.Kp;
   a.ntiles = pl.ntiles;
   a.nz = pl.nz;
+  a.nsub = pl.nsub;
+  a.ksub = pl.ksub;
   a.part = reinterpret_cast<double *>(ws + pl.off_part);
   a.chunk_max = maxS;
   a.slices = slices;
-  r->items_d0 = pl.ntiles * pl.nz;
-  r->rd = oa_sreduce_args{a.part, n, pl.nz, alpha, psi, ld, kx0_end, 0, Sout, 0.0, nullptr};
-  r->items_rd = cdv(pl.ntiles * tile * tile, 256);
+  r->items_d0 = cdv(pl.ntiles * pl.nz * pl.nsub, 8) * 8;
+  r->rd = oa_sreduce_args{a.part, n, pl.nz * pl.nsub, alpha, psi, ld, kx0_end, 0, Sout, 0.0, nullptr};
+  r->items_rd = pl.ntiles * (tile / 16) * (tile / 16);
   r->rows = oa_rows_args{T, n, transT, ws + pl.off_dt, pl.np, 0,
                          reinterpret_cast<int *>(ws + pl.off_fexp),
                          reinterpret_cast<double *>(ws + pl.off_diag)};
@@ -1415,7 +1499,7 @@ void fill_inst(const oa_split_plan &pl, int n, int K, const double *psi, long ld
   b.kchunk = pl.kchunk;
   b.nz = pl.nz;
   b.slices = slices;
-  r->items_d1 = cdv(n, tile) * cdv(K, tile);
+  r->items_d1 = cdv(cdv(n, tile) * cdv(K, tile), 8) * 8;
 }
 
 template <int DT, int S>
@@ -1438,13 +1522,13 @@ int run_overlap(hipStream_t s, const oa_split_plan &pl, int n, int K, const doub
   fill_inst(pl, n, K, psi, ld, kx0_end, alpha, Sout, nullptr, 0, 0.0, nullptr, 0, ws, nullptr,
             nullptr, &r);
   launch_slice_psi<DT, S>(s, pl, r, true);
-  OA_LAUNCH_PERSISTENT((digit_nt_kernel<DT, S, 0, S - 1, 128>),
+  OA_LAUNCH_ITEMS((digit_nt_kernel<DT, S, 0, S - 1, 128>),
                   (DigitCfg<DT, S, 0, S - 1, 128>::NTHR), r.items_d0, s, r.d0);
   unsigned long long *md = reinterpret_cast<unsigned long long *>(maxdev);
   if (md) hipLaunchKernelGGL(fill_u64, dim3(1), dim3(64), 0, s, md, 1L);
   r.rd.diag = diag;
   r.rd.maxdev = md;
-  OA_LAUNCH_ITEMS(split_reduce_kernel<128>, 256, r.items_rd, s, r.rd);
+  OA_LAUNCH_ITEMS(split_reduce_kernel<128>, 1024, r.items_rd, s, r.rd);
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
@@ -1489,7 +1573,7 @@ LambdaPlan make_lambda_plan(int prec, int n, int K) {
   lp.off_y = take((size_t)pl.S * pl.np * pl.Kp * pl.es);
   lp.off_mx = take((size_t)2 * pl.nz * 8);
   lp.off_my = take((size_t)2 * pl.nz * 8);
-  lp.off_part = take((size_t)pl.nz * lp.ntiles * 128 * 128 * 8);
+  lp.off_part = take((size_t)pl.nz * pl.nsub * lp.ntiles * 128 * 128 * 8);
   lp.total = off;
   return lp;
 }
@@ -1524,14 +1608,16 @@ int run_lambda(hipStream_t s, const LambdaPlan &lp, int n, int K, const double *
   a.kfull = pl.Kp;
   a.ntiles = lp.ntiles;
   a.nz = pl.nz;
+  a.nsub = pl.nsub;
+  a.ksub = pl.ksub;
   a.part = reinterpret_cast<double *>(ws + lp.off_part);
   a.chunk_max = mx;
   a.colmax = my;
   OA_LAUNCH_PERSISTENT((digit_nt_kernel<DT, S, 2, S - 1, 128>),
-                  (DigitCfg<DT, S, 2, S - 1, 128>::NTHR), lp.ntiles * pl.nz, s, a);
+                  (DigitCfg<DT, S, 2, S - 1, 128>::NTHR), lp.ntiles * pl.nz * pl.nsub, s, a);
   const long total = (long)lp.ntiles * 128 * 128;
   hipLaunchKernelGGL(lambda_reduce_kernel<128>, dim3((unsigned)cdv((int)total, 256)), dim3(256),
-                     0, s, (const double *)a.part, n, pl.nz, alpha, L);
+                     0, s, (const double *)a.part, n, pl.nz * pl.nsub, alpha, L);
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
@@ -1654,7 +1740,7 @@ int grouped_phase(hipStream_t s, int phase, const oa_group &g) {
                         (DigitCfg<DT, S, 0, S - 1, TILE>::NTHR), s, g, oa_digit_args);
       break;
     case OA_SP_REDUCE:
-      OA_LAUNCH_GROUPED(split_reduce_grouped<TILE>, 256, s, g, oa_sreduce_args);
+      OA_LAUNCH_GROUPED(split_reduce_grouped<TILE>, 1024, s, g, oa_sreduce_args);
       break;
     case OA_SP_ROWS:
       OA_LAUNCH_GROUPED((slice_rows_grouped<DT, NLB>), 256, s, g, oa_rows_args);
@@ -1837,7 +1923,7 @@ ZimagPlan make_zimag_plan(int prec, int n, int K) {
   zp.ntiles = T * (T + 1) / 2;
   zp.off_yj = (pl.total + 255) / 256 * 256;
   zp.off_part = zp.off_yj + ((size_t)pl.S * pl.np * pl.Kp * pl.es + 255) / 256 * 256;
-  zp.total = zp.off_part + (size_t)pl.nz * zp.ntiles * 128 * 128 * 8;
+  zp.total = zp.off_part + (size_t)pl.nz * pl.nsub * zp.ntiles * 128 * 128 * 8;
   return zp;
 }
 
@@ -1860,12 +1946,14 @@ int run_zimag(hipStream_t s, const ZimagPlan &zp, int n, double alpha, double *L
   a.kfull = pl.Kp;
   a.ntiles = zp.ntiles;
   a.nz = pl.nz;
+  a.nsub = pl.nsub;
+  a.ksub = pl.ksub;
   a.part = reinterpret_cast<double *>(ws + zp.off_part);
   a.chunk_max = mS;
-  OA_LAUNCH_PERSISTENT((digit_nt_kernel<DT, S, 0, S - 1, 128>),
-                  (DigitCfg<DT, S, 0, S - 1, 128>::NTHR), zp.ntiles * pl.nz, s, a);
-  const oa_sreduce_args rd{a.part, n, pl.nz, alpha, nullptr, 0, 0, 0, Li, 0.0, nullptr};
-  OA_LAUNCH_ITEMS(split_reduce_kernel<128>, 256, cdv(zp.ntiles * 128 * 128, 256), s, rd);
+  OA_LAUNCH_ITEMS((digit_nt_kernel<DT, S, 0, S - 1, 128>),
+                  (DigitCfg<DT, S, 0, S - 1, 128>::NTHR), zp.ntiles * pl.nz * pl.nsub, s, a);
+  const oa_sreduce_args rd{a.part, n, pl.nz * pl.nsub, alpha, nullptr, 0, 0, 0, Li, 0.0, nullptr};
+  OA_LAUNCH_ITEMS(split_reduce_kernel<128>, 1024, zp.ntiles * 64, s, rd);
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 

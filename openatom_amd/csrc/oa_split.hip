@@ -201,6 +201,14 @@ __host__ __device__ __forceinline__ double rinv(int l) {
   return t[l];
 }
 
+// 2^k, -1022 <= k <= 1023.
+__device__ __forceinline__ double pow2(int k) {
+  return __longlong_as_double((long long)(k + 1023) << 52);
+}
+// Added to a row's exponent (at most 1100 in size) where the row's diagonal
+// element is so large or small that scaling it needs care.
+constexpr int WILD_DIAG = 8192;
+
 // Split one value into S digits given its exponent.
 // Only the leading nd digits are formed (the rest are left at 0): an
 // adaptive split keeps s_z <= S digits of chunk z.
@@ -591,8 +599,9 @@ __device__ __forceinline__ void slice_rows_body(const oa_rows_args &a, int r) {
   }
   const int e = chunk_exp(red[0]);
   if (threadIdx.x == 0) {
-    a.fexp[r] = e;
-    a.diagv[r] = (r < n) ? M[(long)r * n + r] : 0.0;
+    const double d = (r < n) ? M[(long)r * n + r] : 0.0;
+    a.fexp[r] = e + (fabs(d) > 1e200 || (d != 0.0 && fabs(d) < 1e-200) ? WILD_DIAG : 0);
+    a.diagv[r] = d;
   }
   for (int c = threadIdx.x; c < npk; c += 256) {
     double d[S];
@@ -941,7 +950,7 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
   for (int j = 0; j < WJ; j++) {
     const int ln = yrow + j * 32 + (lane & 31);
     const int nn = n0 + ln;
-    const int xr = xrow + i * 32;
+    const int xr = xrow + i * 32, xru = (wu / WC) * 32 * WI + i * 32;
     auto level_sum = [&](int v) { return facc[i][j][v]; };
     if (MODE != 1) {
       // the chunk's scale, read once (the partial-tile stores could alias it)
@@ -964,13 +973,25 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
     for (int g = 0; g < 4; g++) {
       // elements v = 4g + r sit in rows mg + r, mg = m0 + xr + 8g + 4 (lane / 32)
       const int mg = m0 + xr + 8 * g + 4 * (lane >> 5);
-      double pd[4] = {0.0, 0.0, 0.0, 0.0}, dv[4];
+      double pd[4] = {0.0, 0.0, 0.0, 0.0}, dv[4], rs[4];
       int fe[4];
+      // T's exponents and diagonal of the 8 rows of both halves of the wave (the
+      // arrays reach over whole tiles), by scalar loads: as vector loads they
+      // were 64 of a wave's 100 memory instructions in here.  With the factors
+      // below and absent digits left out: T psi n = 512 int8x6a 432 -> 400 us, n
+      // = 1024 4.70 -> 4.51 ms
+      bool wild = abs(ez) > 900;
+      const auto *gd = (const __attribute__((address_space(4))) double *)(a.diagv + m0 + xru + 8 * g);
+      const auto *gf = (const __attribute__((address_space(4))) int *)(a.fexp + m0 + xru + 8 * g);
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int m = min(mg + r, a.M - 1);
-        dv[r] = a.diagv[m];
-        fe[r] = a.fexp[m];
+        const double d0 = gd[r], d1 = gd[4 + r];
+        const int f0 = gf[r], f1 = gf[4 + r];
+        wild = wild || abs(f0) > 900 || abs(f1) > 900;
+        dv[r] = lane >> 5 ? d1 : d0;
+        fe[r] = lane >> 5 ? f1 : f0;
+        const int h0 = (f0 - 7 + 1023) << 20, h1 = (f1 - 7 + 1023) << 20;
+        rs[r] = __hiloint2double(lane >> 5 ? h1 : h0, 0);  // 2^(f - 7)
       }
       // psi~[m][nn] for these rows, rebuilt from all S digits; with DIAG_LDS
       // the leading NL slices come from the ring: row block m0/SK + xr/SK was
@@ -980,14 +1001,16 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
       if constexpr (DT == DT_I8) {
         // the four rows' digits of slice p sit in one dword (byte r = row
         // mg + r); the leading min(S, 4) digits combine exactly in int32
-        // (|sum| <= 127 (254^3 + 254^2 + 254 + 1) < 2^31), absent digits
-        // (p >= SD) as zeros, and the rest (S > 4) add in FP64
+        // (|sum| <= 127 (254^3 + 254^2 + 254 + 1) < 2^31), absent digits as
+        // zeros, and the rest (S > 4) add in FP64.  A chunk with NLR levels has
+        // SX digits (or fewer, at one level)
+        constexpr int SX = NLR + S - NLB;
         constexpr int PI = S < 4 ? S : 4;
         int wq[S];
 #pragma unroll
         for (int p = 0; p < S; p++) {
           wq[p] = 0;
-          if (p >= SD) continue;
+          if (p >= SX || (NLR == 1 && p >= SD)) continue;
           if (DIAG_LDS && p < NL) {
             const char *yb = smem + ((nst - ND + xr / SK) % NBUF) * STAGE + NL * PANEL + p * YPANEL;
             wq[p] = *reinterpret_cast<const int *>(
@@ -1004,10 +1027,11 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
         for (int r = 0; r < 4; r++) {
           int iv = 0;
 #pragma unroll
-          for (int p = 0; p < PI; p++) iv = iv * 254 + (int)(int8_t)((wq[p] >> (8 * r)) & 0xff);
+          for (int p = 0; p < PI; p++)  // factors of 24 bits: at most 8,225,917
+            iv = __mul24(iv, 254) + (int)(int8_t)((wq[p] >> (8 * r)) & 0xff);
           double t = 0.0;
 #pragma unroll
-          for (int p = S - 1; p >= PI; p--)
+          for (int p = SX - 1; p >= PI; p--)
             t = fma((double)(int8_t)((wq[p] >> (8 * r)) & 0xff), rinv(p), t);
           pd[r] = fma((double)iv, rinv(PI - 1), t);
         }
@@ -1023,11 +1047,26 @@ __device__ __forceinline__ void digit_core(const oa_digit_args &a, int bi, int b
         }
       }
       // explicit fma / __dmul_rn: the same rounding in every kernel that
-      // inlines this body (single and grouped launches) and every build
-      auto value = [&](int r) {
-        return __dmul_rn(al, fma(dv[r], ldexp(pd[r], ez - 7),
-                                 ldexp(level_sum(4 * g + r), fe[r] + ez - 14)));
-      };
+      // inlines this body (single and grouped launches) and every build.  The
+      // scales are powers of two, applied as factors (ldexp runs at a quarter
+      // of a multiplication's rate) unless one could leave the range of normal
+      // numbers; both ways round alike.
+      double val[4];
+      if (wild || __any(!(fabs(al) < 1e30 && fabs(al) > 1e-30))) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int f = fe[r] > WILD_DIAG / 2 ? fe[r] - WILD_DIAG : fe[r];
+          val[r] = __dmul_rn(al, fma(dv[r], ldexp(pd[r], ez - 7),
+                                     ldexp(level_sum(4 * g + r), f + ez - 14)));
+        }
+      } else {
+        const double sc = __dmul_rn(al, pow2(ez - 7));
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          val[r] =
+              __dmul_rn(sc, fma(dv[r], pd[r], __dmul_rn(level_sum(4 * g + r), rs[r])));
+      }
+      auto value = [&](int r) { return val[r]; };
       double *o = a.out + (size_t)mg * a.ldo + nn;
       if (!edge) {
         if (a.beta == 0.0) {

@@ -1019,7 +1019,11 @@ __device__ __forceinline__ void ns_gemm_body(const oa_ns_args &a, int mode, int 
                                              int which, int logical, double *smem) {
   const int t = cdiv(a.np, C::BM);
   if (logical >= t * t) return;
-  if (mode != NS_B1 && (a.rep->done || it > a.maxit)) return;
+  // one answer for the workgroup: during a C launch the first one stores the
+  // report, and waves that saw it differently would go on to different items
+  int ended = mode != NS_B1 && (a.rep->done || it > a.maxit);
+  if (mode == NS_C) ended = __syncthreads_or(ended);
+  if (ended) return;
   const int part = Z ? which & 1 : 0;
   const bool second = (Z ? which >> 1 : which) != 0;
   if (mode == NS_B1 || (mode == NS_C && it >= 2)) {

@@ -401,7 +401,7 @@ int oa_scatter_rows(oa_handle_t h, int count, const int *row0, const int *nrows,
  * and bead; cpaimd.C:2566-2593 builds each instance's PairCalculator pair
  * and Ortho array) -- advance together: every phase
  * of the step (chunk maxima, slicing, overlap products, reduction, each S->T
- * iteration, back-multiply) is ONE persistent grouped launch over all
+ * iteration, back-multiply) is one grouped launch over all
  * instances, walking a device table of per-instance arguments.  Results are
  * those of oa_ortho_step on each instance alone, bit for bit (the digit
  * products are exact and the chunking depends on (n, npw) only). */

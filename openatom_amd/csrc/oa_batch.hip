@@ -1,7 +1,6 @@
 // Batched independent instances: one step of many orthonormalisation
-// problems of uneven size, each phase ONE persistent grouped launch over all
-// instances (split precision) or one grouped launch per S->T phase (both
-// precisions), replayable as a hipGraph, with a tile autotuner.
+// problems of uneven size, each phase one grouped launch over all instances
+// (per tile in use), replayable as a hipGraph, with a tile autotuner.
 //
 // The reference runs one GSP/PC/Ortho instance set per (spin, temper,
 // k-point, bead) index (cpaimd.C:600-664, cpaimd.C:2566-2593); the instances

@@ -19,8 +19,9 @@
 // level L = p + q <= S + 1 (the Ozaki triangular truncation); level sums are
 // combined in FP64 with weights R^(-(L-2)) and the chunk scales.  Because the
 // level sums are exact, every result is independent of the tile shape, the
-// split-K grouping and the launch (single or grouped): only the chunk length
-// enters the numerics, and it depends on (n, K) alone.
+// order of k and the launch (single or grouped): only the chunk length and the
+// parts a chunk is summed in enter the numerics, and they depend on (n, K) and
+// the number of slices alone.
 //
 // Layout.  Every digit matrix (rows R, contraction C) is stored k-blocked:
 // element (p, r, c) at p*R*C + ((c / B)*R + r)*B + c % B with B = 32 bytes of
@@ -1171,7 +1172,7 @@ __attribute__((amdgpu_waves_per_eu(DigitCfg<DT, S, MODE, NLB, TILE>::WPE,
                                    DigitCfg<DT, S, MODE, NLB, TILE>::WPE))) void digit_nt_kernel(
     oa_digit_args a, int total) {
   __shared__ __attribute__((aligned(1024))) char smem[DigitCfg<DT, S, MODE, NLB, TILE>::SMEM];
-  // persistent: one workgroup per CU walks its XCD's items (a workgroup per
+  // back-multiply: one workgroup per CU walks its XCD's items (a workgroup per
   // item paid the 160 KB LDS allocation and wave launch at every tile:
   // int8x6a back-multiply 4.62 -> 4.54 ms, int8x5 5.97 -> 5.79 ms)
   for_items(total, [&](int item) { digit_body<DT, S, MODE, NLB, TILE>(a, item, smem); });
@@ -1324,7 +1325,7 @@ int chunk_len(int dt, int S, int n, int K) {
   const int T128 = cdv(n, 128);
   const long t128 = (long)T128 * (T128 + 1) / 2;
   const int K128 = cdv(K, 128) * 128;
-  // The chunk is both the split-K unit and the scale block: short chunks
+  // The chunk is the scale block, and the longest split-K unit: short chunks
   // keep each chunk's exponent close to its own coefficients (the envelope
   // falls steeply with |G|), and the int32 sums stay exact below the cap.
   long cap = (dt == DT_I8) ? (2147483647L / level_bound(S)) : (1L << 30);
@@ -1337,8 +1338,9 @@ int chunk_len(int dt, int S, int n, int K) {
   return max(128, kchunk / 128 * 128);
 }
 
-// Parts of a chunk in the split-K products over ntiles 128-tiles (any tile
-// shape and launch form: the parts decide the rounding of S).  32 CUs of an XCD
+// Parts of a chunk in the split-K products over ntiles 128-tiles.  They decide
+// the rounding of S, so they are the same for any tile shape and launch form,
+// digit type, and adaptive or uniform counts.  32 CUs of an XCD
 // each take one item at a time, so a count that fills them a little over once
 // leaves most idle half of the time.  The cost of a depth: rounds of items, each
 // of stages at 0.35 us and 0.061 us per level product (measured at 10 and 15
@@ -1349,9 +1351,9 @@ int chunk_len(int dt, int S, int n, int K) {
 // 2624, 2630, 2658 / 64, 123, 178, 233.  (One workgroup per item, as they come
 // free, against resident workgroups with fixed shares: 249 -> 237 us at 512,
 // 598 -> 564 at 777.)
-int chunk_parts(int dt, int S, bool adaptive, int ntiles, int nz, int kchunk) {
-  const int stages = kchunk / (dt == DT_I8 ? 32 : (dt == DT_F32 ? 8 : 16));
-  const int lv = adaptive && S > 3 ? S - 2 : S;  // most chunks drop slices
+int chunk_parts(int S, int ntiles, int nz, int kchunk) {
+  const int stages = kchunk / DBK;       // of int8 digits
+  const int lv = S > 3 ? S - 2 : S;      // adaptive: most chunks drop slices
   const double stage_us = 0.35 + lv * (lv + 1) / 2 * 0.061;
   int best = 1;
   double best_cost = 0.0;
@@ -1392,7 +1394,7 @@ oa_split_plan make_plan(int prec, int n, int K, int tile) {
   pl.nz = cdv(pl.Kp, pl.kchunk);
   pl.adaptive = (prec & OA_PREC_ADAPTIVE) ? 1 : 0;
   const int T128 = cdv(n, 128);
-  pl.nsub = chunk_parts(pl.dt, pl.S, pl.adaptive != 0, T128 * (T128 + 1) / 2, pl.nz, pl.kchunk);
+  pl.nsub = chunk_parts(pl.S, T128 * (T128 + 1) / 2, pl.nz, pl.kchunk);
   pl.ksub = cdv(cdv(pl.kchunk, pl.nsub), DBK) * DBK;
   size_t off = 0;
   auto take = [&](size_t bytes) {

@@ -143,7 +143,7 @@ int oa_create(oa_handle_t *out, int device) {
   c->device = device;
   if (hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&c->report, sizeof(oa_ns_report)) != hipSuccess ||
-      hipHostMalloc(&c->host_report, sizeof(oa_ns_report), hipHostMallocDefault) != hipSuccess) {
+      hipHostMalloc(&c->host, sizeof(oa_ns_host), hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     oa_destroy(c);
     return OA_ERR_HIP;
@@ -166,7 +166,7 @@ int oa_destroy(oa_handle_t c) {
   if (c->ws.ptr) (void)hipFree(c->ws.ptr);
   if (c->ns.ptr) (void)hipFree(c->ns.ptr);
   if (c->report) (void)hipFree(c->report);
-  if (c->host_report) (void)hipHostFree(c->host_report);
+  if (c->host) (void)hipHostFree(c->host);
   if (c->pinned.ptr) (void)hipHostFree(c->pinned.ptr);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   if (tl_default == c) tl_default = nullptr;
@@ -446,55 +446,74 @@ int oa_lambda(oa_handle_t c, int n, int npw, const double *psi, long ldpsi, cons
 
 }  // extern "C"
 
-// Waits until the report of iteration `upto`, or the last one, has reached the
-// handle's pinned mirror (pad = 2 * iteration + done, stored last), while the
-// stream runs on: a stream synchronisation per look left the device idle for
-// 15 to 25 us (the step at n = 128 took 111 us, of which 85 on the device).
-int oa_ns_wait(oa_context *c, int upto) {
+// Spins until done(), with looks at the stream in between: once it is idle or
+// has failed, no kernel can make done() true any more.
+template <class Done>
+static int ns_poll(oa_context *c, Done done) {
   for (unsigned spin = 1;; spin++) {
-    const int w = __atomic_load_n(&c->host_report->pad, __ATOMIC_ACQUIRE);
-    if ((w & 1) || (w >> 1) >= upto) return OA_SUCCESS;
+    if (done()) return OA_SUCCESS;
     __builtin_ia32_pause();
     if (spin % 4096 == 0) {
-      // an idle or failed stream writes no more reports
       const hipError_t e = hipStreamQuery(c->stream);
       if (e == hipErrorNotReady) continue;
       OA_HIP_CHECK(e);
-      const int v = __atomic_load_n(&c->host_report->pad, __ATOMIC_ACQUIRE);
-      return (v & 1) || (v >> 1) >= upto ? OA_SUCCESS : OA_ERR_HIP;
+      return done() ? OA_SUCCESS : OA_ERR_HIP;
     }
   }
 }
 
-int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
-                   double *T, int *iters, double *err, void *ws, oa_ns_report *rep, bool z,
-                   int modulus) {
-  oa_ns_args a;
-  oa_ns_fill(n, S, nspin, tol, maxit, T, rep, c->host_report, ws, &a, z, modulus);
-  *c->host_report = oa_ns_report{};
+// Waits until the report of iteration `upto`, or the last one, has reached the
+// handle's pinned memory (pad = 2 * iteration + done, stored last), while the
+// stream runs on: a stream synchronisation per look left the device idle for
+// 15 to 25 us (the step at n = 128 took 111 us, of which 85 on the device).
+static int ns_wait(oa_context *c, int upto) {
+  return ns_poll(c, [=] {
+    const int w = __atomic_load_n(&c->host->rep.pad, __ATOMIC_ACQUIRE);
+    return (w & 1) || (w >> 1) >= upto;
+  });
+}
+
+int oa_ns_drain(oa_context *c) {
+  return ns_poll(c, [=] { return __atomic_load_n(&c->host->drained, __ATOMIC_ACQUIRE) != 0; });
+}
+
+static int ns_sync_loop(oa_context *c, const oa_ns_args &a) {
   int st = oa_ns_begin(c->stream, a);
-  if (st == OA_SUCCESS && maxit > 1) st = oa_ns_check(c->stream, a, 1);
+  if (st == OA_SUCCESS && a.maxit > 1) st = oa_ns_check(c->stream, a, 1);
   if (st) return st;
   // One iteration is always enqueued beyond the one the host waits for, so the
   // device never waits for the host; states a step away from orthonormal take
   // three or four, so four go in at once.
   int enq = 1;  // iterations enqueued with their checks
-  while (enq < maxit) {
+  while (enq < a.maxit) {
     if (enq >= 4) {
-      st = oa_ns_wait(c, enq - 1);
+      st = ns_wait(c, enq - 1);
       if (st) return st;
-      if (c->host_report->pad & 1) break;
+      if (c->host->rep.pad & 1) break;
     }
     st = oa_ns_iterate(c->stream, a, enq);
     if (st == OA_SUCCESS) st = oa_ns_check(c->stream, a, enq + 1);
     if (st) return st;
     enq++;
   }
-  st = oa_ns_wait(c, enq);
-  if (st) return st;
-  if (iters) *iters = c->host_report->iterations;
-  if (err) *err = c->host_report->error;
-  return c->host_report->done ? c->host_report->status : OA_ERR_NOT_CONVERGED;
+  st = ns_wait(c, enq);
+  return st ? st : oa_ns_mark(c->stream, &c->host->drained);
+}
+
+int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
+                   double *T, int *iters, double *err, void *ws, oa_ns_report *rep, bool z,
+                   int modulus) {
+  oa_ns_args a;
+  oa_ns_fill(n, S, nspin, tol, maxit, T, rep, &c->host->rep, ws, &a, z, modulus);
+  *c->host = oa_ns_host{};
+  const int st = ns_sync_loop(c, a);
+  if (st) {
+    (void)hipStreamSynchronize(c->stream);  // what was enqueued ends here
+    return st;
+  }
+  if (iters) *iters = c->host->rep.iterations;
+  if (err) *err = c->host->rep.error;
+  return c->host->rep.done ? c->host->rep.status : OA_ERR_NOT_CONVERGED;
 }
 
 extern "C" {
@@ -647,7 +666,8 @@ int oa_ortho_step(oa_handle_t c, int n, int npw, const double *psi, long ldpsi, 
                                      c->report);
     if (st_ns != OA_SUCCESS && st_ns != OA_ERR_NOT_CONVERGED) return st_ns;
     st = oa_backmul(c, n, npw, T, 0, psi, ldpsi, 1.0, 0.0, psi_out, ldout, bprec);
-    return st ? st : st_ns;
+    const int st_dr = oa_ns_drain(c);
+    return st ? st : (st_dr ? st_dr : st_ns);
   }
   st = oa_launch_s_to_t(c->stream, n, S, nspin, tol, maxit, T, c->report, c->ns.ptr);
   if (st) return st;

@@ -1099,6 +1099,11 @@ __global__ __launch_bounds__(NT) void ns_init_kernel(oa_ns_args a) {
   ns_init_body<Z>(a, blockIdx.x, gridDim.x, red);
 }
 
+// A launch starts when the ones before it on the stream have ended.
+__global__ void ns_mark_kernel(int *flag) {
+  __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <class C, bool Z>
 __global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
 void ns_gemm_kernel(oa_ns_args a, int mode, int it, int npart) {
@@ -1548,6 +1553,11 @@ int oa_ns_check(hipStream_t s, const oa_ns_args &a, int it) { return launch_ns(s
 
 int oa_ns_iterate(hipStream_t s, const oa_ns_args &a, int it) {
   return launch_ns(s, a, NS_PAIR, it);
+}
+
+int oa_ns_mark(hipStream_t s, int *flag) {
+  hipLaunchKernelGGL(ns_mark_kernel, dim3(1), dim3(1), 0, s, flag);
+  return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
 
 int oa_launch_s_to_t(hipStream_t s, int n, const double *S, int nspin, double tol, int maxit,

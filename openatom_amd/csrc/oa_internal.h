@@ -34,6 +34,12 @@ struct oa_digit_tag {
   int n = 0, K = 0, prec = 0;
 };
 
+// Pinned host memory the S->T kernels write to and the host polls.
+struct oa_ns_host {
+  oa_ns_report rep;  // the latest report
+  int drained;       // 1: nothing of the call's S->T is left on the device
+};
+
 struct oa_context {
   int device = 0;
   hipStream_t own_stream = nullptr;
@@ -41,7 +47,7 @@ struct oa_context {
   oa_workspace ws;          // split-K partials and digit slices
   oa_workspace ns;          // S->T ping-pong buffers (kept apart so digits survive)
   oa_ns_report *report = nullptr;  // device report for synchronous S->T
-  oa_ns_report *host_report = nullptr;  // pinned mirror
+  oa_ns_host *host = nullptr;      // pinned
   oa_digit_tag digits;      // contents of ws's digit area
   oa_workspace pinned;      // pinned host staging of the transport calls
 };
@@ -53,16 +59,19 @@ int oa_ws_require(oa_context *c, size_t bytes);
 int oa_noalloc_init(int device);
 
 // S->T on the handle's stream with the buffers at ws (oa_ns_ws_bytes(n)) and
-// the device report rep; returns when the loop's outcome is known (iterations
-// that do nothing may still be enqueued, and T is complete for later work on
-// the stream).  The kernels write every report to the handle's pinned mirror
-// too, where the host waits for it.
+// the device report rep; returns when the loop's outcome is known.  Iterations
+// that do nothing may still be enqueued then; they read rep and the buffers,
+// which the next S->T on the handle (or, of the no-alloc step, on the device)
+// writes, on whatever stream that runs.  So every caller enqueues what needs T
+// and then waits with oa_ns_drain (or for the stream) before it returns.  The
+// kernels write every report to the handle's pinned memory too, where the host
+// waits for it.
 int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
                    double *T, int *iters, double *err, void *ws, oa_ns_report *rep,
                    bool z = false, int modulus = 0);
 
-// Waits for the report of iteration `upto` (or the last one) in the mirror.
-int oa_ns_wait(oa_context *c, int upto);
+// Waits until nothing of the last oa_s_to_t_sync is left on the device.
+int oa_ns_drain(oa_context *c);
 
 // Makes the handle's device current for the scope of an API call and
 // restores the caller's device afterwards.
@@ -169,6 +178,8 @@ void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double
 int oa_ns_begin(hipStream_t s, const oa_ns_args &a);
 int oa_ns_check(hipStream_t s, const oa_ns_args &a, int it);
 int oa_ns_iterate(hipStream_t s, const oa_ns_args &a, int it);
+// Stores 1 to *flag (pinned host memory) once the work enqueued so far is done.
+int oa_ns_mark(hipStream_t s, int *flag);
 int oa_launch_s_to_t(hipStream_t s, int n, const double *S, int nspin,
                      double tol, int maxit, double *T, oa_ns_report *report,
                      void *ws);

@@ -348,7 +348,8 @@ int oa_zortho_step(oa_handle_t c, int n, int npw, const double *psi, long ldpsi,
   // buffers of its own), from which the back-multiply makes J psi's
   st = zbackward(c->stream, n, npw, T, 0, psi, ldpsi, 1.0, 0.0, psi_out, ldout, ws, c->ws.bytes,
                  prec, is_split(prec));
-  return st ? st : st_ns;
+  const int st_dr = oa_ns_drain(c);
+  return st ? st : (st_dr ? st_dr : st_ns);
 }
 
 }  // extern "C"

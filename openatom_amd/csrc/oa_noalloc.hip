@@ -105,7 +105,8 @@ int oa_ortho_step_noalloc(oa_handle_t c, int n, int npw, const double *psi, long
     const int st_ns = oa_s_to_t_sync(c, n, S, nspin, tol, maxit, T, iters, err, ns, rep);
     if (st_ns != OA_SUCCESS && st_ns != OA_ERR_NOT_CONVERGED) return st_ns;
     st = oa_launch_gemm_f64(c->stream, false, false, &p, 1, nullptr);
-    return st ? st : st_ns;
+    const int st_dr = oa_ns_drain(c);
+    return st ? st : (st_dr ? st_dr : st_ns);
   }
   st = oa_launch_s_to_t(c->stream, n, S, nspin, tol, maxit, T, rep, ns);
   if (st) return st;

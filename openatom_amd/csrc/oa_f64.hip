@@ -507,11 +507,11 @@ __device__ __forceinline__ ProbRegs pick_problem(const oa_gemm_problem &p0,
 }
 
 struct NoEpi {
-  __device__ __forceinline__ void operator()(int, int, double) const {}
+  __device__ __forceinline__ double operator()(int, int, double x) const { return x; }
 };
 
 // One BM x BN output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I (the
-// product by SEG); epi(m, n, value) sees every output stored.
+// product by SEG); epi(m, n, value) returns what is stored for each output.
 template <bool TX, bool TY, class C, Seg SEG, class Epi>
 __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double *smem,
                                           Epi &&epi) {
@@ -573,16 +573,15 @@ __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double
               o[0] = fma(al, acc[i * WN + j][v], fma(beta, old[0], d));
               o[1] = fma(al1, acc[i * WN + jo][v], fma(beta, old[1], d1));
             }
+            o[0] = epi(m, n, o[0]);
+            o[1] = epi(m, n + 1, o[1]);
             *reinterpret_cast<d2u *>(crow + n) = o;
-            epi(m, n, o[0]);
-            epi(m, n + 1, o[1]);
             continue;
           }
         }
         const double o = (beta == 0.0) ? fma(al, acc[i * WN + j][v], d)
                                        : fma(al, acc[i * WN + j][v], fma(beta, crow[n], d));
-        crow[n] = o;
-        epi(m, n, o);
+        crow[n] = epi(m, n, o);
       }
     }
 }
@@ -1080,12 +1079,16 @@ __device__ __forceinline__ void ns_gemm_body(const oa_ns_args &a, int mode, int 
   const double *old = part ? Y + im : Y;
   double s = 0.0;
   gemm_body<false, false, C, Z ? SEG_TWO : SEG_ONE>(P, logical, smem, [&](int m, int n, double x) {
+    // the padding stays zero whatever the matrix holds: an infinity of a
+    // diverging iterate times the zeros of the other operand's padding is NaN,
+    // which the next product would carry into the matrix
+    if (m >= a.n || n >= a.n) return 0.0;
     if (res) {
       const double d = old[(long)m * a.np + n] - x;
       s += d * d;
-      if (m < a.n && n < a.n)
-        a.T[Z ? 2 * ((long)m * a.n + n) + part : (long)m * a.n + n] = x;
+      a.T[Z ? 2 * ((long)m * a.n + n) + part : (long)m * a.n + n] = x;
     }
+    return x;
   });
   if (res) {
     s = block_sum(s, smem);

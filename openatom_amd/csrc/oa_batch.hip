@@ -415,6 +415,13 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
     const InstPlan &p = b->ip[i];
     oa_ns_fill(p.n, p.S, p.nspin, p.tol, p.maxit, p.T, drep + i, nullptr, p.ns_ws, &na[i]);
   }
+  std::vector<Range> s_at, t_at;
+  for (const InstPlan &p : b->ip) {
+    s_at.emplace_back(p.S, p.n, p.n, p.n);
+    t_at.emplace_back(p.T, p.n, p.n, p.n);
+  }
+  for (int i = 0; i < count; i++)
+    for (int j = 0; j < count; j++) na[i].late |= j != i && t_at[i].meets(s_at[j]);
   auto ns_args = [&](const InstPlan &, int i) { return na[i]; };
   add_group<oa_ns_args>(
       blob, b->seq, LK_NS, OA_NS_INIT, 0, b->ip, ns_args,

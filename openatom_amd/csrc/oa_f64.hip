@@ -889,7 +889,8 @@ __global__ void fill_u64_kernel(unsigned long long *p, unsigned long long v, int
 // its products (n = 128: 3 x 4 MFLOP), so its launches are few:
 //   INIT  B = S/2 or S.  A = I makes the first iteration elementwise:
 //         C = 3I - B, A' = C/2, with the residual of A' - I.
-//   B1    B' = B C / 2.
+//   B1    B' = B C / 2; T = A' where INIT must not store it (`late`: T shares
+//         memory with an S that other threads still read).
 //   C     C = 3I - A B.
 //   PAIR  B' and A' side by side; A' tiles also sum (A - A')^2 and store T.
 // A residual left as partial sums by INIT or PAIR is added up by every
@@ -934,13 +935,15 @@ __device__ __forceinline__ void ns_init_body(const oa_ns_args &a, int w, int nwg
       if (Z) {
         bi = half * a.S[2 * k + 1];
         xi = -0.5 * bi;
-        a.T[2 * k] = x;
-        a.T[2 * k + 1] = xi;
+        if (!a.late) {
+          a.T[2 * k] = x;
+          a.T[2 * k + 1] = xi;
+        }
         const bool ok = isfinite(d) && isfinite(xi);
         s += ok ? d * d : nan;
         si += ok ? xi * xi : nan;
       } else {
-        a.T[k] = x;
+        if (!a.late) a.T[k] = x;
         s += (isfinite(d) || n == 1) ? d * d : nan;
       }
     }
@@ -1028,19 +1031,23 @@ __device__ __forceinline__ void ns_gemm_body(const oa_ns_args &a, int mode, int 
   if (mode == NS_B1 || (mode == NS_C && it >= 2)) {
     double err;
     const bool done = ns_update<Z>(a, it, npart, logical == 0 && which == 0, smem, err);
-    if (mode == NS_B1 && isnan(err)) {
+    if (mode == NS_B1) {
       // S's identity product with a non-finite S is NaN everywhere (a complex
-      // residual may also be NaN by its rule: then T stands)
-      bool bad = !Z;
-      if (Z) {
+      // residual may also be NaN by its rule: then A' stands)
+      bool bad = isnan(err);
+      if (Z && bad) {
         double s = 0.0;
         for (int i = threadIdx.x; i < npart; i += blockDim.x) s += a.partial[i];
         bad = isnan(block_sum(s, smem));
       }
+      const double *x = a.A[1] + (part ? a.zs : 0);
+      const bool put = bad || a.late;
       const int m0 = (logical % t) * C::BM, n0 = (logical / t) * C::BN;
-      for (int e = threadIdx.x; bad && e < C::BM * C::BN; e += C::NTHR) {
+      for (int e = threadIdx.x; put && e < C::BM * C::BN; e += C::NTHR) {
         const int m = m0 + e / C::BN, n = n0 + e % C::BN;
-        if (m < a.n && n < a.n) a.T[Z ? 2 * ((long)m * a.n + n) + part : (long)m * a.n + n] = err;
+        if (m < a.n && n < a.n)
+          a.T[Z ? 2 * ((long)m * a.n + n) + part : (long)m * a.n + n] =
+              bad ? err : x[(long)m * a.np + n];
       }
     }
     if (done) return;
@@ -1516,6 +1523,9 @@ void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double
   a->T = T;
   a->rep = rep;
   a->mirror = mirror;
+  const uintptr_t s0 = (uintptr_t)S, t0 = (uintptr_t)T,
+                  len = (uintptr_t)(z ? 2 : 1) * n * n * sizeof(double);
+  a->late = s0 != t0 && s0 < t0 + len && t0 < s0 + len;
   a->zs = z ? nn / 2 : 0;
   a->modulus = modulus;
 }

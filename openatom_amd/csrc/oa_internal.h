@@ -170,6 +170,9 @@ struct oa_ns_args {
   oa_ns_report *rep, *mirror;
   long zs;      // complex S and T: elements from a buffer's real to its imaginary plane
   int modulus;  // complex: stop on sum |dA|^2 instead of Re sum (dA)^2
+  // T shares memory with an S it is not equal to (its own, or in a joint launch
+  // another instance's): stored after every S has been read
+  int late;
 };
 size_t oa_ns_ws_bytes(int n, bool z = false);
 void oa_ns_fill(int n, const double *S, int nspin, double tol, int maxit, double *T,

@@ -124,9 +124,9 @@ int oa_launch_zgemm(hipStream_t s, char ta, char tb, int m, int n, int k, const 
   };
   const oa_gemm_problem p1[2] = {prob(Ar, Br, P), prob(Ar, Bi, P + 2 * mn)};
   const oa_gemm_problem p2[2] = {prob(Ai, Bi, P + mn), prob(Ai, Br, P + 3 * mn)};
-  int st = oa_launch_gemm_f64(s, !notb, !nota, p1, 2, nullptr);
+  int st = oa_launch_gemm_f64(s, !notb, !nota, p1, 2);
   if (st) return st;
-  st = oa_launch_gemm_f64(s, !notb, !nota, p2, 2, nullptr);
+  st = oa_launch_gemm_f64(s, !notb, !nota, p2, 2);
   if (st) return st;
   hipLaunchKernelGGL(zcombine_kernel, dim3(blocks_for((long)mn)), dim3(256), 0, s, m, n,
                      (const double *)P, ar, ai, br, bi, C, (long)ldc);

@@ -588,8 +588,9 @@ __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double
 
 template <bool TX, bool TY, class C>
 __global__ __launch_bounds__(C::NTHR) __attribute__((amdgpu_waves_per_eu(C::WPE, C::WPE)))
-void gemm_f64_kernel(oa_gemm_problem p0, oa_gemm_problem p1, const int32_t *skip) {
-  if (skip && *skip) return;
+void gemm_f64_kernel(oa_gemm_problem p0, oa_gemm_problem p1, int *mark) {
+  if (mark && blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(mark, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   const ProbRegs P = pick_problem(p0, p1);
   __shared__ __attribute__((aligned(1024))) double smem[C::SMEM];
   gemm_body<TX, TY, C, SEG_ONE>(P, xcd_logical(blockIdx.x, gridDim.x), smem, NoEpi{});
@@ -1197,7 +1198,7 @@ void with_tile(TilePick t, F &&f) {
 }
 
 template <bool TX, bool TY>
-int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_t *skip) {
+int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, int *mark) {
   auto tiles = [&](int bm, int bn) {
     long t = 0;
     for (int i = 0; i < nprob; i++) t = max(t, gemm_tiles(p[i], bm, bn));
@@ -1208,7 +1209,7 @@ int launch_gemm(hipStream_t s, const oa_gemm_problem *p, int nprob, const int32_
     typedef decltype(c) C;
     hipLaunchKernelGGL((gemm_f64_kernel<TX, TY, C>),
                        dim3((unsigned)((tiles(C::BM, C::BN) + 7) / 8 * 8), nprob),
-                       dim3(C::NTHR), 0, s, p[0], p[nprob > 1 ? 1 : 0], skip);
+                       dim3(C::NTHR), 0, s, p[0], p[nprob > 1 ? 1 : 0], mark);
   });
   return hipPeekAtLastError() == hipSuccess ? OA_SUCCESS : OA_ERR_HIP;
 }
@@ -1337,12 +1338,12 @@ int oa_launch_scale_cols(hipStream_t s, int rows, int ncols, double *X, long ld,
 }
 
 int oa_launch_gemm_f64(hipStream_t s, bool tx, bool ty, const oa_gemm_problem *p, int nprob,
-                       const int32_t *skip) {
+                       int *mark) {
   if (nprob < 1 || nprob > 2) return OA_ERR_UNSUPPORTED;
-  if (!tx && !ty) return launch_gemm<false, false>(s, p, nprob, skip);
-  if (!tx && ty) return launch_gemm<false, true>(s, p, nprob, skip);
-  if (tx && !ty) return launch_gemm<true, false>(s, p, nprob, skip);
-  return launch_gemm<true, true>(s, p, nprob, skip);
+  if (!tx && !ty) return launch_gemm<false, false>(s, p, nprob, mark);
+  if (!tx && ty) return launch_gemm<false, true>(s, p, nprob, mark);
+  if (tx && !ty) return launch_gemm<true, false>(s, p, nprob, mark);
+  return launch_gemm<true, true>(s, p, nprob, mark);
 }
 
 int oa_launch_zback_f64(hipStream_t s, bool tx, int n, int K, const double *Mr, const double *Mi,

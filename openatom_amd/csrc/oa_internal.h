@@ -63,15 +63,20 @@ int oa_noalloc_init(int device);
 // that do nothing may still be enqueued then; they read rep and the buffers,
 // which the next S->T on the handle (or, of the no-alloc step, on the device)
 // writes, on whatever stream that runs.  So every caller enqueues what needs T
-// and then waits with oa_ns_drain (or for the stream) before it returns.  The
-// kernels write every report to the handle's pinned memory too, where the host
-// waits for it.
+// and something that sets c->host->drained (that launch itself, or oa_ns_mark
+// before it), and waits with oa_ns_drain before it returns; or it waits for the
+// stream.  The kernels write every report to the handle's pinned memory too,
+// where the host waits for it.
 int oa_s_to_t_sync(oa_context *c, int n, const double *S, int nspin, double tol, int maxit,
                    double *T, int *iters, double *err, void *ws, oa_ns_report *rep,
                    bool z = false, int modulus = 0);
 
 // Waits until nothing of the last oa_s_to_t_sync is left on the device.
 int oa_ns_drain(oa_context *c);
+
+// out = T psi in FP64 on the handle's stream; mark as in oa_launch_gemm_f64.
+int oa_tpsi_f64(oa_context *c, int n, int npw, const double *T, const double *psi, long ldpsi,
+                double *out, long ldout, int *mark);
 
 // Makes the handle's device current for the scope of an API call and
 // restores the caller's device afterwards.
@@ -110,10 +115,10 @@ struct oa_gemm_problem {
 };
 
 // Launch one or two independent problems of the same shape class in one grid
-// (grid.y selects the problem).  `skip` (device int, may be null) turns the
-// launch into a no-op when nonzero (used by guarded S->T iterations).
+// (grid.y selects the problem).  `mark` (pinned host memory, may be null)
+// receives 1 as the launch starts, so once the work before it is done.
 int oa_launch_gemm_f64(hipStream_t s, bool tx, bool ty, const oa_gemm_problem *p,
-                       int nprob, const int32_t *skip);
+                       int nprob, int *mark = nullptr);
 
 // Symmetric overlap, FP64 MFMA, upper-triangle tiles, split-K.
 // S (row-major n x n, full) = alpha * sum_k w_k psi[x][k] psi[y][k] with

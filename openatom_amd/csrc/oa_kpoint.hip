@@ -346,8 +346,10 @@ int oa_zortho_step(oa_handle_t c, int n, int npw, const double *psi, long ldpsi,
   if (st_ns != OA_SUCCESS && st_ns != OA_ERR_NOT_CONVERGED) return st_ns;
   // a split forward left psi's digits in the kernel workspace (S->T has
   // buffers of its own), from which the back-multiply makes J psi's
-  st = zbackward(c->stream, n, npw, T, 0, psi, ldpsi, 1.0, 0.0, psi_out, ldout, ws, c->ws.bytes,
-                 prec, is_split(prec));
+  st = oa_ns_mark(c->stream, &c->host->drained);
+  if (st == OA_SUCCESS)
+    st = zbackward(c->stream, n, npw, T, 0, psi, ldpsi, 1.0, 0.0, psi_out, ldout, ws, c->ws.bytes,
+                   prec, is_split(prec));
   const int st_dr = oa_ns_drain(c);
   return st ? st : (st_dr ? st_dr : st_ns);
 }

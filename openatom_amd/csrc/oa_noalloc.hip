@@ -88,29 +88,16 @@ int oa_ortho_step_noalloc(oa_handle_t c, int n, int npw, const double *psi, long
   int st = oa_launch_overlap_f64_fit(c->stream, n, K, psi, ldpsi, 2 * nkx0, 2.0, S, 0.0,
                                      nullptr, part, part_bytes);
   if (st) return st;
-  oa_gemm_problem p{};
-  p.M = n;
-  p.N = K;
-  p.K = n;
-  p.X = T;
-  p.ldx = n;
-  p.Y = psi;
-  p.ldy = ldpsi;
-  p.C = psi_out;
-  p.ldc = ldout;
-  p.alpha = 1.0;
-  p.beta = 0.0;
-  p.diag_add = 0.0;
   if (iters || err) {
     const int st_ns = oa_s_to_t_sync(c, n, S, nspin, tol, maxit, T, iters, err, ns, rep);
     if (st_ns != OA_SUCCESS && st_ns != OA_ERR_NOT_CONVERGED) return st_ns;
-    st = oa_launch_gemm_f64(c->stream, false, false, &p, 1, nullptr);
+    st = oa_tpsi_f64(c, n, npw, T, psi, ldpsi, psi_out, ldout, &c->host->drained);
     const int st_dr = oa_ns_drain(c);
     return st ? st : (st_dr ? st_dr : st_ns);
   }
   st = oa_launch_s_to_t(c->stream, n, S, nspin, tol, maxit, T, rep, ns);
   if (st) return st;
-  return oa_launch_gemm_f64(c->stream, false, false, &p, 1, nullptr);
+  return oa_tpsi_f64(c, n, npw, T, psi, ldpsi, psi_out, ldout, nullptr);
 }
 
 }  // extern "C"

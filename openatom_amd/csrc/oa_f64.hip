@@ -1000,13 +1000,15 @@ __device__ __forceinline__ bool ns_update(const oa_ns_args &a, int it, int npart
     *a.rep = r;
     if (a.mirror) {
       // host memory; `pad` is the word the host polls, stored when the rest
-      // has arrived
+      // has arrived.  (A release at system scope would write back the whole L2;
+      // these stores go through it, so waiting for them is enough, and the
+      // clobber keeps the compiler from moving them.)
       __hip_atomic_store(&a.mirror->error, err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       __hip_atomic_store(&a.mirror->status, r.status, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_SYSTEM);
       __hip_atomic_store(&a.mirror->done, r.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       __hip_atomic_store(&a.mirror->iterations, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      wait_vm<0>();
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __hip_atomic_store(&a.mirror->pad, 2 * it + r.done, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_SYSTEM);
     }

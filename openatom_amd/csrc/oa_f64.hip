@@ -507,11 +507,12 @@ __device__ __forceinline__ ProbRegs pick_problem(const oa_gemm_problem &p0,
 }
 
 struct NoEpi {
-  __device__ __forceinline__ double operator()(int, int, double x) const { return x; }
+  __device__ __forceinline__ double operator()(int, int, int, double x) const { return x; }
 };
 
 // One BM x BN output tile `logical` of C = alpha*op(X)*op(Y) + beta*C + d*I (the
-// product by SEG); epi(m, n, value) returns what is stored for each output.
+// product by SEG); epi(b, m, n, value) returns what is stored for
+// each output, of the wave's block b = i * WN + j.
 template <bool TX, bool TY, class C, Seg SEG, class Epi>
 __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double *smem,
                                           Epi &&epi) {
@@ -573,15 +574,15 @@ __device__ __forceinline__ void gemm_body(const ProbRegs &P, int logical, double
               o[0] = fma(al, acc[i * WN + j][v], fma(beta, old[0], d));
               o[1] = fma(al1, acc[i * WN + jo][v], fma(beta, old[1], d1));
             }
-            o[0] = epi(m, n, o[0]);
-            o[1] = epi(m, n + 1, o[1]);
+            o[0] = epi(i * WN + j, m, n, o[0]);
+            o[1] = epi(i * WN + jo, m, n + 1, o[1]);
             *reinterpret_cast<d2u *>(crow + n) = o;
             continue;
           }
         }
         const double o = (beta == 0.0) ? fma(al, acc[i * WN + j][v], d)
                                        : fma(al, acc[i * WN + j][v], fma(beta, crow[n], d));
-        crow[n] = epi(m, n, o);
+        crow[n] = epi(i * WN + j, m, n, o);
       }
     }
 }
@@ -896,7 +897,9 @@ __global__ void fill_u64_kernel(unsigned long long *p, unsigned long long v, int
 //   PAIR  B' and A' side by side; A' tiles also sum (A - A')^2 and store T.
 // A residual left as partial sums by INIT or PAIR is added up by every
 // workgroup of the next launch (B1 or C), each of which then knows by itself
-// whether the loop has ended; the first one writes the report.  T holds the
+// whether the loop has ended; the first one writes the report.  The sums run in
+// one order whatever the tiles of either launch (PAIR leaves one per 32 x 32
+// block, added up by 256 threads), so all launch forms end alike.  T holds the
 // latest iterate throughout.  Before: four launches an iteration, of which a
 // one-thread sum of 128 partials took 5 to 9 us, and a final copy to T.
 enum NsMode { NS_B1 = 0, NS_C = 1, NS_PAIR = 2 };
@@ -941,11 +944,11 @@ __device__ __forceinline__ void ns_init_body(const oa_ns_args &a, int w, int nwg
           a.T[2 * k + 1] = xi;
         }
         const bool ok = isfinite(d) && isfinite(xi);
-        s += ok ? d * d : nan;
-        si += ok ? xi * xi : nan;
+        s = ok ? fma(d, d, s) : nan;
+        si = ok ? fma(xi, xi, si) : nan;
       } else {
         if (!a.late) a.T[k] = x;
-        s += (isfinite(d) || n == 1) ? d * d : nan;
+        s = (isfinite(d) || n == 1) ? fma(d, d, s) : nan;
       }
     }
     a.B[0][idx] = b;
@@ -972,6 +975,15 @@ __device__ __forceinline__ void ns_init_body(const oa_ns_args &a, int w, int nwg
   }
 }
 
+// Sum of npart partial sums by the first 256 threads.
+__device__ __forceinline__ double partial_sum(const double *p, int npart, double *red) {
+  double s = 0.0;
+  if (threadIdx.x < NT)
+#pragma unroll 4
+    for (int i = threadIdx.x; i < npart; i += NT) s += p[i];
+  return block_sum(s, red);
+}
+
 // Residual of the iteration `it` (1-based) from its npart partial sums (Z: of
 // either part); returns whether the loop ends there.  `writer` stores the
 // report.  The complex rule is the reference's Re sum (dA)^2, NaN where that is
@@ -979,13 +991,9 @@ __device__ __forceinline__ void ns_init_body(const oa_ns_args &a, int w, int nwg
 template <bool Z>
 __device__ __forceinline__ bool ns_update(const oa_ns_args &a, int it, int npart, bool writer,
                                           double *red, double &err) {
-  double s = 0.0;
-  for (int i = threadIdx.x; i < npart; i += blockDim.x) s += a.partial[i];
-  s = block_sum(s, red);
+  double s = partial_sum(a.partial, npart, red);
   if (Z) {
-    double si = 0.0;
-    for (int i = threadIdx.x; i < npart; i += blockDim.x) si += a.partial[npart + i];
-    si = block_sum(si, red);
+    const double si = partial_sum(a.partial + npart, npart, red);
     s = a.modulus ? s + si : s - si;
   }
   err = sqrt(s / ((double)a.n * (double)a.n));
@@ -1016,6 +1024,47 @@ __device__ __forceinline__ bool ns_update(const oa_ns_args &a, int it, int npart
   return done;
 }
 
+// Blocks of 32 rows of an S->T matrix of np rows: their squares share a partial
+// sum of the residual.
+__host__ __device__ __forceinline__ int ns_blocks(int np) { return cdiv(np, 32); }
+
+// The partial sums of a tile's 32 x 32 blocks from the lanes' sums s[i * WN + j]
+// over their four elements of block (i, j).  One tree for every tile: column
+// pairs, eight columns each, the four row groups, the two halves of a 32 column
+// span, the two 16 row blocks.  (PAIR lanes hold adjacent columns, other
+// lanes one column of 16.)
+template <class C>
+__device__ __forceinline__ void ns_residual(const oa_ns_args &a, int part, int m0, int n0,
+                                            const double (&s)[C::WM * C::WN], double *red) {
+  constexpr bool PAIR = RowMap<C::WN, C::WC, false>::PAIR;
+  static_assert(PAIR ? C::WN == 2 : C::WN == 1, "one column span per wave");
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < C::WM; i++) {
+    double x = PAIR ? s[i * C::WN] + s[i * C::WN + C::WN - 1] : s[i];
+#pragma unroll
+    for (int o = 1; o <= (PAIR ? 4 : 8); o <<= 1) x += __shfl_xor(x, o);
+    x += __shfl_xor(x, 16);
+    x += __shfl_xor(x, 32);
+    if (PAIR) x += __shfl_xor(x, 8);
+    if (lane == 0) red[i * C::NW + w] = x;
+  }
+  __syncthreads();
+  const int t = threadIdx.x, nb = ns_blocks(a.np);
+  if (t < (C::BM / 32) * (C::BN / 32)) {
+    const int rb = t / (C::BN / 32), cb = t % (C::BN / 32);
+    // rows: block k = i * WR + wr of 16; columns: span wc, or the halves 2 cb, 2 cb + 1
+    auto row = [&](int k) {
+      const double *p = red + (k / C::WR) * C::NW + (k % C::WR) * C::WC;
+      return PAIR ? p[cb] : p[2 * cb] + p[2 * cb + 1];
+    };
+    const double x = row(2 * rb) + row(2 * rb + 1);
+    const int br = m0 / 32 + rb, bc = n0 / 32 + cb;
+    if (br < nb && bc < nb) a.partial[(part * nb + br) * nb + bc] = x;
+  }
+  __syncthreads();  // red may be refilled
+}
+
 // Output tile `logical` of an NS_B1, NS_C or NS_PAIR launch after `it` iterations.
 // `which` of the launch's products: 0 = B', 1 = A' of a pair; with Z the real
 // and the imaginary part of each in turn (four real products in two sums).
@@ -1038,11 +1087,7 @@ __device__ __forceinline__ void ns_gemm_body(const oa_ns_args &a, int mode, int 
       // S's identity product with a non-finite S is NaN everywhere (a complex
       // residual may also be NaN by its rule: then A' stands)
       bool bad = isnan(err);
-      if (Z && bad) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < npart; i += blockDim.x) s += a.partial[i];
-        bad = isnan(block_sum(s, smem));
-      }
+      if (Z && bad) bad = isnan(partial_sum(a.partial, npart, smem));
       const double *x = a.A[1] + (part ? a.zs : 0);
       const bool put = bad || a.late;
       const int m0 = (logical % t) * C::BM, n0 = (logical / t) * C::BN;
@@ -1087,23 +1132,22 @@ __device__ __forceinline__ void ns_gemm_body(const oa_ns_args &a, int mode, int 
   P.neg1 = part == 0;
   const bool res = mode == NS_PAIR && second;
   const double *old = part ? Y + im : Y;
-  double s = 0.0;
-  gemm_body<false, false, C, Z ? SEG_TWO : SEG_ONE>(P, logical, smem, [&](int m, int n, double x) {
+  double s[C::WM * C::WN] = {};
+  gemm_body<false, false, C, Z ? SEG_TWO : SEG_ONE>(P, logical, smem,
+                                                    [&](int b, int m, int n, double x) {
     // the padding stays zero whatever the matrix holds: an infinity of a
     // diverging iterate times the zeros of the other operand's padding is NaN,
     // which the next product would carry into the matrix
     if (m >= a.n || n >= a.n) return 0.0;
     if (res) {
       const double d = old[(long)m * a.np + n] - x;
-      s += d * d;
+      s[b] = fma(d, d, s[b]);
       a.T[Z ? 2 * ((long)m * a.n + n) + part : (long)m * a.n + n] = x;
     }
     return x;
   });
-  if (res) {
-    s = block_sum(s, smem);
-    if (threadIdx.x == 0) a.partial[part * t * t + logical] = s;
-  }
+  if (res)
+    ns_residual<C>(a, part, (logical % t) * C::BM, (logical / t) * C::BN, s, smem);
 }
 
 template <bool Z>
@@ -1145,7 +1189,8 @@ void ns_gemm_grouped(const oa_ns_args *__restrict__ t, const int *__restrict__ p
     const int i = group_find(prefix, count, item);
     const oa_ns_args &a = t[i];
     const int tiles = cdiv(a.np, C::BM) * cdiv(a.np, C::BM), k = item - prefix[i];
-    ns_gemm_body<C, false>(a, mode, it, mode == NS_B1 ? a.nwg : tiles, k / tiles, k % tiles,
+    const int nb = ns_blocks(a.np);
+    ns_gemm_body<C, false>(a, mode, it, mode == NS_B1 ? a.nwg : nb * nb, k / tiles, k % tiles,
                            smem);
   });
 }
@@ -1497,7 +1542,7 @@ static int ns_init_wg(int n) {
   return (int)(b > 256 ? 256 : b);
 }
 static size_t ns_partials(int n) {
-  const size_t t = (size_t)cdiv((int)ns_np(n), 32);
+  const size_t t = (size_t)ns_blocks((int)ns_np(n));
   return t * t > 256 ? t * t : 256;
 }
 
@@ -1542,8 +1587,7 @@ static int ns_tile(int np, int nprob) {
 
 static int launch_ns(hipStream_t s, const oa_ns_args &a, int mode, int it) {
   const int z = a.zs ? 2 : 1, nprob = z * (mode == NS_PAIR ? 2 : 1);
-  const int pt = cdiv(a.np, ns_tile(a.np, 2 * z));
-  const int npart = mode == NS_B1 ? a.nwg : pt * pt;
+  const int nb = ns_blocks(a.np), npart = mode == NS_B1 ? a.nwg : nb * nb;
   const int edge = ns_tile(a.np, nprob);
   with_tile(edge == 128 ? PICK_128 : (edge == 64 ? PICK_64W : PICK_32), [&](auto c) {
     typedef decltype(c) C;

@@ -335,13 +335,26 @@ __device__ __forceinline__ void count_switch(int v, F &&f) {
 
 // Runs mma(X panel, Y panel, first) over the stages of k in [ka, kb) of one
 // tile; with SEG over those of (X1, Y1) first.  YSAME: the Y panel is the X
-// panel (diagonal tile of a symmetric product), loaded once.
-template <class C, bool XKC, bool YKC, bool YSAME, Seg SEG = SEG_ONE, class Mma>
+// panel (diagonal tile of a symmetric product), loaded once.  KZ: the first kz
+// (even) columns are cleared in LDS, so that they add nothing, whatever they hold.
+template <class C, bool XKC, bool YKC, bool YSAME, Seg SEG = SEG_ONE, bool KZ = false, class Mma>
 __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mlim,
                                       const double *Y, long ldy, int n0, int nlim, int ka,
                                       int kb, double *smem, Mma &&mma,
-                                      const double *X1 = nullptr, const double *Y1 = nullptr) {
+                                      const double *X1 = nullptr, const double *Y1 = nullptr,
+                                      int kz = 0) {
   constexpr int NBUF = C::NBUF, G = C::GRP, YOFF = YSAME ? 0 : C::BM * BK;
+  static_assert(!KZ || (XKC && YKC && G == 1 && SEG == SEG_ONE), "panels as cleared below");
+  auto clear = [&](double *buf, int stage) {  // the two panels' rows lie one after another
+    constexpr int R = C::BM + (YSAME ? 0 : C::BN);
+    const int cols = min(BK, kz - stage * BK);
+    if (!KZ || cols <= 0) return;
+    for (int i = threadIdx.x; i < R * (cols / 2); i += C::NTHR) {
+      const int row = i % R, pair = i / R;
+      *reinterpret_cast<d2v *>(buf + row * BK + 2 * (pair ^ ((row >> 1) & 7))) = d2v{0.0, 0.0};
+    }
+    ring_barrier();
+  };
   constexpr bool TWO = SEG != SEG_ONE;
   typedef Panel<C::BM, XKC, C::NW> PX;
   typedef Panel<C::BN, YKC, C::NW> PY;
@@ -388,6 +401,7 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
       else wait_vm<0>();
       ring_barrier();
       next(s + NBUF - 1);
+      if (KZ) clear(smem + (s % NBUF) * C::STAGE, s);
       const double *cur = smem + (s % NBUF) * (G * C::STAGE);
 #pragma unroll
       for (int j = 0; j < G; j++)
@@ -445,6 +459,7 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
       wait_vm<0>();
       ring_barrier();
       if (s + 1 < total) load(s + 1);
+      if (KZ) clear(smem + (s & 1) * C::STAGE, s);
       const double *cur = smem + (s & 1) * C::STAGE;
       mma(cur, cur + YOFF, TWO && s < nfull);
       if (s + 1 < total) finish(s + 1);
@@ -459,6 +474,7 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
       PX::masked(TWO && !seg ? X1 : X, ldx, m0, mlim, k0, kb, smem, w, lane);
       if (!YSAME) PY::masked(TWO && !seg ? Y1 : Y, ldy, n0, nlim, k0, kb, smem + YOFF, w, lane);
       ring_barrier();
+      if (KZ) clear(smem, nfull);
       mma(smem, smem + YOFF, TWO && !seg);
     }
   }
@@ -705,14 +721,18 @@ __device__ __forceinline__ void ovl_body(const oa_ovl_args &a, int block, int nb
   const bool diag = SYM && bi == bj;
   const int nbr = min(BM / 16, cdiv(a.M - m0, 16)), nbc = min(BM / 16, cdiv(a.N - n0, 16));
   const int nblk = diag ? nbr * (nbr + 1) / 2 : nbr * nbc;
+  constexpr bool KZ = SYM && !YJ;
+  const int kz = KZ && ka == 0 ? a.kx0_add : 0;
   if (nblk == (BM / 16) * (BM / 16)) {
     d4 acc[WM * WN];
 #pragma unroll
     for (int i = 0; i < WM * WN; i++) acc[i] = d4{0, 0, 0, 0};
-    kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, a.Y, a.ldy, n0, a.N, ka, kb, smem,
-                                [&](const double *Xs, const double *Ys, bool) {
-                                  mma_rows<C, true, true, WM, YJ>(Xs, Ys, wr, wc, lane, acc);
-                                });
+    kloop<C, true, true, false, SEG_ONE, KZ>(
+        a.X, a.ldx, m0, a.M, a.Y, a.ldy, n0, a.N, ka, kb, smem,
+        [&](const double *Xs, const double *Ys, bool) {
+          mma_rows<C, true, true, WM, YJ>(Xs, Ys, wr, wc, lane, acc);
+        },
+        nullptr, nullptr, kz);
 #pragma unroll
     for (int i = 0; i < WM; i++)
 #pragma unroll
@@ -743,9 +763,11 @@ __device__ __forceinline__ void ovl_body(const oa_ovl_args &a, int block, int nb
       mma_list<NB, YJ>(Xs, Ys, xr, yr, lane, acc);
     };
     if (diag)
-      kloop<C, true, true, true>(a.X, a.ldx, m0, a.M, a.X, a.ldx, n0, a.N, ka, kb, smem, mma);
+      kloop<C, true, true, true, SEG_ONE, KZ>(a.X, a.ldx, m0, a.M, a.X, a.ldx, n0, a.N, ka, kb,
+                                              smem, mma, nullptr, nullptr, kz);
     else
-      kloop<C, true, true, false>(a.X, a.ldx, m0, a.M, a.Y, a.ldy, n0, a.N, ka, kb, smem, mma);
+      kloop<C, true, true, false, SEG_ONE, KZ>(a.X, a.ldx, m0, a.M, a.Y, a.ldy, n0, a.N, ka, kb,
+                                               smem, mma, nullptr, nullptr, kz);
 #pragma unroll
     for (int t = 0; t < NB; t++)
       if (w + C::NW * t < nblk)
@@ -768,8 +790,10 @@ void ovl_f64_kernel(oa_ovl_args a) {
 // over four uneven instances; this takes 6 and 20.)  The mirror tile is written
 // from LDS, 128 bytes a row.
 //   has_kx0: z = 0 holds the leading kx0 columns and counts half.
-//   kx0_sub: every z counts fully and half the product of the leading
-//            kx0_sub columns of psi is taken off here.
+//   kx0_add: the partial tiles leave out the leading kx0_add columns of psi;
+//            half their product is added here.  (Summed with the others and
+//            half taken off again, a state that lives on these columns lost a
+//            digit and an infinity in them became NaN.)
 template <int BM, bool SYM>
 __device__ __forceinline__ void ovl_reduce_body(const oa_ovl_args &a, int block,
                                                 double (&sums)[4][256], double (&out)[16][17]) {
@@ -806,8 +830,8 @@ __device__ __forceinline__ void ovl_reduce_body(const oa_ovl_args &a, int block,
     s = ((sums[0][t] + sums[1][t]) + sums[2][t]) + sums[3][t];
     if (in) {
       double g = 0.0;
-      for (int k = 0; k < a.kx0_sub; k++) g = fma(psi[(long)i * ld + k], psi[(long)j * ld + k], g);
-      s = a.alpha * fma(-0.5, g, s);
+      for (int k = 0; k < a.kx0_add; k++) g = fma(psi[(long)i * ld + k], psi[(long)j * ld + k], g);
+      s = a.alpha * fma(0.5, g, s);
       C[(long)i * ldc + j] = s;
     }
     out[lr][lc] = s;
@@ -1279,10 +1303,10 @@ struct OvlPlan {
   int kx0_slice;  // columns of a kx = 0 slice (z = 0), 0 for none
 };
 
-// A kx = 0 plane of at most this many columns is multiplied with the rest and
-// half its product taken off in the reduce; a wider one is a z slice of its
-// own, weighted there.
-constexpr int KX0_SUB_MAX = 32;
+// A kx = 0 plane of at most this many columns is cleared in the first chunk's
+// panels and half its product added in the reduce; a wider one is a z slice of
+// its own, weighted there.
+constexpr int KX0_ADD_MAX = 32;
 
 // Split depth nz for ntiles output tiles of BM over K columns, of which the
 // blocks inside the matrix (and above the diagonal) are the fraction `fill`.
@@ -1355,7 +1379,7 @@ OvlPlan plan_ovl(int M, int N, int K, int kx0_end, bool sym, size_t max_part_byt
   }
   // the chunk length comes from K: a slice never adds more than one z
   pl.kchunk = cdiv(cdiv(max(K, 1), nz), BK) * BK;
-  pl.kx0_slice = kx0_end > KX0_SUB_MAX ? kx0_end : 0;
+  pl.kx0_slice = kx0_end > KX0_ADD_MAX ? kx0_end : 0;
   pl.nz_main = max(1, cdiv(max(K - pl.kx0_slice, 1), pl.kchunk));
   pl.nz = pl.nz_main + (pl.kx0_slice > 0 ? 1 : 0);
   return pl;

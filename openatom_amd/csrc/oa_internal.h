@@ -323,7 +323,7 @@ struct oa_ovl_args {
   int nz_main, kchunk;
   double *part;         // [nz][ntiles][bm][bm]
   int bm, nz;
-  int kx0_sub;          // columns of X whose product is taken off by half
+  int kx0_add;          // leading columns left out of the partial tiles, added by half
   double alpha;
   double *C;
   long ldc;

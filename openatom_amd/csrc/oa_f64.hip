@@ -375,8 +375,14 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
   };
   if (dx && dy) {
     constexpr int PER = G * (PX::CH + (YSAME ? 0 : PY::CH));  // loads of a slot per wave
-    const int ngrp = nfull / G, rem = nfull % G;  // whole slots, then rem stages
-    const int total = TWO ? 2 * ngrp : ngrp;
+    // a product's whole slots, then rem stages: of a lone product after the loop,
+    // of two as one more slot of each, so that the first ends before the second
+    // begins in every tile
+    const int ngrp = nfull / G, rem = nfull % G;
+    const int per = TWO && rem > 0 ? ngrp + 1 : ngrp, total = TWO ? 2 * per : ngrp;
+    auto stages = [&](int s) {
+      return TWO && G > 1 && rem > 0 && (s == per - 1 || s == total - 1) ? rem : G;
+    };
     auto issue = [&](int s, int m) {
       double *buf = smem + (s % NBUF) * (G * C::STAGE);
 #pragma unroll
@@ -385,8 +391,8 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
     };
     auto next = [&](int s) {
       if (s < total) {
-        if (TWO && s == ngrp) start(false, ka);
-        issue(s, G);
+        if (TWO && s == per) start(false, ka);
+        issue(s, stages(s));
       } else if (!TWO && G > 1 && s == ngrp && rem > 0) {
         issue(s, rem);
       }
@@ -403,24 +409,22 @@ __device__ __forceinline__ void kloop(const double *X, long ldx, int m0, int mli
       next(s + NBUF - 1);
       if (KZ) clear(smem + (s % NBUF) * C::STAGE, s);
       const double *cur = smem + (s % NBUF) * (G * C::STAGE);
+      const int m = stages(s);
+      if (m == G) {
 #pragma unroll
-      for (int j = 0; j < G; j++)
-        mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF, TWO && s < ngrp);
-    }
-    if (G > 1 && rem > 0) {
-#pragma nounroll
-      for (int seg = TWO ? 0 : 1; seg < 2; seg++) {
-        if (TWO) {
-          ring_barrier();
-          start(seg == 0, ka + ngrp * G * BK);
-          issue(ngrp, rem);
-        }
-        wait_vm<0>();
-        ring_barrier();
-        const double *cur = smem + (ngrp % NBUF) * (G * C::STAGE);
-        for (int j = 0; j < rem; j++)
-          mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF, seg == 0);
+        for (int j = 0; j < G; j++)
+          mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF, TWO && s < per);
+      } else {
+        for (int j = 0; j < m; j++)
+          mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF, TWO && s < per);
       }
+    }
+    if (!TWO && G > 1 && rem > 0) {
+      wait_vm<0>();
+      ring_barrier();
+      const double *cur = smem + (ngrp % NBUF) * (G * C::STAGE);
+      for (int j = 0; j < rem; j++)
+        mma(cur + j * C::STAGE, cur + j * C::STAGE + YOFF, false);
     }
   } else {
     // one operand at least goes through registers: loaded while the stage

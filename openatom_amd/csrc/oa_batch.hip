@@ -209,19 +209,22 @@ struct Range {
   bool meets(const Range &o) const { return lo < o.hi && o.lo < hi; }
 };
 
+// What a launch reads and writes of one instance.
+struct Access {
+  Range write, read[2];
+};
+
 // Splits the instances, in order, into runs that may execute at once: no
 // member writes what another one reads or writes.
-template <class Reads, class Writes>
-std::vector<std::vector<int>> runs(int count, Reads reads, Writes writes) {
+std::vector<std::vector<int>> runs(const std::vector<Access> &a) {
+  auto apart = [](const Access &x, const Access &y) {
+    return !x.write.meets(y.write) && !x.write.meets(y.read[0]) && !x.write.meets(y.read[1]) &&
+           !y.write.meets(x.read[0]) && !y.write.meets(x.read[1]);
+  };
   std::vector<std::vector<int>> out;
-  for (int i = 0; i < count; i++) {
+  for (int i = 0; i < (int)a.size(); i++) {
     bool fits = !out.empty();
-    for (size_t k = 0; fits && k < out.back().size(); k++) {
-      const int j = out.back()[k];
-      fits = !writes(i).meets(writes(j));
-      for (const Range &r : reads(j)) fits = fits && !writes(i).meets(r);
-      for (const Range &r : reads(i)) fits = fits && !writes(j).meets(r);
-    }
+    for (size_t k = 0; fits && k < out.back().size(); k++) fits = apart(a[i], a[out.back()[k]]);
     if (!fits) out.emplace_back();
     out.back().push_back(i);
   }
@@ -338,9 +341,8 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
   auto dcnt = [&](long k) { return (unsigned long long *)(dbase + off_cnt) + k; };
   oa_ns_report *drep = (oa_ns_report *)(dbase + off_rep);
   auto all = [](const InstPlan &) { return true; };
-  auto psi_range = [&](int i) {
-    return Range(b->ip[i].psi, b->ip[i].n, b->ip[i].ld, b->ip[i].K);
-  };
+  auto psi_range = [](const InstPlan &p) { return Range(p.psi, p.n, p.ld, p.K); };
+  auto square = [](const double *m, const InstPlan &p) { return Range(m, p.n, p.n, p.n); };
   if (split) {
     for (int i = 0; i < count; i++) {
       InstPlan &p = b->ip[i];
@@ -390,9 +392,10 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
       if (st) return st;
     }
     auto args = [&](const InstPlan &, int i) { return oa[i]; };
-    for (std::vector<int> &run : runs(
-             count, [&](int i) { return std::vector<Range>{psi_range(i)}; },
-             [&](int i) { return Range(b->ip[i].S, b->ip[i].n, b->ip[i].n, b->ip[i].n); })) {
+    std::vector<Access> acc;
+    for (const InstPlan &p : b->ip)
+      acc.push_back({square(p.S, p), {psi_range(p), psi_range(p)}});
+    for (std::vector<int> &run : runs(acc)) {
       std::stable_sort(run.begin(), run.end(),
                        [&](int i, int j) { return oa[i].kchunk > oa[j].kchunk; });
       for (int bm : {128, 64}) {
@@ -417,8 +420,8 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
   }
   std::vector<Range> s_at, t_at;
   for (const InstPlan &p : b->ip) {
-    s_at.emplace_back(p.S, p.n, p.n, p.n);
-    t_at.emplace_back(p.T, p.n, p.n, p.n);
+    s_at.push_back(square(p.S, p));
+    t_at.push_back(square(p.T, p));
   }
   for (int i = 0; i < count; i++)
     for (int j = 0; j < count; j++) na[i].late |= j != i && t_at[i].meets(s_at[j]);
@@ -466,13 +469,10 @@ int plan(oa_batch *b, int count, const oa_instance *in, int prec) {
           [&](const InstPlan &, int i) { return sa[i].items_d1; }, sel, fix, &order);
     }
   } else {
-    for (std::vector<int> &run : runs(
-             count,
-             [&](int i) {
-               const InstPlan &p = b->ip[i];
-               return std::vector<Range>{psi_range(i), Range(p.T, p.n, p.n, p.n)};
-             },
-             [&](int i) { return Range(b->ip[i].out, b->ip[i].n, b->ip[i].ldout, b->ip[i].K); })) {
+    std::vector<Access> acc;
+    for (const InstPlan &p : b->ip)
+      acc.push_back({Range(p.out, p.n, p.ldout, p.K), {psi_range(p), square(p.T, p)}});
+    for (std::vector<int> &run : runs(acc)) {
       std::stable_sort(run.begin(), run.end(),
                        [&](int i, int j) { return b->ip[i].n > b->ip[j].n; });
       std::vector<oa_gemm_problem> gp;

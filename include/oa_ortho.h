@@ -240,7 +240,8 @@ int oa_scale_kx0(oa_handle_t h, int n, int npw, double *X, long ld, int nkx0,
  * ckPairCalculator.C:821 -> ortho.C:153..971 -> ckPairCalculator.C:1201 ->
  * CP_State_GSpacePlane.C:3232).  S, T (n*n) and psi_out ([n][ldout]) are
  * device outputs; psi_out must not alias psi.  Synchronous when iters/err
- * are non-NULL host pointers, else asynchronous. */
+ * are non-NULL host pointers (S, T and the outcome are complete on return,
+ * psi_out in the order of the stream), else asynchronous. */
 int oa_ortho_step(oa_handle_t h, int n, int npw, const double *psi, long ldpsi,
                   int nkx0, int nspin, double tol, int maxit, int prec,
                   double *S, double *T, double *psi_out, long ldout,
@@ -252,9 +253,10 @@ int oa_ortho_step(oa_handle_t h, int n, int npw, const double *psi, long ldpsi,
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Every
  * buffer beyond the arguments lives in one scratch array of
  * oa_noalloc_scratch_bytes() (64 MiB) that each device holds for the life of
- * the process: the S->T report and buffers (5 n^2 doubles) and the overlap's
- * split-K partial tiles, whose depth is capped to what is left (S, T and
- * psi_out then differ from oa_ortho_step's by k-sum rounding only).  Sizes
+ * the process: the S->T report and buffers (five matrices with rows padded to
+ * 16, and partial sums) and, before them in time, the overlap's split-K partial
+ * tiles, whose depth is capped to what 5 n^2 doubles leave (S, T and psi_out
+ * then differ from oa_ortho_step's by k-sum rounding only).  Sizes
  * whose buffers do not fit (n above about 1300) return OA_ERR_CAPACITY;
  * npw must be at least 1.  Calls on one device share the array: calls that
  * overlap in time on one device race. */
@@ -401,10 +403,12 @@ int oa_scatter_rows(oa_handle_t h, int count, const int *row0, const int *nrows,
  * and bead; cpaimd.C:2566-2593 builds each instance's PairCalculator pair
  * and Ortho array) -- advance together: every phase
  * of the step (chunk maxima, slicing, overlap products, reduction, each S->T
- * iteration, back-multiply) is one grouped launch over all
- * instances, walking a device table of per-instance arguments.  Results are
- * those of oa_ortho_step on each instance alone, bit for bit (the digit
- * products are exact and the chunking depends on (n, npw) only). */
+ * iteration, back-multiply) is one grouped launch per tile in use over all
+ * instances, reading a device table of per-instance arguments (in FP64 more
+ * where one instance's buffers overlap another's).  Results, reports included,
+ * are those of oa_ortho_step on each instance alone, bit for bit: every sum runs
+ * in one order whatever the tile, and the chunks and the parts they are summed
+ * in depend on (n, npw) and the precision's slice count only. */
 typedef struct oa_instance {
   int n;              /* states                                          */
   int npw;            /* plane waves (2*npw doubles per state)           */

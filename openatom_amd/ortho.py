@@ -380,9 +380,9 @@ class Handle:
 
 class Batch:
     """Many independent instances (beads, k-points, tempering replicas) of
-    uneven size advanced together: each phase of the step is one persistent
-    grouped launch over all of them (oa_batch_*).  Each instance's results
-    equal Handle.ortho_step on that instance alone, bit for bit."""
+    uneven size advanced together: each phase of the step is one grouped
+    launch per tile in use over all of them (oa_batch_*).  Each instance's
+    results equal Handle.ortho_step on that instance alone, bit for bit."""
 
     def __init__(self, handle: Handle | None = None):
         self.handle = handle or default_handle()

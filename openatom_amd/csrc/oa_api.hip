@@ -143,7 +143,7 @@ int oa_create(oa_handle_t *out, int device) {
   c->device = device;
   if (hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&c->report, sizeof(oa_ns_report)) != hipSuccess ||
-      hipHostMalloc(&c->host, sizeof(oa_ns_host), hipHostMallocDefault) != hipSuccess) {
+      hipHostMalloc(&c->host, sizeof(oa_ns_host), hipHostMallocCoherent) != hipSuccess) {
     (void)hipGetLastError();
     oa_destroy(c);
     return OA_ERR_HIP;

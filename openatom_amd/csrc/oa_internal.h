@@ -34,7 +34,8 @@ struct oa_digit_tag {
   int n = 0, K = 0, prec = 0;
 };
 
-// Pinned host memory the S->T kernels write to and the host polls.
+// Pinned host memory the S->T kernels write to and the host polls while they run:
+// coherent whatever HIP_HOST_COHERENT says.
 struct oa_ns_host {
   oa_ns_report rep;  // the latest report
   int drained;       // 1: nothing of the call's S->T is left on the device
